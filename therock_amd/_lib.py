@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import struct
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # MI355_MOE_LIB names another build of the same library (A/B timing of two builds in one process each)
@@ -135,6 +136,25 @@ PROTOTYPES = {
 
 _lib = None
 
+# The per-pass calls hand their argument blocks over as packed bytes: struct.Struct.pack is several times cheaper than
+# building a ctypes structure field by field, and on the smallest batches the host side is all there is.  Native sizes
+# and alignment ("@"), padded at the end like the C structures ("0P"); the layouts are those of the classes above.
+PACK_SORTING_ARGS = struct.Struct("@10P6i0P")
+PACK_SORTING_TRAITS = struct.Struct("@6i")
+PACK_FUSED_TRAITS = struct.Struct("@13i")
+PACK_GEMM_ARGS = struct.Struct("@12P6i0P")
+PACK_FUSED_ARGS = struct.Struct("@16P7i0P")
+PACK_TOPK_ARGS = struct.Struct("@3P5i0P")
+PACK_TOPK_TRAITS = struct.Struct("@5i")
+PACK_FLATMM_ARGS = struct.Struct("@7P12i3P4i2fi0P")
+PACK_SMOOTHQUANT_ARGS = struct.Struct("@5P6i0P")
+PACK_WORKSPACE = struct.Struct("@PN")
+for _pack, _cls in ((PACK_SORTING_ARGS, SortingArgs), (PACK_SORTING_TRAITS, SortingTraits), (PACK_FUSED_TRAITS, FusedMoeTraits),
+                    (PACK_GEMM_ARGS, FusedMoeGemmArgs), (PACK_FUSED_ARGS, FusedMoeArgs), (PACK_TOPK_ARGS, TopkSoftmaxArgs),
+                    (PACK_TOPK_TRAITS, TopkSoftmaxTraits), (PACK_FLATMM_ARGS, FlatmmArgs),
+                    (PACK_SMOOTHQUANT_ARGS, SmoothquantArgs), (PACK_WORKSPACE, Workspace)):
+    assert _pack.size == C.sizeof(_cls), _cls.__name__
+
 
 def header_version() -> int:
     """MI355_MOE_VERSION as include/mi355_moe.h defines it (what a freshly built library must report)."""
@@ -164,6 +184,20 @@ def load():
             fn.restype, fn.argtypes = res, args
         _lib = lib
     return _lib
+
+
+_packed = {}
+
+
+def packed(name: str):
+    """The entry point `name` as a function that takes its argument blocks as packed bytes (None: a null pointer)."""
+    fn = _packed.get(name)
+    if fn is None or _lib is None:
+        fn = load()[name]  # (a function object of its own: the prototypes above stay as they are)
+        res, args = PROTOTYPES[name]
+        fn.restype, fn.argtypes = res, [a if a in (C.c_int32, C.c_int64) else C.c_void_p for a in args]
+        _packed[name] = fn
+    return fn
 
 
 NUM_KERNELS = 10

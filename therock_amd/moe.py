@@ -32,6 +32,16 @@ class fused_moe_traits:
     local_expert_masking: bool = False
     weight_permute: int = 0  # 1: g and d in ck_tile's pre-shuffled layout b_nr_kr_kw_nw_kv
 
+    def packed(self) -> bytes:
+        d = _lib.DTYPES
+        try:
+            return _lib.PACK_FUSED_TRAITS.pack(d[self.prec_i], d[self.prec_w], d[self.prec_o], d[self.prec_st],
+                                               d[self.prec_sw], d[self.prec_sq], d[self.prec_kw], self.block_m,
+                                               self.activation, self.gate_only, self.fused_quant,
+                                               int(self.local_expert_masking), int(self.weight_permute))
+        except KeyError:
+            return bytes(self.pod())  # raises with the name of the field
+
     def pod(self) -> _lib.FusedMoeTraits:
         d = _lib.DTYPES
         for k in ("prec_i", "prec_w", "prec_o", "prec_st", "prec_sw", "prec_sq", "prec_kw"):
@@ -54,9 +64,10 @@ class moe_sorting_trait:
     skip_experts_with_zero_tokens: bool = True
 
 
-def _ptr(t) -> Optional[int]:
+def _ptr(t) -> int:
+    """Device address of a tensor (0 for None; an int is one already)."""
     if t is None:
-        return None
+        return 0
     if isinstance(t, int):
         return t
     if not t.is_cuda:
@@ -66,11 +77,20 @@ def _ptr(t) -> Optional[int]:
     return t.data_ptr()
 
 
-def _stream(stream) -> Optional[int]:
-    import torch
+_torch_c = None
 
+
+def _stream(stream) -> int:
+    """Handle of `stream`, by default torch's current one: read as a plain number (a Stream object made by
+    torch.cuda.current_stream() costs 3 us, as much as launching a kernel)."""
+    global _torch_c
     if stream is None:
-        stream = torch.cuda.current_stream()
+        if _torch_c is None:
+            import torch
+
+            torch.cuda.current_stream()  # initialises CUDA, with torch's own error where there is no device
+            _torch_c = torch._C
+        return _torch_c._cuda_getCurrentRawStream(_torch_c._cuda_getDevice())
     return stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream)
 
 
@@ -139,14 +159,14 @@ def moe_sorting(trait: moe_sorting_trait, a: moe_sorting_args, stream=None) -> f
     """Returns 0.0 on success, -1.0 when the trait has no kernel (as CK's dispatcher does)."""
     if trait.index_type != "int32" or trait.weight_type != "fp32":
         return -1.0
-    t = _lib.SortingTraits(_lib.DTYPES["int32"], _lib.DTYPES["fp32"], int(trait.local_expert_masking),
-                           int(trait.clear_workspace_inside_api), int(trait.dispatch_policy),
-                           int(trait.skip_experts_with_zero_tokens))
-    s = _lib.SortingArgs(_ptr(a.p_topk_ids), _ptr(a.p_weights), _ptr(a.p_local_expert_mask), _ptr(a.p_local_tokens),
-                         _ptr(a.p_sorted_token_ids), _ptr(a.p_sorted_weights), _ptr(a.p_sorted_expert_ids),
-                         _ptr(a.p_total_tokens_post_pad), _ptr(a.p_moe_buf), _ptr(a.p_ws), a.tokens, a.unit_size,
-                         a.num_experts, a.topk, a.moe_buf_interm_dim, a.moe_buf_elem_bytes)
-    _check(_lib.load().mi355_moe_sorting2(C.byref(t), C.byref(s), _stream(stream)), "moe_sorting")
+    t = _lib.PACK_SORTING_TRAITS.pack(_lib.DTYPES["int32"], _lib.DTYPES["fp32"], int(trait.local_expert_masking),
+                                      int(trait.clear_workspace_inside_api), int(trait.dispatch_policy),
+                                      int(trait.skip_experts_with_zero_tokens))
+    s = _lib.PACK_SORTING_ARGS.pack(_ptr(a.p_topk_ids), _ptr(a.p_weights), _ptr(a.p_local_expert_mask), _ptr(a.p_local_tokens),
+                                    _ptr(a.p_sorted_token_ids), _ptr(a.p_sorted_weights), _ptr(a.p_sorted_expert_ids),
+                                    _ptr(a.p_total_tokens_post_pad), _ptr(a.p_moe_buf), _ptr(a.p_ws), a.tokens, a.unit_size,
+                                    a.num_experts, a.topk, a.moe_buf_interm_dim, a.moe_buf_elem_bytes)
+    _check(_lib.packed("mi355_moe_sorting2")(t, s, _stream(stream)), "moe_sorting")
     return 0.0
 
 
@@ -157,33 +177,51 @@ def fused_moe_get_workspace_size(traits: fused_moe_traits, tokens, num_experts, 
                                                           intermediate_size))
 
 
-def _workspace(ws) -> "_lib.Workspace":
-    return _lib.Workspace(_ptr(ws), 0 if ws is None else ws.numel() * ws.element_size())
+def _workspace(ws) -> bytes:
+    return _lib.PACK_WORKSPACE.pack(_ptr(ws), 0 if ws is None else ws.numel() * ws.element_size())
 
 
-def _fused_args(a: fused_moe_args) -> "_lib.FusedMoeArgs":
-    return _lib.FusedMoeArgs(_ptr(a.a_ptr), _ptr(a.a_scale_ptr), _ptr(a.g_ptr), _ptr(a.d_ptr), _ptr(a.g_scale_ptr),
-                             _ptr(a.d_scale_ptr), _ptr(a.y_smooth_scale_ptr), _ptr(a.local_expert_mask_ptr),
-                             _ptr(a.o_ptr), _ptr(a.ws_ptr), _ptr(a.topk_ids_ptr),
-                             _ptr(a.topk_weight_ptr), _ptr(a.sorted_token_ids_ptr), _ptr(a.sorted_weight_ptr),
-                             _ptr(a.sorted_expert_ids_ptr), _ptr(a.num_sorted_tiles_ptr), a.block_m, a.hidden_size,
-                             a.intermediate_size, a.num_tokens, a.num_experts, a.topk, a.stride_token)
+def _fused_args(a: fused_moe_args) -> bytes:
+    return _lib.PACK_FUSED_ARGS.pack(
+        _ptr(a.a_ptr), _ptr(a.a_scale_ptr), _ptr(a.g_ptr), _ptr(a.d_ptr), _ptr(a.g_scale_ptr), _ptr(a.d_scale_ptr),
+        _ptr(a.y_smooth_scale_ptr), _ptr(a.local_expert_mask_ptr), _ptr(a.o_ptr), _ptr(a.ws_ptr), _ptr(a.topk_ids_ptr),
+        _ptr(a.topk_weight_ptr), _ptr(a.sorted_token_ids_ptr), _ptr(a.sorted_weight_ptr), _ptr(a.sorted_expert_ids_ptr),
+        _ptr(a.num_sorted_tiles_ptr), a.block_m, a.hidden_size, a.intermediate_size, a.num_tokens, a.num_experts, a.topk,
+        a.stride_token)
+
+
+def _gemm_args(a: fused_moe_args) -> bytes:
+    return _lib.PACK_GEMM_ARGS.pack(
+        _ptr(a.a_ptr), _ptr(a.a_scale_ptr), _ptr(a.g_ptr), _ptr(a.d_ptr), _ptr(a.g_scale_ptr), _ptr(a.d_scale_ptr),
+        _ptr(a.y_smooth_scale_ptr), _ptr(a.o_ptr), _ptr(a.sorted_token_ids_ptr), _ptr(a.sorted_weight_ptr),
+        _ptr(a.sorted_expert_ids_ptr), _ptr(a.num_sorted_tiles_ptr), a.hidden_size, a.intermediate_size, a.num_tokens,
+        a.num_experts, a.topk, a.stride_token)
+
+
+def _run_fused(name: str, what: str, traits: fused_moe_traits, pack, a: fused_moe_args, with_ws: bool, stream) -> float:
+    fn = _lib.packed(name)
+    t = traits.packed()
+    try:
+        f = pack(a)
+        ws = _workspace(a.workspace) if with_ws else None
+        s = _stream(stream)
+    except Exception:
+        if not _lib.packed("mi355_fused_moe_supported")(t):  # traits without a kernel: whatever the tensors are
+            return -1.0
+        raise
+    rc = fn(t, f, ws, s) if with_ws else fn(t, f, s)
+    if rc == _lib.OK:
+        return 0.0
+    if rc == _lib.E_UNSUPPORTED:  # (the library checks the traits before anything else)
+        return -1.0
+    _check(rc, what)
+    return 0.0
 
 
 def fused_moe(traits: fused_moe_traits, a: fused_moe_args, stream=None) -> float:
     """Sort + gate/up GEMM + SiLU*up + down GEMM + top-k combine.  0.0 on success, -1.0 when no
     kernel matches the traits."""
-    lib = _lib.load()
-    t = traits.pod()
-    if not lib.mi355_fused_moe_supported(C.byref(t)):
-        return -1.0
-    f = _fused_args(a)
-    ws = _workspace(a.workspace)
-    rc = lib.mi355_fused_moe(C.byref(t), C.byref(f), C.byref(ws), _stream(stream))
-    if rc == _lib.E_UNSUPPORTED:
-        return -1.0
-    _check(rc, "fused_moe")
-    return 0.0
+    return _run_fused("mi355_fused_moe", "fused_moe", traits, _fused_args, a, True, stream)
 
 
 def fused_moe_static_ws_capacity() -> int:
@@ -193,34 +231,12 @@ def fused_moe_static_ws_capacity() -> int:
 def fused_moe_static_ws(traits: fused_moe_traits, a: fused_moe_args, stream=None) -> float:
     """fused_moe() on the library-owned workspace: allocates nothing, a.workspace is ignored.  Problems that need
     more than fused_moe_static_ws_capacity() bytes raise; calls that overlap on one GPU race."""
-    lib = _lib.load()
-    t = traits.pod()
-    if not lib.mi355_fused_moe_supported(C.byref(t)):
-        return -1.0
-    rc = lib.mi355_fused_moe_static_ws(C.byref(t), C.byref(_fused_args(a)), _stream(stream))
-    if rc == _lib.E_UNSUPPORTED:
-        return -1.0
-    _check(rc, "fused_moe_static_ws")
-    return 0.0
+    return _run_fused("mi355_fused_moe_static_ws", "fused_moe_static_ws", traits, _fused_args, a, False, stream)
 
 
 def fused_moegemm(traits: fused_moe_traits, a: fused_moe_args, stream=None) -> float:
     """GEMM half only: consumes sorted_* / num_sorted_tiles already written by moe_sorting."""
-    lib = _lib.load()
-    t = traits.pod()
-    if not lib.mi355_fused_moe_supported(C.byref(t)):
-        return -1.0
-    g = _lib.FusedMoeGemmArgs(_ptr(a.a_ptr), _ptr(a.a_scale_ptr), _ptr(a.g_ptr), _ptr(a.d_ptr), _ptr(a.g_scale_ptr),
-                              _ptr(a.d_scale_ptr), _ptr(a.y_smooth_scale_ptr), _ptr(a.o_ptr),
-                              _ptr(a.sorted_token_ids_ptr), _ptr(a.sorted_weight_ptr), _ptr(a.sorted_expert_ids_ptr),
-                              _ptr(a.num_sorted_tiles_ptr), a.hidden_size,
-                              a.intermediate_size, a.num_tokens, a.num_experts, a.topk, a.stride_token)
-    ws = _workspace(a.workspace)
-    rc = lib.mi355_fused_moegemm(C.byref(t), C.byref(g), C.byref(ws), _stream(stream))
-    if rc == _lib.E_UNSUPPORTED:
-        return -1.0
-    _check(rc, "fused_moegemm")
-    return 0.0
+    return _run_fused("mi355_fused_moegemm", "fused_moegemm", traits, _gemm_args, a, True, stream)
 
 
 def rowwise_quant(x, q_dtype: str, stream=None):
@@ -231,8 +247,8 @@ def rowwise_quant(x, q_dtype: str, stream=None):
     st = {"fp8": torch.float8_e4m3fn, "int8": torch.int8}[q_dtype]
     q = torch.empty((rows, cols), dtype=st, device=x.device)
     scale = torch.empty((rows,), dtype=torch.float32, device=x.device)
-    _check(_lib.load().mi355_moe_rowwise_quant(_ptr(x), rows, cols, x.stride(0), _lib.DTYPES[q_dtype], _ptr(q),
-                                               _ptr(scale), _stream(stream)), "rowwise_quant")
+    _check(_lib.packed("mi355_moe_rowwise_quant")(_ptr(x), rows, cols, x.stride(0), _lib.DTYPES[q_dtype], _ptr(q),
+                                                  _ptr(scale), _stream(stream)), "rowwise_quant")
     return q, scale
 
 
@@ -244,16 +260,16 @@ ACT_SILU, ACT_SWIGLU = 0, 1
 
 def _flatmm_args(kind, a, b, c, sorted_ids, sorted_eid, max_token_id, num_tokens, topk, block_m, sorted_weights,
                  scale_m, scale_n, exp_bias, activation, swiglu_alpha, swiglu_limit, n_padded_zeros, k_padded_zeros,
-                 b_shuffle=0):
+                 b_shuffle=0) -> bytes:
     import torch
 
     experts, n, k = b.shape
     dt = {torch.bfloat16: "bf16", torch.float16: "fp16", torch.int8: "int8", torch.float8_e4m3fn: "fp8", torch.uint8: "fp8"}
-    return _lib.FlatmmArgs(_ptr(sorted_ids), _ptr(sorted_weights), _ptr(sorted_eid), _ptr(max_token_id), _ptr(a), _ptr(b),
-                           _ptr(c), num_tokens, experts, topk, 1, sorted_ids.numel(), n, k, a.stride(0), k, c.stride(0),
-                           n_padded_zeros, k_padded_zeros, _ptr(scale_m), _ptr(scale_n), _ptr(exp_bias),
-                           _lib.DTYPES[dt[a.dtype]], _lib.DTYPES[dt[b.dtype]], block_m, activation, swiglu_alpha,
-                           swiglu_limit, b_shuffle)
+    return _lib.PACK_FLATMM_ARGS.pack(
+        _ptr(sorted_ids), _ptr(sorted_weights), _ptr(sorted_eid), _ptr(max_token_id), _ptr(a), _ptr(b), _ptr(c), num_tokens,
+        experts, topk, 1, sorted_ids.numel(), n, k, a.stride(0), k, c.stride(0), n_padded_zeros, k_padded_zeros,
+        _ptr(scale_m), _ptr(scale_n), _ptr(exp_bias), _lib.DTYPES[dt[a.dtype]], _lib.DTYPES[dt[b.dtype]], block_m, activation,
+        swiglu_alpha, swiglu_limit, b_shuffle)
 
 
 def moe_flatmm_get_workspace_size(kind: int, a, b, c, sorted_ids, sorted_eid, max_token_id, num_tokens: int, topk: int,
@@ -261,7 +277,7 @@ def moe_flatmm_get_workspace_size(kind: int, a, b, c, sorted_ids, sorted_eid, ma
     """Bytes of the workspace tensor moe_flatmm needs for these arguments (0: no kernel)."""
     args = _flatmm_args(kind, a, b, c, sorted_ids, sorted_eid, max_token_id, num_tokens, topk, block_m, None, None, None,
                         None, ACT_SILU, 1.702, 7.0, kw.get("n_padded_zeros", 0), kw.get("k_padded_zeros", 0))
-    return int(_lib.load().mi355_moe_flatmm_workspace_size(kind, C.byref(args)))
+    return int(_lib.packed("mi355_moe_flatmm_workspace_size")(kind, args))
 
 
 def moe_flatmm(kind: int, a, b, c, sorted_ids, sorted_eid, max_token_id, num_tokens: int, topk: int, block_m: int,
@@ -279,14 +295,12 @@ def moe_flatmm(kind: int, a, b, c, sorted_ids, sorted_eid, max_token_id, num_tok
     args = _flatmm_args(kind, a, b, c, sorted_ids, sorted_eid, max_token_id, num_tokens, topk, block_m, sorted_weights,
                         scale_m, scale_n, exp_bias, activation, swiglu_alpha, swiglu_limit, n_padded_zeros, k_padded_zeros,
                         b_shuffle)
-    lib = _lib.load()
     if workspace is None:
         if stream is not None and _stream(stream) != _stream(None):
             raise ValueError("moe_flatmm: pass a caller-owned workspace when launching on a stream other than the current one")
-        ws_bytes = int(lib.mi355_moe_flatmm_workspace_size(kind, C.byref(args)))
+        ws_bytes = int(_lib.packed("mi355_moe_flatmm_workspace_size")(kind, args))
         workspace = torch.empty((max(ws_bytes, 256),), dtype=torch.uint8, device=a.device)
-    ws = _workspace(workspace)
-    rc = lib.mi355_moe_flatmm(kind, C.byref(args), C.byref(ws), _stream(stream))
+    rc = _lib.packed("mi355_moe_flatmm")(kind, args, _workspace(workspace), _stream(stream))
     if rc == _lib.E_UNSUPPORTED:
         return -1.0
     _check(rc, "moe_flatmm")
@@ -323,9 +337,9 @@ def moe_smoothquant(x, smscale, topk_ids, q_dtype: str = "int8", stream=None, ou
     else:
         qy = torch.empty((topk, tokens, hidden), dtype=st, device=x.device)
         ys = torch.empty((topk, tokens), dtype=torch.float32, device=x.device)
-    a = _lib.SmoothquantArgs(_ptr(x), _ptr(smscale), _ptr(topk_ids), _ptr(ys), _ptr(qy), tokens, hidden, experts, topk,
-                             x.stride(0) if tokens else hidden, hidden)
-    _check(_lib.load().mi355_moe_smoothquant(C.byref(a), _lib.DTYPES[q_dtype], _stream(stream)), "moe_smoothquant")
+    a = _lib.PACK_SMOOTHQUANT_ARGS.pack(_ptr(x), _ptr(smscale), _ptr(topk_ids), _ptr(ys), _ptr(qy), tokens, hidden, experts,
+                                        topk, x.stride(0) if tokens else hidden, hidden)
+    _check(_lib.packed("mi355_moe_smoothquant")(a, _lib.DTYPES[q_dtype], _stream(stream)), "moe_smoothquant")
     return qy, ys
 
 
@@ -340,10 +354,11 @@ def topk_softmax(logits, topk: int, activation: str = "softmax", renormalize: bo
     kind = {torch.float32: "fp32", torch.bfloat16: "bf16", torch.float16: "fp16"}[logits.dtype]
     w = torch.empty((rows, topk), dtype=torch.float32, device=logits.device)
     ids = torch.empty((rows, topk), dtype=torch.int32, device=logits.device)
-    t = _lib.TopkSoftmaxTraits(_lib.DTYPES[kind], _lib.DTYPES["fp32"], experts,
-                               {"softmax": 0, "sigmoid": 1}[activation], int(bool(renormalize)))
-    a = _lib.TopkSoftmaxArgs(_ptr(logits), _ptr(w), _ptr(ids), rows, experts, topk, logits.stride(0) if rows else experts, topk)
-    _check(_lib.load().mi355_topk_softmax(C.byref(t), C.byref(a), _stream(stream)), "topk_softmax")
+    t = _lib.PACK_TOPK_TRAITS.pack(_lib.DTYPES[kind], _lib.DTYPES["fp32"], experts,
+                                   {"softmax": 0, "sigmoid": 1}[activation], int(bool(renormalize)))
+    a = _lib.PACK_TOPK_ARGS.pack(_ptr(logits), _ptr(w), _ptr(ids), rows, experts, topk,
+                                 logits.stride(0) if rows else experts, topk)
+    _check(_lib.packed("mi355_topk_softmax")(t, a, _stream(stream)), "topk_softmax")
     return w, ids
 
 
@@ -360,7 +375,7 @@ def fused_moe_chosen_tile_rows(traits: fused_moe_traits, buf, tokens, num_expert
     """The tile height the last fused_moe call on buf's workspace ran with (where the routing decides, the sort's
     choice on the device, read back after a stream synchronisation; else fused_moe_tile_rows)."""
     t = traits.pod()
-    ws = _workspace(buf.ws)
+    ws = _lib.Workspace(_ptr(buf.ws), buf.ws.numel() * buf.ws.element_size())
     return int(_lib.load().mi355_fused_moe_chosen_tile_rows(C.byref(t), tokens, num_experts, topk, hidden_size,
                                                             intermediate_size, C.byref(ws), _stream(stream)))
 
