@@ -100,8 +100,7 @@ struct KernelTimerGroup
 };
 
 // ---- work list of the grouped GEMMs: int32 [kMapHdr + kMapEnt * max_tiles]; [0] = live tiles, [1] = the tile
-// height (rows) the list was built for when the sort chose between two (else 0), then per
-// tile (local expert id, first sorted row, rows, first tile of the expert, tiles of the expert, first sorted
+// height (rows) the list was built for, then per tile (local expert id, first sorted row, rows, first tile of the expert, tiles of the expert, first sorted
 // row of the expert, rows of the expert, rows per tile of the expert): any tile of an expert can be worked
 // out from the entry of any other.  Entries are 32-byte aligned.
 constexpr int kMapHdr = 8;
