@@ -318,18 +318,16 @@ __global__ __launch_bounds__(kPrepBlock) void moe_prep_kernel(const int* __restr
         }
         const int rows = (hi - lo) * unit;
         // the same choice between two tile heights as the sort makes in the fused entry point (see alt_mblk), from
-        // the rows per active expert; 0 in the header: no choice, the kernels do not look
+        // the rows per active expert
         if(alt_rows_per_tile > 0) // (uniform; experts <= 1024 = one pass of this loop)
         {
             int active;
             (void)block_exclusive_scan<kPrepWaves>(rows > 0 ? 1 : 0, s_wave, active);
             if(active >= alt_min_active && (int64_t)nunits * unit >= (int64_t)alt_min_rows * active)
                 rows_per_tile = alt_rows_per_tile;
-            if(threadIdx.x == 0)
-                tile_map[1] = rows_per_tile;
         }
-        else if(threadIdx.x == 0)
-            tile_map[1] = 0;
+        if(threadIdx.x == 0)
+            tile_map[1] = rows_per_tile;
         const int nt   = ceil_div(rows, rows_per_tile);
         int sum;
         const int tb   = total + block_exclusive_scan<kPrepWaves>(nt, s_wave, sum);
@@ -545,13 +543,42 @@ inline int pick_mblk(const mi355_fused_moe_traits& t, int64_t tokens, int topk, 
 // large tiles anyway) the sort chooses between the two tile heights from the counts it holds, and both kernel
 // families are launched: the workgroups of the one whose tile height was not chosen leave at once (two short empty
 // launches per pass).  Returns the second tile height in 32-row blocks, 0: no choice.
-inline int alt_mblk(const mi355_fused_moe_traits& t, int64_t tokens, int topk, int experts, int hidden, int inter)
+constexpr int kAltMinRows = 48; // padded rows per active expert from which the large tiles are chosen
+
+// The most experts that can be active while their padded rows average kAltMinRows: an expert with c entries holds at
+// most c + block_m rows, so the c of the active ones add up to at least (kAltMinRows - block_m) each.
+inline int64_t alt_most_active(const mi355_fused_moe_traits& t, int64_t tokens, int topk, int experts)
 {
-    if(t.prec_i != MI355_MOE_FP8 || t.fused_quant != 0 || !big_tile_ok(t, tokens, topk, experts, hidden, inter))
+    const int64_t n = std::min<int64_t>(tokens * topk, experts);
+    return t.block_m < kAltMinRows ? std::min(n, tokens * topk / (kAltMinRows - t.block_m)) : n;
+}
+
+// min_active: active experts from which the large tiles may be chosen.  A batch that cannot have as many (few tokens)
+// gets no second candidate, hence no empty launches (13 tokens of the 256-expert model: two of them, 16 us of 627).
+inline int alt_mblk(const mi355_fused_moe_traits& t, int64_t tokens, int topk, int experts, int hidden, int inter, int min_active)
+{
+    if(t.prec_i != MI355_MOE_FP8 || t.fused_quant != 0 || alt_most_active(t, tokens, topk, experts) < min_active ||
+       !big_tile_ok(t, tokens, topk, experts, hidden, inter))
         return 0;
     return pick_mblk(t, tokens, topk, experts, hidden, inter) <= 4 ? big_tile_rows() / 32 : 0;
 }
-constexpr int kAltMinRows = 48; // padded rows per active expert from which the large tiles are chosen
+
+// enough active experts for tiles of 256 of their weight_rows weight rows to fill the chip
+inline int alt_min_active(int weight_rows) { return ceil_div(device_info().num_cu, ceil_div(weight_rows, 256)); }
+inline int alt_mblk_fused(const mi355_fused_moe_traits& t, int64_t tokens, int topk, int experts, int hidden, int inter)
+{
+    return alt_mblk(t, tokens, topk, experts, hidden, inter, alt_min_active((t.gate_only ? 1 : 2) * inter));
+}
+
+// The most tiles of `rows` rows that `active` experts can need for n entries between them: an expert's c entries are
+// padded to c + unit - 1 rows at most and these split into ceil(rows of the expert / rows) tiles.  What a launch is
+// sized by where the sort's list is known to follow this (the fused entry point): the list's capacity allows every
+// expert a tile and every pad cell a row, twice as many workgroups at decode sizes.
+inline int most_tiles(int64_t n, int64_t active, int unit, int rows)
+{
+    active = std::min(active, n);
+    return (int)(rows % unit == 0 ? active + (n - active) / rows : (n + active * (unit + rows - 2)) / rows);
+}
 
 template <int MODE, bool GEMM0>
 int launch_gemm(int mblk, const GemmParams& p, int max_tiles, hipStream_t stream)
@@ -653,7 +680,7 @@ int gemm_tile_rows(const mi355_fused_moe_traits& t, int32_t tokens, int32_t expe
 int gemm_alt_tile_rows(const mi355_fused_moe_traits& t, int32_t tokens, int32_t experts, int32_t topk, int32_t hidden,
                        int32_t inter)
 {
-    return alt_mblk(t, tokens, topk, experts, hidden, inter) * 32;
+    return alt_mblk_fused(t, tokens, topk, experts, hidden, inter) * 32;
 }
 
 WorkspaceLayout workspace_layout(const mi355_fused_moe_traits& t, int32_t tokens, int32_t experts, int32_t topk,
@@ -695,9 +722,9 @@ GemmPlan make_gemm_plan(const mi355_fused_moe_traits& t, void* ws_ptr, int32_t t
     g.max_tiles     = ws.max_tiles;
     g.inv           = reinterpret_cast<int*>(wsb + ws.inv_off);
     // the second candidate needs enough active experts for its gate+up tiles (256 weight rows each) to fill the chip
-    g.alt_rows_per_tile = alt_mblk(t, tokens, topk, experts, hidden, inter) * 32;
+    g.alt_rows_per_tile = alt_mblk_fused(t, tokens, topk, experts, hidden, inter) * 32;
     g.alt_min_rows      = kAltMinRows;
-    g.alt_min_active    = ceil_div(device_info().num_cu, ceil_div((t.gate_only ? 1 : 2) * inter, 256));
+    g.alt_min_active    = alt_min_active((t.gate_only ? 1 : 2) * inter);
     return g;
 }
 
@@ -779,8 +806,14 @@ int launch_fused_moegemm(const mi355_fused_moe_traits& t, const mi355_fused_moeg
     const int mblk     = pick_mblk(t, T, K, E, H, I);
     const int max_units = (int)ceil_div<int64_t>(ws.max_pad, t.block_m);
     // the sort chose between two tile heights (see alt_mblk): both kernel families are launched for each GEMM
-    const int alt           = alt_mblk(t, T, K, E, H, I);
-    const int alt_max_tiles = alt ? (int)std::min<int64_t>(ws.max_tiles, E + ws.max_pad / (alt * 32) + 1) : 0;
+    const int alt     = alt_mblk_fused(t, T, K, E, H, I);
+    int max_tiles     = ws.max_tiles;
+    int alt_max_tiles = alt ? (int)std::min<int64_t>(ws.max_tiles, E + ws.max_pad / (alt * 32) + 1) : 0;
+    if(prep_done)
+    {
+        max_tiles     = std::min(max_tiles, most_tiles((int64_t)T * K, E, t.block_m, mblk * 32));
+        alt_max_tiles = std::min(alt_max_tiles, most_tiles((int64_t)T * K, alt_most_active(t, T, K, E), t.block_m, std::max(alt, 1) * 32));
+    }
 
     const int n_inv      = T * K;
     const int prep_grid  = 1 + std::min(ceil_div(n_inv, kPrepBlock * 4), 64);
@@ -791,7 +824,7 @@ int launch_fused_moegemm(const mi355_fused_moe_traits& t, const mi355_fused_moeg
                            static_cast<const int*>(a.sorted_expert_ids_ptr),
                            static_cast<const int*>(a.num_sorted_tiles_ptr), t.block_m, E, mblk * 32, max_units,
                            ws.max_tiles, tile_map, inv, n_inv, alt * 32, kAltMinRows,
-                           ceil_div(device_info().num_cu, ceil_div((t.gate_only ? 1 : 2) * I, 256)));
+                           alt_min_active((t.gate_only ? 1 : 2) * I));
         hipLaunchKernelGGL(moe_inv_kernel, dim3(std::min<int>(ceil_div<int64_t>(ws.max_pad, 256), 1024)), dim3(256), 0,
                            stream, static_cast<const int*>(a.sorted_token_ids_ptr),
                            static_cast<const int*>(a.num_sorted_tiles_ptr), (int)ws.max_pad, T, K, inv);
@@ -840,7 +873,7 @@ int launch_fused_moegemm(const mi355_fused_moe_traits& t, const mi355_fused_moeg
     const int alt_y_slab = (alt && ((int64_t)I * y_b) % 64 == 0) ? (int)((int64_t)I * y_b / 64) : 0;
     {
         KernelTimerGroup both(MI355_MOE_K_GEMM0, stream, alt != 0);
-        rc = launch_grouped_gemm(t.prec_i, true, mblk, decode, p, ws.max_tiles, stream);
+        rc = launch_grouped_gemm(t.prec_i, true, mblk, decode, p, max_tiles, stream);
         if(rc != MI355_MOE_OK)
             return rc;
         if(alt)
@@ -891,7 +924,7 @@ int launch_fused_moegemm(const mi355_fused_moe_traits& t, const mi355_fused_moeg
     {
         KernelTimerGroup both(MI355_MOE_K_GEMM1, stream, alt != 0);
         rc = launch_grouped_gemm(t.prec_i, false, mblk, decode && down_gemm_wants_decode(E, (int64_t)T * K, H), p,
-                                 ws.max_tiles, stream, requant && !requant8);
+                                 max_tiles, stream, requant && !requant8);
         if(rc != MI355_MOE_OK)
             return rc;
         if(alt)
@@ -987,7 +1020,7 @@ int flatmm_layout(int kind, const mi355_moe_flatmm_args& a, FlatmmLayout& L)
         L.mblk = std::min(L.mblk, 4);
     }
     // skewed decode-sized batches: the same choice between two tile heights as the fused entry points make
-    L.alt          = a.k_padded_zeros == 0 ? alt_mblk(L.traits, a.NumTokens, a.TopK, a.NumExperts, L.hidden, L.inter) : 0;
+    L.alt          = a.k_padded_zeros == 0 ? alt_mblk(L.traits, a.NumTokens, a.TopK, a.NumExperts, L.hidden, L.inter, alt_min_active(a.N)) : 0;
     L.max_pad      = (int64_t)a.TopK * a.NumTokens + (int64_t)a.NumExperts * a.block_m - a.TopK;
     L.max_tiles    = (int32_t)(a.NumExperts + L.max_pad / (L.mblk * 32) + 1);
     L.total        = 0;
@@ -1064,7 +1097,7 @@ int launch_moe_flatmm(int kind, const mi355_moe_flatmm_args& a, void* ws_ptr, si
                            static_cast<const int*>(a.p_sorted_expert_ids), static_cast<const int*>(a.p_max_token_id),
                            a.block_m, E, mblk * 32, (int)ceil_div<int64_t>(L.max_pad, a.block_m), L.max_tiles, tile_map,
                            inv, n_inv, alt * 32, kAltMinRows,
-                           ceil_div(device_info().num_cu, ceil_div(a.N, 256))); // enough tiles of this GEMM to fill the chip
+                           alt_min_active(a.N));
         if(!g1)
             hipLaunchKernelGGL(moe_inv_kernel, dim3(std::min<int>(ceil_div<int64_t>(L.max_pad, 256), 1024)), dim3(256), 0,
                                stream, static_cast<const int*>(a.p_sorted_token_ids),
