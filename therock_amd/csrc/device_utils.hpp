@@ -26,23 +26,24 @@ __device__ inline int wave_inclusive_scan(int x)
     return x;
 }
 
-// Wave-wide maximum / minimum of a 32-bit unsigned value, the same in every lane afterwards.  Data-parallel
+// Wave-wide maximum of a 32-bit unsigned integer or a float, the same in every lane afterwards.  Data-parallel
 // primitives instead of LDS-routed shuffles: an inclusive scan over each row of 16 lanes (row_shr 1, 2, 4, 8; lanes
 // shifted in from outside a row read the identity), then lane 15 of rows 0 and 2 is combined into rows 1 and 3
 // (row_bcast:15) and lane 31 into rows 2 and 3 (row_bcast:31): lane 63 holds the result.
-template <bool MAX>
-__device__ inline uint32_t wave_reduce_u32(uint32_t v)
+__device__ inline uint32_t max_of(uint32_t a, uint32_t b) { return max(a, b); }
+__device__ inline float max_of(float a, float b) { return fmaxf(a, b); }
+template <typename T>
+__device__ inline T wave_reduce_max(T v, T identity)
 {
-    constexpr int ident = MAX ? 0 : -1;
-    auto combine = [](uint32_t a, uint32_t b) { return MAX ? max(a, b) : min(a, b); };
-    int x = static_cast<int>(v);
-    x = static_cast<int>(combine(x, __builtin_amdgcn_update_dpp(ident, x, 0x111, 0xf, 0xf, false))); // row_shr:1
-    x = static_cast<int>(combine(x, __builtin_amdgcn_update_dpp(ident, x, 0x112, 0xf, 0xf, false))); // row_shr:2
-    x = static_cast<int>(combine(x, __builtin_amdgcn_update_dpp(ident, x, 0x114, 0xf, 0xf, false))); // row_shr:4
-    x = static_cast<int>(combine(x, __builtin_amdgcn_update_dpp(ident, x, 0x118, 0xf, 0xf, false))); // row_shr:8
-    x = static_cast<int>(combine(x, __builtin_amdgcn_update_dpp(ident, x, 0x142, 0xa, 0xf, false))); // row_bcast:15
-    x = static_cast<int>(combine(x, __builtin_amdgcn_update_dpp(ident, x, 0x143, 0xc, 0xf, false))); // row_bcast:31
-    return static_cast<uint32_t>(__builtin_amdgcn_readlane(x, 63));
+    const int ident = __builtin_bit_cast(int, identity);
+    auto shifted = [&](int x) { return __builtin_bit_cast(T, x); };
+    v = max_of(v, shifted(__builtin_amdgcn_update_dpp(ident, __builtin_bit_cast(int, v), 0x111, 0xf, 0xf, false))); // row_shr:1
+    v = max_of(v, shifted(__builtin_amdgcn_update_dpp(ident, __builtin_bit_cast(int, v), 0x112, 0xf, 0xf, false))); // row_shr:2
+    v = max_of(v, shifted(__builtin_amdgcn_update_dpp(ident, __builtin_bit_cast(int, v), 0x114, 0xf, 0xf, false))); // row_shr:4
+    v = max_of(v, shifted(__builtin_amdgcn_update_dpp(ident, __builtin_bit_cast(int, v), 0x118, 0xf, 0xf, false))); // row_shr:8
+    v = max_of(v, shifted(__builtin_amdgcn_update_dpp(ident, __builtin_bit_cast(int, v), 0x142, 0xa, 0xf, false))); // row_bcast:15
+    v = max_of(v, shifted(__builtin_amdgcn_update_dpp(ident, __builtin_bit_cast(int, v), 0x143, 0xc, 0xf, false))); // row_bcast:31
+    return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
 // Exclusive scan of one int per thread over a block of NWAVES*64 threads.  s_wave needs

@@ -30,13 +30,6 @@ struct RouterParams
     int sigmoid, renorm;
 };
 
-__device__ inline float wave_max(float v)
-{
-#pragma unroll
-    for(int d = 32; d > 0; d >>= 1)
-        v = fmaxf(v, __shfl_xor(v, d));
-    return v;
-}
 __device__ inline float wave_sum(float v)
 {
 #pragma unroll
@@ -82,7 +75,7 @@ __global__ __launch_bounds__(kRouterBlock) void topk_softmax_kernel(const Router
 #pragma unroll
         for(int j = 0; j < PER_LANE; j++)
             m = fmaxf(m, v[j]);
-        m       = wave_max(m);
+        m       = wave_reduce_max(m, -INFINITY);
         float s = 0.f;
 #pragma unroll
         for(int j = 0; j < PER_LANE; j++)
@@ -96,9 +89,11 @@ __global__ __launch_bounds__(kRouterBlock) void topk_softmax_kernel(const Router
             v[j] = lane + j * kWave < p.experts ? v[j] / s : -INFINITY;
     }
     // k rounds of arg-max.  The probabilities are non-negative, so their bit patterns order like unsigned integers:
-    // key = bits + 1 for a live entry, 0 for one that is struck out or beyond the expert count.  A round is two
-    // wave reductions: the largest key, then the lowest expert id among the entries that hold it.  The winner is
-    // struck out of its lane's registers and kept by lane i.
+    // key = bits + 1 for a live entry, 0 for one that is struck out or beyond the expert count.  A round is one wave
+    // reduction for the largest key; the lowest expert id among the entries that hold it is then the first lane of the
+    // first register whose ballot is not empty (experts lane + 64 j: scalar work, where a second reduction over the
+    // ids was another chain of six dependent cross-lane steps).  The winner is struck out of its lane's registers and
+    // kept by lane i.
     uint32_t key[PER_LANE];
 #pragma unroll
     for(int j = 0; j < PER_LANE; j++)
@@ -109,16 +104,18 @@ __global__ __launch_bounds__(kRouterBlock) void topk_softmax_kernel(const Router
     for(int i = 0; i < p.topk; i++)
     {
         uint32_t bk = 0u;
-        int be      = 0x7fffffff;
 #pragma unroll
         for(int j = 0; j < PER_LANE; j++)
-            if(key[j] > bk)
-            {
-                bk = key[j];
-                be = lane + j * kWave;
-            }
-        const uint32_t top = wave_reduce_u32<true>(bk);
-        const int win      = static_cast<int>(wave_reduce_u32<false>(bk == top ? static_cast<uint32_t>(be) : 0x7fffffffu));
+            bk = max(bk, key[j]);
+        const uint32_t top = wave_reduce_max<uint32_t>(bk, 0u);
+        int win            = 0x7fffffff;
+#pragma unroll
+        for(int j = PER_LANE - 1; j >= 0; j--)
+        {
+            const uint64_t holds = __ballot(key[j] == top);
+            if(holds != 0 && top != 0u)
+                win = j * kWave + __builtin_ctzll(holds);
+        }
         const float best   = top != 0u ? __uint_as_float(top - 1u) : -INFINITY;
 #pragma unroll
         for(int j = 0; j < PER_LANE; j++)
