@@ -100,9 +100,11 @@ struct KernelTimerGroup
 };
 
 // ---- work list of the grouped GEMMs: int32 [kMapHdr + kMapEnt * max_tiles]; [0] = live tiles, [1] = the tile
-// height (rows) the list was built for, then per tile (local expert id, first sorted row, rows, first tile of the expert, tiles of the expert, first sorted
-// row of the expert, rows of the expert, rows per tile of the expert): any tile of an expert can be worked
-// out from the entry of any other.  Entries are 32-byte aligned.
+// height (rows) the list was built for, then per tile (local expert id, first sorted row, rows, first tile of the
+// expert, tiles of the expert, first sorted row of the expert, rows of the expert, rows per tile of the expert): any
+// tile of an expert can be worked out from the entry of any other.  Rows are an expert's tokens: the padding up to the
+// sort's unit at its end belongs to no tile (with a unit of 64 and 15 rows per expert every second 32-row tile held
+// nothing else: 1.6 of 3.5 ms).  Entries are 32-byte aligned.
 constexpr int kMapHdr = 8;
 constexpr int kMapEnt = 8;
 
@@ -139,7 +141,7 @@ struct GemmPlan
     int* inv;          // [tokens * topk]: sorted position of every (token, slot), -1 when dropped
     // A second tile height the sort may choose instead, from what only the device knows: with skewed routing the
     // experts that have tokens at all hold many more rows than tokens * topk / experts suggests.  Chosen when at least
-    // alt_min_active experts are active and their padded rows average alt_min_rows or more; 0 rows: no choice.
+    // alt_min_active experts are active and their rows, rounded up to 32, average alt_min_rows or more; 0 rows: no choice.
     int alt_rows_per_tile;
     int alt_min_rows;
     int alt_min_active;

@@ -265,13 +265,15 @@ __global__ __launch_bounds__(kBlock, 2) void moe_gemm_kernel(const GemmParams p)
 }
 
 // ---------------------------------------------------------------------------------------------
-// Tile list: one entry per (expert, group of <= rows_per_tile sorted rows), rows split evenly.
-// Block 0 builds the list from sorted_expert_ids; every block helps reset the inverse map, which
+// Tile list: one entry per (expert, group of <= rows_per_tile sorted rows), rows split evenly; the padding at the end of
+// an expert's last unit is left out.
+// Block 0 builds the list from the sorted arrays; every block helps reset the inverse map, which
 // moe_inv_kernel then fills from the sorted ids (the sort does both itself in the fused entry point).
 constexpr int kPrepBlock = 1024;
 constexpr int kPrepWaves = kPrepBlock / kWave;
 
 __global__ __launch_bounds__(kPrepBlock) void moe_prep_kernel(const int* __restrict__ sorted_eid,
+                                                               const int* __restrict__ sorted_ids, int tokens,
                                                                const int* __restrict__ post_pad_ptr, int unit,
                                                                int experts, int rows_per_tile, int max_units,
                                                                int max_tiles, int* __restrict__ tile_map,
@@ -284,6 +286,8 @@ __global__ __launch_bounds__(kPrepBlock) void moe_prep_kernel(const int* __restr
         return;
     __shared__ int s_wave[kPrepWaves + 1];
     __shared__ int s_lo[kPrepBlock], s_hi[kPrepBlock]; // first and one-past-last sort unit of each expert
+    __shared__ int s_real[kPrepBlock];                 // rows of its last unit up to the last token
+    __shared__ int s_wave2[2][kPrepWaves + 1];
     const int post_pad = post_pad_ptr[0];
     int nunits         = post_pad / unit;
     nunits             = max(0, min(nunits, max_units));
@@ -291,6 +295,7 @@ __global__ __launch_bounds__(kPrepBlock) void moe_prep_kernel(const int* __restr
     // neighbours - independent loads, where a binary search per expert is a chain of a dozen dependent ones
     s_lo[threadIdx.x] = 0;
     s_hi[threadIdx.x] = 0;
+    s_real[threadIdx.x] = 0;
     __syncthreads();
     for(int u = threadIdx.x; u < nunits; u += kPrepBlock)
     {
@@ -306,6 +311,13 @@ __global__ __launch_bounds__(kPrepBlock) void moe_prep_kernel(const int* __restr
         }
     }
     __syncthreads();
+    for(int idx = threadIdx.x; idx < experts * unit; idx += kPrepBlock)
+    {
+        const int e = idx / unit;
+        if(s_hi[e] > s_lo[e] && (sorted_ids[(s_hi[e] - 1) * unit + idx - e * unit] & 0xffffff) < tokens)
+            atomicMax(&s_real[e], idx - e * unit + 1);
+    }
+    __syncthreads();
     int total          = 0;
     for(int e0 = 0; e0 < experts; e0 += kPrepBlock) // experts <= 1024: one pass
     {
@@ -316,14 +328,15 @@ __global__ __launch_bounds__(kPrepBlock) void moe_prep_kernel(const int* __restr
             lo = s_lo[e];
             hi = max(s_hi[e], lo);
         }
-        const int rows = (hi - lo) * unit;
+        const int rows = hi > lo ? (hi - lo - 1) * unit + s_real[e] : 0;
         // the same choice between two tile heights as the sort makes in the fused entry point (see alt_mblk), from
         // the rows per active expert
         if(alt_rows_per_tile > 0) // (uniform; experts <= 1024 = one pass of this loop)
         {
-            int active;
-            (void)block_exclusive_scan<kPrepWaves>(rows > 0 ? 1 : 0, s_wave, active);
-            if(active >= alt_min_active && (int64_t)nunits * unit >= (int64_t)alt_min_rows * active)
+            const int v[2] = {rows > 0 ? 1 : 0, round_up(rows, 32)};
+            int ex[2], sum[2];
+            block_exclusive_scan_n<kPrepWaves, 2>(v, s_wave2, ex, sum);
+            if(sum[0] >= alt_min_active && sum[1] >= (int64_t)alt_min_rows * sum[0])
                 rows_per_tile = alt_rows_per_tile;
         }
         if(threadIdx.x == 0)
@@ -543,21 +556,20 @@ inline int pick_mblk(const mi355_fused_moe_traits& t, int64_t tokens, int topk, 
 // large tiles anyway) the sort chooses between the two tile heights from the counts it holds, and both kernel
 // families are launched: the workgroups of the one whose tile height was not chosen leave at once (two short empty
 // launches per pass).  Returns the second tile height in 32-row blocks, 0: no choice.
-constexpr int kAltMinRows = 48; // padded rows per active expert from which the large tiles are chosen
+constexpr int kAltMinRows = 48; // rows per active expert, rounded up to 32 each, from which the large tiles are chosen
 
-// The most experts that can be active while their padded rows average kAltMinRows: an expert with c entries holds at
-// most c + block_m rows, so the c of the active ones add up to at least (kAltMinRows - block_m) each.
-inline int64_t alt_most_active(const mi355_fused_moe_traits& t, int64_t tokens, int topk, int experts)
+// The most experts that can be active while their rows, each count rounded up to 32, average kAltMinRows: the n entries
+// have to make up for 31 rows of rounding each.
+inline int64_t alt_most_active(int64_t tokens, int topk, int experts)
 {
-    const int64_t n = std::min<int64_t>(tokens * topk, experts);
-    return t.block_m < kAltMinRows ? std::min(n, tokens * topk / (kAltMinRows - t.block_m)) : n;
+    return std::min<int64_t>(experts, tokens * topk / (kAltMinRows - 31));
 }
 
 // min_active: active experts from which the large tiles may be chosen.  A batch that cannot have as many (few tokens)
 // gets no second candidate, hence no empty launches (13 tokens of the 256-expert model: two of them, 16 us of 627).
 inline int alt_mblk(const mi355_fused_moe_traits& t, int64_t tokens, int topk, int experts, int hidden, int inter, int min_active)
 {
-    if(t.prec_i != MI355_MOE_FP8 || t.fused_quant != 0 || alt_most_active(t, tokens, topk, experts) < min_active ||
+    if(t.prec_i != MI355_MOE_FP8 || t.fused_quant != 0 || alt_most_active(tokens, topk, experts) < min_active ||
        !big_tile_ok(t, tokens, topk, experts, hidden, inter))
         return 0;
     return pick_mblk(t, tokens, topk, experts, hidden, inter) <= 4 ? big_tile_rows() / 32 : 0;
@@ -570,14 +582,14 @@ inline int alt_mblk_fused(const mi355_fused_moe_traits& t, int64_t tokens, int t
     return alt_mblk(t, tokens, topk, experts, hidden, inter, alt_min_active((t.gate_only ? 1 : 2) * inter));
 }
 
-// The most tiles of `rows` rows that `active` experts can need for n entries between them: an expert's c entries are
-// padded to c + unit - 1 rows at most and these split into ceil(rows of the expert / rows) tiles.  What a launch is
-// sized by where the sort's list is known to follow this (the fused entry point): the list's capacity allows every
-// expert a tile and every pad cell a row, twice as many workgroups at decode sizes.
-inline int most_tiles(int64_t n, int64_t active, int unit, int rows)
+// The most tiles of `rows` rows that `active` experts can need for n entries between them (an expert's c rows split into
+// ceil(c / rows) tiles).  What a launch is sized by where the sort's list is known to follow this (the fused entry
+// point): the list's capacity allows every expert a tile and every pad cell a row, twice as many workgroups at decode
+// sizes.
+inline int most_tiles(int64_t n, int64_t active, int rows)
 {
     active = std::min(active, n);
-    return (int)(rows % unit == 0 ? active + (n - active) / rows : (n + active * (unit + rows - 2)) / rows);
+    return (int)(active + (n - active) / rows);
 }
 
 template <int MODE, bool GEMM0>
@@ -811,8 +823,8 @@ int launch_fused_moegemm(const mi355_fused_moe_traits& t, const mi355_fused_moeg
     int alt_max_tiles = alt ? (int)std::min<int64_t>(ws.max_tiles, E + ws.max_pad / (alt * 32) + 1) : 0;
     if(prep_done)
     {
-        max_tiles     = std::min(max_tiles, most_tiles((int64_t)T * K, E, t.block_m, mblk * 32));
-        alt_max_tiles = std::min(alt_max_tiles, most_tiles((int64_t)T * K, alt_most_active(t, T, K, E), t.block_m, std::max(alt, 1) * 32));
+        max_tiles     = std::min(max_tiles, most_tiles((int64_t)T * K, E, mblk * 32));
+        alt_max_tiles = std::min(alt_max_tiles, most_tiles((int64_t)T * K, alt_most_active(T, K, E), std::max(alt, 1) * 32));
     }
 
     const int n_inv      = T * K;
@@ -822,6 +834,7 @@ int launch_fused_moegemm(const mi355_fused_moe_traits& t, const mi355_fused_moeg
         KernelTimer timer(MI355_MOE_K_PREP, stream);
         hipLaunchKernelGGL(moe_prep_kernel, dim3(prep_grid), dim3(kPrepBlock), 0, stream,
                            static_cast<const int*>(a.sorted_expert_ids_ptr),
+                           static_cast<const int*>(a.sorted_token_ids_ptr), T,
                            static_cast<const int*>(a.num_sorted_tiles_ptr), t.block_m, E, mblk * 32, max_units,
                            ws.max_tiles, tile_map, inv, n_inv, alt * 32, kAltMinRows,
                            alt_min_active((t.gate_only ? 1 : 2) * I));
@@ -1094,8 +1107,8 @@ int launch_moe_flatmm(int kind, const mi355_moe_flatmm_args& a, void* ws_ptr, si
         const int n_inv     = T * K;
         const int prep_grid = 1 + std::min(ceil_div(n_inv, kPrepBlock * 4), 64);
         hipLaunchKernelGGL(moe_prep_kernel, dim3(prep_grid), dim3(kPrepBlock), 0, stream,
-                           static_cast<const int*>(a.p_sorted_expert_ids), static_cast<const int*>(a.p_max_token_id),
-                           a.block_m, E, mblk * 32, (int)ceil_div<int64_t>(L.max_pad, a.block_m), L.max_tiles, tile_map,
+                           static_cast<const int*>(a.p_sorted_expert_ids), static_cast<const int*>(a.p_sorted_token_ids), T,
+                           static_cast<const int*>(a.p_max_token_id), a.block_m, E, mblk * 32, (int)ceil_div<int64_t>(L.max_pad, a.block_m), L.max_tiles, tile_map,
                            inv, n_inv, alt * 32, kAltMinRows,
                            alt_min_active(a.N));
         if(!g1)

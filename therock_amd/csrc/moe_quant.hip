@@ -443,8 +443,8 @@ __global__ __launch_bounds__(256) void moe_smoothquant_grouped_kernel(const uint
 // instance of these variants to match bit for bit, so the rounding is chosen for accuracy: truncation, which the
 // stand-alone smooth-quant kernel above has to use to match ck_tile's, doubles the error of the down GEMM's
 // input.  One wave per row; a row of up to 2048 columns is read once.
-// Output row-major, or slab-major when segs > 0 (y_slab_offset); padding rows become zeros with scale 0, rows past
-// the sorted prefix are left alone.
+// Output row-major, or slab-major when segs > 0 (y_slab_offset); padding rows and rows past the sorted prefix are left
+// alone.
 // FP8 (the fp8 path with fused_quant): e4m3 codes instead, scale = amax / 448, rounded to nearest even by the
 // conversion instruction.
 template <bool SMOOTH, bool FP8>
@@ -463,15 +463,8 @@ __global__ __launch_bounds__(256) void moe_requant_y_kernel(const uint16_t* __re
     auto dst = [&](int c) {
         return yq + (segs > 0 ? y_slab_offset(row, c * 8, segs) : row * inter + c * 8);
     };
-    const bool real = (sorted_ids[row] & 0xffffff) < tokens;
-    if(!real)
-    {
-        for(int c = lane; c < chunks; c += 64)
-            *reinterpret_cast<uint2*>(dst(c)) = make_uint2(0u, 0u);
-        if(lane == 0)
-            yscale[row] = 0.f;
-        return;
-    }
+    if((sorted_ids[row] & 0xffffff) >= tokens)
+        return; // padding: no GEMM tile holds the row
     const uint16_t* yr = y + row * inter;
     const float* sr    = SMOOTH ? smooth + (int64_t)sorted_expert_ids[row / unit] * inter : nullptr;
     auto load = [&](int c, float (&o)[8]) {

@@ -135,7 +135,7 @@ struct ScanShared
     int tbase[kMaxExperts]; // first output tile of the expert
     int oeid[kMaxExperts];  // expert id written to sorted_expert_ids
     int wave[kScanWaves + 1];
-    int wave3[3][kScanWaves + 1];
+    int wave4[4][kScanWaves + 1];
 };
 
 // Pass 2, run by one 1024-thread block.  counts is [nseg][E] (global or LDS): on entry the
@@ -201,9 +201,10 @@ __device__ inline void scan_phase(ScanShared& s, int* counts, int nseg, int E, i
     const int my_tiles = on_rank ? max(ceil_div(my_cnt, U), keep_empty ? 1 : 0) : 0;
     // one pass of block scans for the first output tile of each expert, the output expert ids and the number of
     // experts that have tokens
-    const int scan_in[3] = {my_tiles, on_rank ? 1 : 0, on_rank && my_cnt > 0 ? 1 : 0};
-    int scan_ex[3], scan_total[3];
-    block_exclusive_scan_n<kScanWaves, 3>(scan_in, s.wave3, scan_ex, scan_total);
+    const int my_rows    = on_rank ? my_cnt : 0;
+    const int scan_in[4] = {my_tiles, on_rank ? 1 : 0, my_rows > 0 ? 1 : 0, round_up(my_rows, 32)};
+    int scan_ex[4], scan_total[4];
+    block_exclusive_scan_n<kScanWaves, 4>(scan_in, s.wave4, scan_ex, scan_total);
     const int tbase = scan_ex[0], oeid = scan_ex[1];
     const int total_tiles = scan_total[0], active = scan_total[2];
     if(tid < kMaxExperts)
@@ -300,14 +301,14 @@ __device__ inline void scan_phase(ScanShared& s, int* counts, int nseg, int E, i
         total[1] = T;
     }
 
-    // work list of the grouped GEMMs: the padded rows of an expert split evenly into tiles
+    // work list of the grouped GEMMs: the rows of an expert (without its padding) split evenly into tiles
     if(plan.tile_map != nullptr)
     {
-        const int rows = tid < E ? s.tiles[tid] * U : 0;
+        const int rows    = my_rows;
         int rows_per_tile = plan.rows_per_tile;
         if(plan.alt_rows_per_tile > 0) // (uniform: every thread takes this branch or none)
         {
-            if(active >= plan.alt_min_active && (int64_t)total_tiles * U >= (int64_t)plan.alt_min_rows * active)
+            if(active >= plan.alt_min_active && scan_total[3] >= (int64_t)plan.alt_min_rows * active)
                 rows_per_tile = plan.alt_rows_per_tile;
         }
         if(tid == 0)
@@ -370,7 +371,7 @@ struct OneShotShared
     int oeid[kOneShotMaxExperts];   // expert id written to sorted_expert_ids
     int ntiles[kOneShotMaxExperts]; // GEMM tiles
     int mbase[kOneShotMaxExperts];  // first GEMM tile
-    int wsum[5][kOneShotMaxExperts / kWave];
+    int wsum[6][kOneShotMaxExperts / kWave];
 };
 
 // last expert whose base[] is at or before t (experts that own nothing share their base with the next one that does,
@@ -476,14 +477,14 @@ __global__ __launch_bounds__(kScanBlock) void moe_sorting_oneshot_kernel(SortPar
     const int my_tiles = on_rank ? max(ceil_div(my_cnt, U), p.keep_empty ? 1 : 0) : 0;
     const bool planned = p.plan.tile_map != nullptr;
     const bool choice  = planned && p.plan.alt_rows_per_tile > 0;
-    const int rows     = my_tiles * U;
-    int v[5]           = {my_tiles, on_rank ? 1 : 0, on_rank && my_cnt > 0 ? 1 : 0,
-                          planned ? ceil_div(rows, p.plan.rows_per_tile) : 0, choice ? ceil_div(rows, p.plan.alt_rows_per_tile) : 0};
-    int ex[5], tot[5];
+    const int rows     = on_rank ? my_cnt : 0; // what the GEMMs compute: the padding is left out
+    int v[6]           = {my_tiles, on_rank ? 1 : 0, rows > 0 ? 1 : 0, planned ? ceil_div(rows, p.plan.rows_per_tile) : 0,
+                          choice ? ceil_div(rows, p.plan.alt_rows_per_tile) : 0, round_up(rows, 32)};
+    int ex[6], tot[6];
     if(wave < kOneShotMaxExperts / kWave)
     {
 #pragma unroll
-        for(int q = 0; q < 5; q++)
+        for(int q = 0; q < 6; q++)
         {
             ex[q] = wave_inclusive_scan(v[q]);
             if(lane == kWave - 1)
@@ -493,7 +494,7 @@ __global__ __launch_bounds__(kScanBlock) void moe_sorting_oneshot_kernel(SortPar
     }
     __syncthreads();
 #pragma unroll
-    for(int q = 0; q < 5; q++)
+    for(int q = 0; q < 6; q++)
     {
         tot[q] = 0;
 #pragma unroll
@@ -507,7 +508,7 @@ __global__ __launch_bounds__(kScanBlock) void moe_sorting_oneshot_kernel(SortPar
     }
     const int total_tiles = tot[0];
     const bool take_alt   = choice && tot[2] >= p.plan.alt_min_active &&
-                          (int64_t)total_tiles * U >= (int64_t)p.plan.alt_min_rows * tot[2];
+                          tot[5] >= (int64_t)p.plan.alt_min_rows * tot[2];
     const int gemm_tiles = take_alt ? tot[4] : tot[3];
     if(tid < E)
     {
@@ -574,7 +575,7 @@ __global__ __launch_bounds__(kScanBlock) void moe_sorting_oneshot_kernel(SortPar
         {
             const int e   = expert_of(sh.mbase, E, m);
             const int nt  = sh.ntiles[e];
-            const int er  = sh.tiles[e] * U;
+            const int er  = sh.cnt[e]; // (experts that own tiles are this rank's)
             const int per = round_up(ceil_div(er, nt), 32);
             const int j   = m - sh.mbase[e];
             const int r0  = sh.tbase[e] * U;
