@@ -410,7 +410,7 @@ mi355_fused_moe_static_ws(const mi355_fused_moe_traits* traits, const mi355_fuse
         return fail(MI355_MOE_E_INVALID, "fused_moe_static_ws: bad sizes (H=%d I=%d T=%d E=%d K=%d)", a->hidden_size,
                     a->intermediate_size, a->num_tokens, a->num_experts, a->topk);
     const size_t need = workspace_layout(*traits, a->num_tokens, a->num_experts, a->topk, a->hidden_size,
-                                         a->intermediate_size).total;
+                                         a->intermediate_size).least;
     if(need > kStaticWsBytes)
         return fail(MI355_MOE_E_WORKSPACE,
                     "fused_moe_static_ws: this problem needs a workspace of %zu bytes, the library-owned one holds %zu; "

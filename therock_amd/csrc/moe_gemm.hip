@@ -392,6 +392,9 @@ __global__ __launch_bounds__(256) void fill_u32x4_kernel(uint4* __restrict__ dst
 }
 
 // O[t, h] = sum over slots (in slot order) of top-k weight * bf16 partial, fp32 accumulate, one rounding
+// SLICED: the down GEMM was cut along K, part is fp32 [slices][tokens * topk][hidden] and a slot's row the sum of its
+// slices in slice order (see down_gemm_slice_bytes).
+template <bool SLICED>
 __global__ __launch_bounds__(256) void moe_combine_kernel(const unsigned char* __restrict__ part,
                                                            const int* __restrict__ inv,
                                                            const float* __restrict__ sorted_w,
@@ -400,7 +403,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const unsigned char* _
                                                            const float* __restrict__ slot_scale,
                                                            const float* __restrict__ bias,
                                                            const int* __restrict__ sorted_eid, int unit, int f16,
-                                                           const float* __restrict__ row_scale = nullptr)
+                                                           const float* __restrict__ row_scale, int slices)
 {
     // f16: the partial rows and the output are fp16 instead of bf16 (a uniform branch)
     const int t  = blockIdx.x;
@@ -427,6 +430,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const unsigned char* _
         int pos[kSlotsPerPass];
         float w[kSlotsPerPass];
         u32x4 v[kSlotsPerPass];
+        float row[kSlotsPerPass][8]; // (SLICED)
 #pragma unroll
         for(int j = 0; j < kSlotsPerPass; j++)
             pos[j] = k0 + j < topk ? __builtin_amdgcn_readfirstlane(inv[t * topk + k0 + j]) : -1;
@@ -442,7 +446,35 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const unsigned char* _
                     w[j] *= slot_scale[t * topk + k0 + j];
                 if(row_scale) // per-row scale of re-quantised e4m3 intermediate activations, in sorted-row order
                     w[j] *= row_scale[pos[j]];
-                v[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(part + ((int64_t)pos[j] * hidden + h0) * 2));
+                if constexpr(!SLICED)
+                    v[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(part + ((int64_t)pos[j] * hidden + h0) * 2));
+            }
+        }
+        if constexpr(SLICED)
+        {
+            using f32x4 = __attribute__((ext_vector_type(4))) float;
+#pragma unroll
+            for(int j = 0; j < kSlotsPerPass; j++)
+            {
+                const f32x4* src = reinterpret_cast<const f32x4*>(part) + ((int64_t)(t * topk + k0 + j) * hidden + h0) / 4;
+                const int64_t slice_f4 = (int64_t)gridDim.x * topk * hidden / 4;
+#pragma unroll
+                for(int i = 0; i < 8; i++)
+                    row[j][i] = 0.f;
+                if(pos[j] < 0) // (dropped slots have no row)
+                    continue;
+#pragma unroll 2
+                for(int s = 0; s < slices; s++)
+                {
+                    const f32x4 a = __builtin_nontemporal_load(src + s * slice_f4);
+                    const f32x4 b = __builtin_nontemporal_load(src + s * slice_f4 + 1);
+#pragma unroll
+                    for(int i = 0; i < 4; i++)
+                    {
+                        row[j][i] += a[i];
+                        row[j][4 + i] += b[i];
+                    }
+                }
             }
         }
 #pragma unroll
@@ -453,6 +485,12 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const unsigned char* _
 #pragma unroll
             for(int i = 0; i < 4; i++)
             {
+                if constexpr(SLICED)
+                {
+                    acc[2 * i] += w[j] * row[j][2 * i];
+                    acc[2 * i + 1] += w[j] * row[j][2 * i + 1];
+                    continue;
+                }
                 acc[2 * i] += w[j] * (f16 ? f16_bits_to_float(v[j][i] & 0xffffu) : __uint_as_float(v[j][i] << 16));
                 acc[2 * i + 1] += w[j] * (f16 ? f16_bits_to_float(v[j][i] >> 16) : __uint_as_float(v[j][i] & 0xffff0000u));
             }
@@ -631,6 +669,12 @@ int launch_grouped_gemm(int prec, bool gemm0, int mblk, bool use_decode, GemmPar
     const int pair = gemm0 && !p.gate_only ? 2 : 1;
     p.max_tiles    = max_tiles;
     p.n_ntiles     = ceil_div(p.n_out, (use_decode ? decode_tile_cols(false) : 256) / pair);
+    p.k_cols       = 0;
+    if(p.k_slice > 0) // (decode and large-tile kernels; set by the callers from down_gemm_slice_bytes)
+    {
+        p.k_cols   = p.n_ntiles;
+        p.n_ntiles = p.k_cols * ceil_div(p.k_bytes_w, p.k_slice);
+    }
     if(use_decode)
         return launch_gemm_decode(prec, gemm0, mblk, p, max_tiles, stream, y_i8);
     if(mblk > 4)
@@ -651,6 +695,70 @@ int launch_grouped_gemm(int prec, bool gemm0, int mblk, bool use_decode, GemmPar
 bool down_gemm_wants_decode(int experts, int64_t entries, int hidden)
 {
     return std::min<int64_t>(experts, entries) * ceil_div(hidden, 256) < device_info().num_cu;
+}
+
+// does the down GEMM run the decode kernel (mblk: the tile height, decode: the sizes allow the decode kernel)
+inline bool down_gemm_decode(int prec, int mblk, bool decode, bool y_i8, int experts, int64_t entries, int hidden)
+{
+    return decode && !(mblk == 2 && prec == MI355_MOE_INT8 && !y_i8) && down_gemm_wants_decode(experts, entries, hidden);
+}
+
+// Slices of K of the down GEMM, as weight bytes of K per slice; 0: not cut.
+//
+// With few experts the down GEMM has fewer tiles than the chip has compute units (hidden / 256 or hidden / 64 columns per
+// expert) while its K, the intermediate size, is long: 128 workgroups of 28 KB of K at 8 experts of 4096 x 14336.  A slice
+// then gets its own workgroup; the slices' shares stay in fp32 and the combine adds them in slice order, so what is rounded
+// to 16 bits is fewer numbers than before.  Whole pass, before -> after: 333 tokens of that layer in bf16 691 -> 586 us
+// (2 slices; 3: 629, 4: 610), one token 162 -> 131; 968 tokens of 9 fp16 experts 1856 x 11648 296 -> 205 (3);
+// 1964 tokens x 3 of 7 bf16 experts 1088 x 4864 376 -> 329 (2; 3: 361).
+//  * Decode kernel: a workgroup alone streams about 33 B/ns, so some 256 of them already take all of HBM's rate: slices up
+//    to that many workgroups (949 tiles: 229 us, cut in two 236), of two steps of 512 bytes at least, and only where the
+//    partial rows are small against the weights.
+//  * Large-tile kernel (one workgroup per compute unit): what a launch takes is its rounds of workgroups, each about
+//    3 us + operand bytes / 40 B/ns, and the combine's traffic at 4 TB/s, which grows with the slices (636 tokens x 3 of 7
+//    fp8 experts 5632 x 3200: 172 us, cut in two 224).  Cut where this says a tenth of it is gained.
+inline int down_gemm_slice_bytes(const mi355_fused_moe_traits& t, int64_t tokens, int topk, int experts, int hidden, int inter)
+{
+    const int mblk    = pick_mblk(t, tokens, topk, experts, hidden, inter);
+    const int64_t n   = tokens * topk;
+    const bool quant  = t.prec_i != MI355_MOE_BF16 && t.prec_i != MI355_MOE_FP16;
+    const bool decode = down_gemm_decode(t.prec_i, mblk, decode_tile(t, mblk), t.prec_i == MI355_MOE_INT8 && t.fused_quant != 0,
+                                         experts, n, hidden);
+    // (two candidate tile heights write one buffer: not cut)
+    if(n == 0 || (!decode && mblk <= 4) || alt_mblk_fused(t, tokens, topk, experts, hidden, inter) != 0)
+        return 0;
+    const int num_cu      = device_info().num_cu;
+    const int64_t active  = std::min<int64_t>(experts, n);
+    const int64_t rows    = ceil_div<int64_t>(n, active);
+    const int64_t tiles   = active * ceil_div<int64_t>(rows, mblk * 32) * ceil_div(hidden, decode ? decode_tile_cols(false) : 256);
+    const int64_t kb      = (int64_t)inter * (quant ? 1 : 2);
+    const int64_t share   = n * hidden * 8; // bytes a slice's partial rows move: written and read once
+    int slices            = 1;
+    if(decode)
+    {
+        if(tiles < num_cu)
+            slices = (int)std::min<int64_t>({ceil_div<int64_t>(num_cu, tiles), kb / 1024, 8});
+        while(slices > 1 && share * slices * 2 > active * hidden * kb)
+            slices--;
+    }
+    else if(tiles < 2 * num_cu)
+    {
+        const double tile_ns = (256.0 * kb + std::min<int64_t>(rows, mblk * 32) * (double)inter * y_bytes(t)) / 40.0;
+        auto ns = [&](int s) { return ceil_div<int64_t>(tiles * s, num_cu) * (tile_ns / s + 3000.0) + (s > 1 ? s : 0.5) * share / 4000.0; };
+        for(int s = 2; s <= 8; s++)
+            if(ns(s) < ns(slices) && ns(s) < 0.9 * ns(1))
+                slices = s;
+    }
+    if(slices < 2 || n * slices >= INT32_MAX)
+        return 0;
+    const int per = (int)round_up<int64_t>(ceil_div<int64_t>(kb, slices), 512);
+    return per < kb ? per : 0;
+}
+
+// bytes of the fp32 rows between a down GEMM cut along K and the combine
+inline size_t slice_rows_bytes(int64_t entries, int hidden, int k_bytes_w, int k_slice)
+{
+    return k_slice > 0 ? round_up<size_t>((size_t)ceil_div(k_bytes_w, k_slice) * entries * hidden * 4, 256) : 0;
 }
 
 } // namespace
@@ -719,7 +827,11 @@ WorkspaceLayout workspace_layout(const mi355_fused_moe_traits& t, int32_t tokens
     w.ys_off         = bump(t.prec_i == MI355_MOE_FP8 ? (size_t)w.ys_kb_stride * (inter / 32) : 0);
     w.yq_off         = bump(requant ? (size_t)round_up<int64_t>(w.max_pad, 16) * inter : 0);
     w.yrs_off        = bump(requant ? (size_t)w.max_pad * sizeof(float) : 0);
+    w.k_slice        = down_gemm_slice_bytes(t, tokens, topk, experts, hidden, inter);
+    const int w_b    = t.prec_i == MI355_MOE_BF16 || t.prec_i == MI355_MOE_FP16 ? 2 : 1;
     w.p_off          = bump((size_t)w.max_pad * hidden * 2);
+    w.least          = w.total;
+    w.total          = std::max(w.total, w.p_off + slice_rows_bytes((int64_t)tokens * topk, hidden, inter * w_b, w.k_slice));
     return w;
 }
 
@@ -760,8 +872,8 @@ int validate_fused_moegemm(const mi355_fused_moe_traits& t, const mi355_fused_mo
         return fail(MI355_MOE_E_INVALID, "fused_moegemm: bad sizes (H=%d I=%d T=%d E=%d K=%d stride=%d)", H, I, T, E,
                     K, a.stride_token);
     const WorkspaceLayout ws = workspace_layout(t, T, E, K, H, I);
-    if(ws_ptr == nullptr || ws_bytes < ws.total)
-        return fail(MI355_MOE_E_WORKSPACE, "fused_moegemm: workspace of %zu bytes needed, %zu given", ws.total,
+    if(ws_ptr == nullptr || ws_bytes < ws.least)
+        return fail(MI355_MOE_E_WORKSPACE, "fused_moegemm: workspace of %zu bytes needed, %zu given", ws.least,
                     ws_ptr ? ws_bytes : (size_t)0);
     if(reinterpret_cast<uintptr_t>(ws_ptr) % 256 != 0)
         return fail(MI355_MOE_E_INVALID, "fused_moegemm: workspace must be 256-byte aligned");
@@ -934,10 +1046,16 @@ int launch_fused_moegemm(const mi355_fused_moe_traits& t, const mi355_fused_moeg
     p.k_bytes_w      = I * eb;
     p.n_out          = H;
     p.n_total        = H;
+    const bool y_i8        = requant && !requant8;
+    const bool decode_down = down_gemm_decode(t.prec_i, mblk, decode, y_i8, E, (int64_t)T * K, H);
+    p.topk                 = K;
+    p.k_slice              = (decode_down || mblk > 4) && ws_bytes >= ws.total ? ws.k_slice : 0;
+    const int slices       = p.k_slice > 0 ? ceil_div(p.k_bytes_w, p.k_slice) : 1;
+    if(slices > 1)
+        p.out_row_bytes = (int64_t)H * 4;
     {
         KernelTimerGroup both(MI355_MOE_K_GEMM1, stream, alt != 0);
-        rc = launch_grouped_gemm(t.prec_i, false, mblk, decode && down_gemm_wants_decode(E, (int64_t)T * K, H), p,
-                                 max_tiles, stream, requant && !requant8);
+        rc = launch_grouped_gemm(t.prec_i, false, mblk, decode_down, p, max_tiles, stream, y_i8);
         if(rc != MI355_MOE_OK)
             return rc;
         if(alt)
@@ -954,11 +1072,11 @@ int launch_fused_moegemm(const mi355_fused_moe_traits& t, const mi355_fused_moeg
     // ---- combine
     {
     KernelTimer timer(MI355_MOE_K_COMBINE, stream);
-    hipLaunchKernelGGL(moe_combine_kernel, dim3(T, ceil_div(H, 256 * 8)), dim3(256), 0, stream, wsb + ws.p_off, inv,
+    hipLaunchKernelGGL(slices > 1 ? moe_combine_kernel<true> : moe_combine_kernel<false>, dim3(T, ceil_div(H, 256 * 8)), dim3(256), 0, stream, wsb + ws.p_off, inv,
                        static_cast<const float*>(a.sorted_weight_ptr), static_cast<unsigned char*>(a.o_ptr), K, H,
                        (int64_t)a.stride_token * 2, 0, static_cast<const float*>(nullptr), static_cast<const float*>(nullptr),
                        static_cast<const int*>(nullptr), 1, t.prec_i == MI355_MOE_FP16 ? 1 : 0,
-                       requant8 ? reinterpret_cast<const float*>(wsb + ws.yrs_off) : static_cast<const float*>(nullptr));
+                       requant8 ? reinterpret_cast<const float*>(wsb + ws.yrs_off) : static_cast<const float*>(nullptr), slices);
     }
     MI355_HIP_TRY(hipGetLastError());
     return MI355_MOE_OK;
@@ -970,10 +1088,11 @@ int launch_fused_moegemm(const mi355_fused_moe_traits& t, const mi355_fused_moeg
 namespace {
 struct FlatmmLayout
 {
-    size_t map_off, inv_off, p_off, ys_off, total;
+    size_t map_off, inv_off, p_off, ys_off, slices_off, least, total; // (see WorkspaceLayout)
     int64_t max_pad, ys_kb_stride;
     int32_t max_tiles;
     int mblk, hidden, inter;
+    int k_slice; // weight bytes of K per slice of the down GEMM, 0: not cut (see down_gemm_slice_bytes)
     int alt; // second tile height (32-row blocks) the tile-list pass may choose from the routing, 0: none (see alt_mblk)
     mi355_fused_moe_traits traits;
 };
@@ -1044,10 +1163,14 @@ int flatmm_layout(int kind, const mi355_moe_flatmm_args& a, FlatmmLayout& L)
     };
     L.map_off = bump(sizeof(int) * (kMapHdr + (size_t)kMapEnt * L.max_tiles));
     L.inv_off = bump(sizeof(int) * (size_t)a.NumTokens * a.TopK);
+    const int b_bytes = w8 || f8 ? 1 : 2;
+    L.k_slice = g1 || L.alt != 0 || a.k_padded_zeros > 0 ? 0 : down_gemm_slice_bytes(L.traits, a.NumTokens, a.TopK, a.NumExperts, L.hidden, L.inter);
     L.p_off   = bump(g1 ? 0 : (size_t)L.max_pad * L.hidden * 2);
     // the fp8 down GEMM runs the block-scaled MFMA: its input carries one scale per row, so every block scale is 2^0
     L.ys_kb_stride = round_up<int64_t>(L.max_pad, 256) + 512;
     L.ys_off       = bump(f8 && !g1 ? (size_t)L.ys_kb_stride * (L.inter / 32) : 0);
+    L.least        = L.total;
+    L.slices_off   = bump(slice_rows_bytes((int64_t)a.NumTokens * a.TopK, L.hidden, L.inter * b_bytes, L.k_slice));
     return MI355_MOE_OK;
 }
 } // namespace
@@ -1088,8 +1211,8 @@ int launch_moe_flatmm(int kind, const mi355_moe_flatmm_args& a, void* ws_ptr, si
             return fail(MI355_MOE_E_INVALID, "moe_flatmm: a, b and c must be 16-byte aligned");
     if(T == 0)
         return MI355_MOE_OK;
-    if(ws_ptr == nullptr || ws_bytes < L.total)
-        return fail(MI355_MOE_E_WORKSPACE, "moe_flatmm: workspace of %zu bytes needed, %zu given", L.total,
+    if(ws_ptr == nullptr || ws_bytes < L.least)
+        return fail(MI355_MOE_E_WORKSPACE, "moe_flatmm: workspace of %zu bytes needed, %zu given", L.least,
                     ws_ptr ? ws_bytes : (size_t)0);
     if(reinterpret_cast<uintptr_t>(ws_ptr) % 256 != 0)
         return fail(MI355_MOE_E_INVALID, "moe_flatmm: workspace must be 256-byte aligned");
@@ -1171,9 +1294,18 @@ int launch_moe_flatmm(int kind, const mi355_moe_flatmm_args& a, void* ws_ptr, si
         hipLaunchKernelGGL(fill_u32x4_kernel, dim3((unsigned)std::min<int64_t>(ceil_div<int64_t>(n16, 256), 4096)), dim3(256), 0,
                            stream, reinterpret_cast<uint4*>(p.y_scale), n16, 0x7f7f7f7fu);
     }
+    const bool decode_down = down_gemm_decode(prec, mblk, decode, false, E, (int64_t)T * K, H);
+    p.topk                 = K;
+    p.k_slice              = (decode_down || mblk > 4) && ws_bytes >= L.total ? L.k_slice : 0;
+    const int slices       = p.k_slice > 0 ? ceil_div(p.k_bytes_w, p.k_slice) : 1;
+    if(slices > 1)
+    {
+        p.out           = wsb + L.slices_off;
+        p.out_row_bytes = (int64_t)H * 4;
+    }
     {
         KernelTimerGroup both(MI355_MOE_K_GEMM1, stream, alt != 0);
-        rc = launch_grouped_gemm(prec, false, mblk, decode && down_gemm_wants_decode(E, (int64_t)T * K, H), p, L.max_tiles, stream);
+        rc = launch_grouped_gemm(prec, false, mblk, decode_down, p, L.max_tiles, stream);
         if(rc == MI355_MOE_OK && alt)
         {
             GemmParams pa = p;
@@ -1185,11 +1317,11 @@ int launch_moe_flatmm(int kind, const mi355_moe_flatmm_args& a, void* ws_ptr, si
         return rc;
     {
         KernelTimer timer(MI355_MOE_K_COMBINE, stream);
-        hipLaunchKernelGGL(moe_combine_kernel, dim3(T, ceil_div(H, 256 * 8)), dim3(256), 0, stream, wsb + L.p_off, inv,
+        hipLaunchKernelGGL(slices > 1 ? moe_combine_kernel<true> : moe_combine_kernel<false>, dim3(T, ceil_div(H, 256 * 8)), dim3(256), 0, stream, p.out, inv,
                            static_cast<const float*>(a.p_sorted_expert_weights), static_cast<unsigned char*>(a.c_ptr), K, H,
                            (int64_t)a.stride_C * 2, 1, f8 ? static_cast<const float*>(a.scale_m) : nullptr,
                            static_cast<const float*>(a.exp_bias), static_cast<const int*>(a.p_sorted_expert_ids), a.block_m,
-                           prec == MI355_MOE_FP16 ? 1 : 0);
+                           prec == MI355_MOE_FP16 ? 1 : 0, static_cast<const float*>(nullptr), slices);
     }
     MI355_HIP_TRY(hipGetLastError());
     return MI355_MOE_OK;

@@ -16,8 +16,10 @@ struct WorkspaceLayout
     int64_t ys_kb_stride;
     size_t yq_off;     // int8 (e4m3) copy of Y [max_pad, inter] and ...
     size_t yrs_off;    // ... its fp32 per-row scales [max_pad] (int8 and fp8 paths with fused_quant 1 / 2 only)
-    size_t p_off;      // partial outputs per sorted row [max_pad, hidden] bf16
+    size_t p_off;      // partial outputs per sorted row [max_pad, hidden] bf16, or per slice and slot in fp32
+    int k_slice;       // weight bytes of K per slice of the down GEMM (0: not cut), see down_gemm_slice_bytes
     size_t total;
+    size_t least;      // without the room for a down GEMM cut along K: a call with less than total bytes is not cut
     int64_t max_pad;
     int32_t max_tiles; // upper bound of M tiles
 };

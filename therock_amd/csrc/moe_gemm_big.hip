@@ -172,7 +172,8 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
         return;
     const int expert = tile.expert;
     const int row0   = tile.row0;
-    const int nt     = tile.nt;
+    const int slice  = !GEMM0 && p.k_cols > 0 ? tile.nt / p.k_cols : 0; // slice of K (down GEMM)
+    const int nt     = tile.nt - slice * p.k_cols;
     const int nrows  = tile.nrows;
     const int nmb    = ceil_div(nrows, 32);
     const bool paired = GEMM0 && !p.gate_only; // gate rows paired with up rows (see run_epilogue)
@@ -267,7 +268,19 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
     const int x_step      = (!GEMM0 && p.y_slab > 0) ? 1024 : kStepKB; // bytes between token steps
 
     const uint32_t lds_base = lds_offset(lds);
-    const int kt_count      = p.k_bytes_x / kStepKB; // compute steps (even; a multiple of four with int8 weights)
+    // compute steps (even; a multiple of four with int8 weights): this workgroup's slice of K, whose first bytes the
+    // base addresses point at (a slice is a multiple of 512 weight bytes)
+    int kt_count = p.k_bytes_x / kStepKB;
+    const unsigned char* ys_base = p.y_scale;
+    if(!GEMM0 && p.k_cols > 0)
+    {
+        const int slice_steps = p.k_slice / (kW8 ? kStepKB / 2 : kStepKB);
+        const int step0       = slice * slice_steps;
+        kt_count              = min(kt_count - step0, slice_steps);
+        dbase = uniform_ptr(dbase + (w_role ? (int64_t)slice * weight_k_advance(p, p.k_slice) : (int64_t)step0 * x_step));
+        if constexpr(kMx)
+            ys_base += step0 * ys_step;
+    }
     const int n_wunits      = kW8 ? kt_count / 2 : kt_count; // two units (row halves) per 128 bytes of weight K
 
     // weight role: unit u (half u & 1) -> ring slot u % 6
@@ -309,7 +322,7 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
             if(j < groups)
                 dma16(src, doff[j], __builtin_amdgcn_readfirstlane(sbase + j * 4096));
         if constexpr(kMx)
-            dma4(p.y_scale + x * ys_step, doff[5],
+            dma4(ys_base + x * ys_step, doff[5],
                  __builtin_amdgcn_readfirstlane(lds_base + kYsOffset + (x % kXStages) * kYsStageBytes +
                                                 (q4 >> 1) * kYsRows + (q4 & 1) * 256));
     };
@@ -684,7 +697,7 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
     }
 
     // ---- epilogue
-    run_epilogue<MODE, GEMM0, kMaxNB, false>(p, acc, expert, row0, nrows, wt * 32, 64, nb_w, n_base, ww, r32, kg);
+    run_epilogue<MODE, GEMM0, kMaxNB, false>(p, acc, expert, row0, nrows, wt * 32, 64, nb_w, n_base, ww, r32, kg, slice);
 }
 
 template <int MODE, bool GEMM0, bool WPERM>

@@ -58,7 +58,8 @@ __global__ __launch_bounds__(kBlock, (NXB > 1 || MODE == kBf16W8 || MODE == kFp8
         return;
     const int expert = tile.expert;
     const int row0   = tile.row0;
-    const int nt     = tile.nt;
+    const int slice  = !GEMM0 && p.k_cols > 0 ? tile.nt / p.k_cols : 0; // slice of K (down GEMM)
+    const int nt     = tile.nt - slice * p.k_cols;
     const int nrows  = min(tile.nrows, 32 * NXB);
     // a tile of at most 32 rows leaves the second token block out: no LDS traffic and no MFMAs for it (its loads are
     // masked row by row anyway)
@@ -191,7 +192,11 @@ __global__ __launch_bounds__(kBlock, (NXB > 1 || MODE == kBf16W8 || MODE == kFp8
             for(int v = 0; v < 16; v++)
                 acc[i][b][v] = 0;
 
-    const int kt_count = ceil_div(p.k_bytes_w, kDecWKB);
+    // the steps [kt_first, kt_count) of K are this workgroup's
+    const int kt_all   = ceil_div(p.k_bytes_w, kDecWKB);
+    const int kt_slice = !GEMM0 && p.k_cols > 0 ? p.k_slice / kDecWKB : kt_all;
+    const int kt_first = slice * kt_slice;
+    const int kt_count = min(kt_all, kt_first + kt_slice);
     auto k_step = [&](int kt, auto buf_tag) __attribute__((always_inline)) {
         constexpr int B = decltype(buf_tag)::value;
         auto& xv        = xv_[B];
@@ -253,10 +258,10 @@ __global__ __launch_bounds__(kBlock, (NXB > 1 || MODE == kBf16W8 || MODE == kFp8
     };
     using B0 = std::integral_constant<int, 0>;
     using B1 = std::integral_constant<int, 1>;
-    load_tiles(0, B0{});
-    if(1 < kt_count)
-        load_tiles(1, B1{});
-    for(int kt = 0; kt < kt_count; kt += 2)
+    load_tiles(kt_first, B0{});
+    if(kt_first + 1 < kt_count)
+        load_tiles(kt_first + 1, B1{});
+    for(int kt = kt_first; kt < kt_count; kt += 2)
     {
         k_step(kt, B0{});
         if(kt + 1 < kt_count)
@@ -299,7 +304,7 @@ __global__ __launch_bounds__(kBlock, (NXB > 1 || MODE == kBf16W8 || MODE == kFp8
                     acc[i][b][v] += red[(((w * NXB + i) * 2 + b) * 16 + v) * 64 + lane];
         }
 
-    run_epilogue<MODE, GEMM0, NXB, true>(p, acc, expert, row0, nrows, 0, 32, ceil_div(nrows, 32), n_base, 0, r32, kg);
+    run_epilogue<MODE, GEMM0, NXB, true>(p, acc, expert, row0, nrows, 0, 32, ceil_div(nrows, 32), n_base, 0, r32, kg, slice);
 }
 
 template <int MODE, bool GEMM0, int NXB, bool WPERM>

@@ -84,6 +84,12 @@ struct GemmParams
     // x [topk, tokens, .] with scales [topk, tokens] (ck_tile's MoeSmoothquant output, moe_sorting_kernel.hpp:82-83);
     // x_slot_major = 1 selects that addressing, 0 the usual row per token
     int x_slot_major;
+    // Down GEMM cut along K (k_cols > 0; see down_gemm_slice_bytes): the tile list's column index counts k_cols column tiles
+    // per slice of k_slice weight bytes of K, n_ntiles = slices * k_cols, and every slice stores its share of the dot
+    // products in fp32, one row per (slice, token * topk + slot): out [slices, tokens * topk, out_row_bytes].
+    int k_cols;
+    int k_slice;
+    int topk;
 };
 
 // row of the gate+up GEMM's activations (and index of its per-row scale) a sorted id refers to
@@ -517,6 +523,17 @@ __device__ __attribute__((always_inline)) inline void epilogue_gemm1(const GemmP
         y[v] = static_cast<float>(acc[v]) * (sa * ds[v]);
     if(p.bias != nullptr || p.n_padded > 0) // uniform: stand-alone down GEMM with a bias or padded rows
         bias_and_padding(p, y, expert, col0);
+    if(p.k_cols > 0) // uniform: a slice of K, its share stays in fp32
+    {
+        if(store)
+        {
+            float4* d4 = reinterpret_cast<float4*>(p.out + prow * p.out_row_bytes + (int64_t)col0 * 4);
+#pragma unroll
+            for(int q = 0; q < 4; q++)
+                d4[q] = make_float4(y[4 * q], y[4 * q + 1], y[4 * q + 2], y[4 * q + 3]);
+        }
+        return;
+    }
     uint4 o0, o1;
     o0.x = pack_out2<MODE>(y[0], y[1]);   o0.y = pack_out2<MODE>(y[2], y[3]);
     o0.z = pack_out2<MODE>(y[4], y[5]);   o0.w = pack_out2<MODE>(y[6], y[7]);
@@ -541,7 +558,7 @@ struct EpilogueRows
 {
     float sa[NBLK];  // per-row scale
     bool real[NBLK]; // the row holds a token (not a padding id)
-    int orow[NBLK];  // output row (the launchers keep tokens * topk below 2^31)
+    int orow[NBLK];  // output row (the launchers keep tokens * topk, and slices * tokens * topk, below 2^31)
 };
 struct EpilogueColumns
 {
@@ -572,7 +589,7 @@ __device__ __attribute__((always_inline)) inline EpilogueColumns epilogue_column
 
 template <int MODE, bool GEMM0, int NBLK, bool SKIP_PAD>
 __device__ __attribute__((always_inline)) inline void load_epilogue_rows(const GemmParams& p, EpilogueRows<NBLK>& o, int row0, int nrows, int first_row,
-                                          int row_step, int r32)
+                                          int row_step, int r32, int slice = 0)
 {
 #pragma unroll
     for(int i = 0; i < NBLK; i++)
@@ -580,7 +597,7 @@ __device__ __attribute__((always_inline)) inline void load_epilogue_rows(const G
         o.sa[i]   = 1.0f;
         o.real[i] = true;
         o.orow[i] = row0 + first_row + i * row_step + r32;
-        if((GEMM0 && (p.x_scale != nullptr || p.slot_rows > 0)) || (!GEMM0 && SKIP_PAD))
+        if((GEMM0 && (p.x_scale != nullptr || p.slot_rows > 0)) || (!GEMM0 && (SKIP_PAD || p.k_cols > 0)))
         {
             const int r   = min(first_row + i * row_step + r32, nrows - 1); // clamped: always a valid cell
             const int sid = p.sorted_ids[row0 + r];
@@ -593,6 +610,8 @@ __device__ __attribute__((always_inline)) inline void load_epilogue_rows(const G
                 if(p.slot_rows > 0)
                     o.orow[i] = o.real[i] ? (int)slot_row(sid, p.slot_rows) : 0;
             }
+            else if(p.k_cols > 0)
+                o.orow[i] = o.real[i] ? slice * p.tokens * p.topk + (int)slot_row(sid, p.topk) : 0;
         }
         if constexpr(!GEMM0 && MODE == kI8)
         {
@@ -617,14 +636,14 @@ __device__ __attribute__((always_inline)) inline void pin_epilogue_rows(Epilogue
 
 template <int MODE, bool GEMM0, int NBLK, bool SKIP_PAD>
 __device__ __attribute__((always_inline)) inline void load_epilogue(const GemmParams& p, EpilogueOperands<NBLK>& o, int expert, int row0, int nrows,
-                                     int first_row, int row_step, int n_base, int wblk, int r32, int kg)
+                                     int first_row, int row_step, int n_base, int wblk, int r32, int kg, int slice = 0)
 {
     o.cols             = epilogue_columns<GEMM0>(p, n_base, wblk, kg);
     const float* sbase = p.w_scale ? p.w_scale + (int64_t)expert * p.n_total : nullptr;
     load_channel_scales(sbase && o.cols.a_ok ? sbase + o.cols.col_a : nullptr, o.sc0);
     load_channel_scales(sbase && o.cols.b_ok ? sbase + (o.cols.paired ? p.n_out + o.cols.col_a : o.cols.col_b) : nullptr,
                         o.sc1);
-    load_epilogue_rows<MODE, GEMM0, NBLK, SKIP_PAD>(p, o.rows, row0, nrows, first_row, row_step, r32);
+    load_epilogue_rows<MODE, GEMM0, NBLK, SKIP_PAD>(p, o.rows, row0, nrows, first_row, row_step, r32, slice);
 }
 
 // Every load of load_epilogue completes here, on every path: a load left pending on a path that does not use
@@ -659,9 +678,9 @@ __device__ __attribute__((always_inline)) inline void apply_epilogue_block(const
     {
         const bool in_tile = r < nrows;
         if(c.a_ok)
-            epilogue_gemm1<MODE>(p, acc[0], sc0, rows.sa[i], row0 + r, in_tile && rows.real[i], c.col_a, expert);
+            epilogue_gemm1<MODE>(p, acc[0], sc0, rows.sa[i], rows.orow[i], in_tile && rows.real[i], c.col_a, expert);
         if(c.b_ok)
-            epilogue_gemm1<MODE>(p, acc[1], sc1, rows.sa[i], row0 + r, in_tile && rows.real[i], c.col_b, expert);
+            epilogue_gemm1<MODE>(p, acc[1], sc1, rows.sa[i], rows.orow[i], in_tile && rows.real[i], c.col_b, expert);
     }
 }
 
@@ -685,10 +704,10 @@ __device__ __attribute__((always_inline)) inline void apply_epilogue(const GemmP
 template <int MODE, bool GEMM0, int NBLK, bool SKIP_PAD>
 __device__ __attribute__((always_inline)) inline void run_epilogue(const GemmParams& p, typename ModeTraits<MODE>::Acc (&acc)[NBLK][2], int expert,
                                     int row0, int nrows, int first_row, int row_step, int nblk_live, int n_base,
-                                    int wblk, int r32, int kg)
+                                    int wblk, int r32, int kg, int slice = 0)
 {
     EpilogueOperands<NBLK> o;
-    load_epilogue<MODE, GEMM0, NBLK, SKIP_PAD>(p, o, expert, row0, nrows, first_row, row_step, n_base, wblk, r32, kg);
+    load_epilogue<MODE, GEMM0, NBLK, SKIP_PAD>(p, o, expert, row0, nrows, first_row, row_step, n_base, wblk, r32, kg, slice);
     pin_epilogue(o);
     apply_epilogue<MODE, GEMM0, NBLK>(p, acc, o, row0, nrows, first_row, row_step, nblk_live, r32, kg, expert);
 }
