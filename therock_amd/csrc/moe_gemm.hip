@@ -561,6 +561,43 @@ inline bool big_tile_ok(const mi355_fused_moe_traits& t, int64_t tokens, int top
            big_tile_supported(t.prec_i, hidden * eb, inter * y_b, y_b == 1);
 }
 
+// Few experts or a narrow layer: the gate+up GEMM has fewer large tiles than the chip has compute units, and smaller
+// tiles, which re-read weights and tokens more often, win by filling it.  What decides is measured on layers of
+// 4 .. 32 experts, hidden 1024 .. 4096, inter 512 .. 2048 (whole passes in us, large tiles / 128 / 64 rows; 32 for fp8):
+//   bf16, 8 x 1024 x 512, 160 rows per expert (32 large tiles)  60 / 54 / 39    16 x 2048 x 512, 300 (64)  127 / 96 / 128
+//   bf16, 4 x 1024 x 1024, 100 (32)  55 / 66 / 33               16 x 4096 x 1024, 600 (256)  272 / 398 / 553: not narrow
+//   bf16, 32 x 2048 x 768, 100 (192)  96 / 109 / 116            16 x 4096 x 1024, 160 (128)  152 / 160 / 186
+//   fp8, 8 x 1024 x 2048, 300 (128)  98 / 79 / 67               16 x 1024 x 1024, 160 (128)  61 / 57 / 50
+//   fp8, 4 x 4096 x 2048, 44 (64)  69 / 82 / 75 / 47            32 x 2048 x 768, 300 (192)  132 / 141 / 138
+// So: the large tiles stay where those of both GEMMs together are 5/4 of the compute units or more (the 16 x 4096 x 1024
+// rows above), for 16-bit and int8 operands also up to 256 rows from half the compute units on; else 64-row tiles (fp8
+// with few rows: 32), or, for 16-bit and int8 operands and more than 128 rows, 128-row tiles where those fill half the
+// chip.  Layers under 2^19 weights per matrix are a handful of workgroups either way and are left to the rules of
+// pick_mblk.  Returns 0: no choice made.
+inline int pick_mblk_narrow(const mi355_fused_moe_traits& t, int64_t avg, int experts, int hidden, int inter, bool big_ok, bool fits)
+{
+    const int64_t cu = device_info().num_cu, cols = ceil_div(inter, t.gate_only ? 256 : 128);
+    const int64_t big_rows = experts * ceil_div<int64_t>(avg, big_tile_rows()), mid = experts * ceil_div<int64_t>(avg, 128) * cols;
+    const int64_t big = big_rows * cols, both = big + big_rows * ceil_div(hidden, 256);
+    if((int64_t)hidden * inter < (1 << 19) || big >= cu)
+        return 0;
+    const bool fills = big > cu / 2 || both >= cu * 5 / 4;
+    if(t.prec_i == MI355_MOE_FP8)
+    {
+        if(big_ok && avg >= 160 && fills)
+            return big_tile_rows() / 32;
+        if(avg <= (experts <= 8 ? 64 : 48) && big <= cu / 4)
+            return 1;
+        return big <= cu / 2 || (avg < 160 && mid < cu) ? 2 : 0;
+    }
+    const bool w8 = t.prec_i == MI355_MOE_INT8 && t.fused_quant == 0; // (64-row tiles have no decode kernel for its down GEMM)
+    if(big_ok && avg > 56 && (fills || (big == cu / 2 && avg < 256 && (avg > 64 || w8))))
+        return big_tile_rows() / 32;
+    if(!fits || big > cu / 2)
+        return 0;
+    return avg <= 128 || mid < cu / 2 || (mid == cu / 2 && experts <= 8) ? 2 : 4;
+}
+
 // 32-row blocks per M tile, from the expected rows per expert; big_tile_rows() / 32 selects the large-tile kernel
 inline int pick_mblk(const mi355_fused_moe_traits& t, int64_t tokens, int topk, int experts, int hidden, int inter)
 {
@@ -578,7 +615,12 @@ inline int pick_mblk(const mi355_fused_moe_traits& t, int64_t tokens, int topk, 
         return 2;
     const int64_t big_tiles = (int64_t)experts * std::max<int64_t>(1, ceil_div<int64_t>(avg, big_tile_rows())) * ceil_div(inter, 128);
     const bool big_ok = big_tile_ok(t, tokens, topk, experts, hidden, inter);
-    if(big_ok && (avg >= 160 || (avg >= 28 && big_tiles >= device_info().num_cu)))
+    if(big_ok && avg >= 28 && big_tiles >= device_info().num_cu)
+        return big_tile_rows() / 32;
+    const int narrow = avg > 32 ? pick_mblk_narrow(t, avg, experts, hidden, inter, big_ok, fits) : 0;
+    if(narrow > 0)
+        return narrow;
+    if(big_ok && avg >= 160)
         return big_tile_rows() / 32;
     if(avg <= 32)
         return 1;
