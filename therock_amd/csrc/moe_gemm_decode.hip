@@ -70,33 +70,20 @@ __global__ __launch_bounds__(kBlock, (NXB > 1 || MODE == kBf16W8 || MODE == kFp8
     // ---- global -> register staging assignments: 32 consecutive lanes fetch 512 contiguous bytes
     const int xchunk = tid % (kXKB / 16);
     const int xrow   = tid / (kXKB / 16);
-    // addresses are a uniform base plus a 32-bit byte offset (the launcher checks that this suffices)
-    uint32_t xoff[kXLoads];
-    bool xvalid[kXLoads];
+    // The sorted ids of the token rows: fetched first, used only after the first step's weights are on their way.  Nothing
+    // of the weights' addresses depends on them, and a workgroup's life is short enough (some 10 us) for a round trip to
+    // show: with the epilogue's operands fetched behind the K loop's last step instead of after the reduction, 256
+    // Zipf-routed tokens of 128 int8 experts 247.7 -> 242.9 us.  (The second step's weights ahead of the ids as well:
+    // two-block tiles lose 1 to 2 %, their first step then waits for both.)
+    int sid[kXLoads];
+    const bool by_id = GEMM0 || p.slot_rows > 0;
 #pragma unroll
     for(int j = 0; j < kXLoads; j++)
     {
         const int r = xrow + kXRowsPerPass * j;
-        if constexpr(GEMM0)
-        {
-            int sid = p.tokens;
-            if(r < nrows)
-                sid = p.sorted_ids[row0 + r];
-            xvalid[j] = (sid & 0xffffff) < p.tokens;
-            xoff[j]   = (xvalid[j] ? token_row(p, sid) : 0u) * (uint32_t)p.x_row_bytes + xchunk * 16;
-        }
-        else
-        {
-            xvalid[j]   = r < nrows;
-            int64_t src = row0 + (xvalid[j] ? r : 0);
-            if(p.slot_rows > 0)
-            {
-                const int sid = p.sorted_ids[src];
-                xvalid[j]     = xvalid[j] && (sid & 0xffffff) < p.tokens;
-                src           = xvalid[j] ? slot_row(sid, p.slot_rows) : 0;
-            }
-            xoff[j] = (uint32_t)src * (uint32_t)p.x_row_bytes + xchunk * 16;
-        }
+        sid[j]      = r < nrows ? 0 : p.tokens;
+        if(by_id && r < nrows)
+            sid[j] = p.sorted_ids[row0 + r];
     }
     // Which 16 bytes of the 64 x 512-byte weight tile thread `tid` fetches with load j, as (tile row, 16-byte chunk) =
     // (w_row0 + w_row_add(j), w_chunk0 + w_chunk_add(j)).  Row-major weights: 32 consecutive threads walk the 512
@@ -140,19 +127,9 @@ __global__ __launch_bounds__(kBlock, (NXB > 1 || MODE == kBf16W8 || MODE == kFp8
         ys_next_[0][i] = ys_next_[1][i] = ys_cur[i] = 0x7f7f7f7fu;
     const uint4 zero4 = {0u, 0u, 0u, 0u};
 
-    auto load_tiles = [&](int kt, auto buf_tag) __attribute__((always_inline)) {
+    auto load_w = [&](int kt, auto buf_tag) __attribute__((always_inline)) {
         constexpr int B   = decltype(buf_tag)::value;
-        auto& xv          = xv_[B];
         auto& wv          = wv_[B];
-        auto& ys_next     = ys_next_[B];
-        const int kx = kt * kXKB + xchunk * 16;
-#pragma unroll
-        for(int j = 0; j < kXLoads; j++)
-        {
-            xv[j] = zero4;
-            if(xvalid[j] && kx < p.k_bytes_x)
-                xv[j] = *reinterpret_cast<const uint4*>(p.x + (xoff[j] + (uint32_t)(kt * kXKB)));
-        }
         const int kw = kt * kDecWKB + w_chunk0 * 16;
 #pragma unroll
         for(int j = 0; j < kWLoads; j++)
@@ -164,6 +141,45 @@ __global__ __launch_bounds__(kBlock, (NXB > 1 || MODE == kBf16W8 || MODE == kFp8
                 const u32x4_t t = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(wbase + (woff[j] + (uint32_t)(kt * w_kadv))));
                 wv[j]           = make_uint4(t[0], t[1], t[2], t[3]);
             }
+        }
+    };
+
+    // the steps [kt_first, kt_count) of K are this workgroup's
+    const int kt_all   = ceil_div(p.k_bytes_w, kDecWKB);
+    const int kt_slice = !GEMM0 && p.k_cols > 0 ? p.k_slice / kDecWKB : kt_all;
+    const int kt_first = slice * kt_slice;
+    const int kt_count = min(kt_all, kt_first + kt_slice);
+    using B0 = std::integral_constant<int, 0>;
+    using B1 = std::integral_constant<int, 1>;
+    load_w(kt_first, B0{});
+    __builtin_amdgcn_sched_barrier(0); // (the scheduler would put the ids' wait first)
+
+    // addresses are a uniform base plus a 32-bit byte offset (the launcher checks that this suffices)
+    uint32_t xoff[kXLoads];
+    bool xvalid[kXLoads];
+#pragma unroll
+    for(int j = 0; j < kXLoads; j++)
+    {
+        const int r   = xrow + kXRowsPerPass * j;
+        xvalid[j]     = r < nrows && (!by_id || (sid[j] & 0xffffff) < p.tokens);
+        uint32_t src  = row0 + r;
+        if constexpr(GEMM0)
+            src = token_row(p, sid[j]);
+        else if(p.slot_rows > 0)
+            src = (uint32_t)slot_row(sid[j], p.slot_rows);
+        xoff[j] = (xvalid[j] ? src : 0u) * (uint32_t)p.x_row_bytes + xchunk * 16;
+    }
+    auto load_x = [&](int kt, auto buf_tag) __attribute__((always_inline)) {
+        constexpr int B   = decltype(buf_tag)::value;
+        auto& xv          = xv_[B];
+        auto& ys_next     = ys_next_[B];
+        const int kx = kt * kXKB + xchunk * 16;
+#pragma unroll
+        for(int j = 0; j < kXLoads; j++)
+        {
+            xv[j] = zero4;
+            if(xvalid[j] && kx < p.k_bytes_x)
+                xv[j] = *reinterpret_cast<const uint4*>(p.x + (xoff[j] + (uint32_t)(kt * kXKB)));
         }
         if constexpr(kMx)
         {
@@ -192,11 +208,6 @@ __global__ __launch_bounds__(kBlock, (NXB > 1 || MODE == kBf16W8 || MODE == kFp8
             for(int v = 0; v < 16; v++)
                 acc[i][b][v] = 0;
 
-    // the steps [kt_first, kt_count) of K are this workgroup's
-    const int kt_all   = ceil_div(p.k_bytes_w, kDecWKB);
-    const int kt_slice = !GEMM0 && p.k_cols > 0 ? p.k_slice / kDecWKB : kt_all;
-    const int kt_first = slice * kt_slice;
-    const int kt_count = min(kt_all, kt_first + kt_slice);
     auto k_step = [&](int kt, auto buf_tag) __attribute__((always_inline)) {
         constexpr int B = decltype(buf_tag)::value;
         auto& xv        = xv_[B];
@@ -213,7 +224,10 @@ __global__ __launch_bounds__(kBlock, (NXB > 1 || MODE == kBf16W8 || MODE == kFp8
             ys_cur[i] = ys_next_[B][i];
         __syncthreads();
         if(kt + 2 < kt_count)
-            load_tiles(kt + 2, buf_tag);
+        {
+            load_x(kt + 2, buf_tag);
+            load_w(kt + 2, buf_tag);
+        }
         const unsigned char* xp = lds_x + r32 * kXStride + wave * kWaveWB * kXMul;
 #pragma unroll
         for(int s = 0; s < kSteps; s++)
@@ -256,11 +270,12 @@ __global__ __launch_bounds__(kBlock, (NXB > 1 || MODE == kBf16W8 || MODE == kFp8
         }
         __syncthreads();
     };
-    using B0 = std::integral_constant<int, 0>;
-    using B1 = std::integral_constant<int, 1>;
-    load_tiles(kt_first, B0{});
+    load_x(kt_first, B0{});
     if(kt_first + 1 < kt_count)
-        load_tiles(kt_first + 1, B1{});
+    {
+        load_x(kt_first + 1, B1{});
+        load_w(kt_first + 1, B1{});
+    }
     for(int kt = kt_first; kt < kt_count; kt += 2)
     {
         k_step(kt, B0{});
@@ -271,6 +286,10 @@ __global__ __launch_bounds__(kBlock, (NXB > 1 || MODE == kBf16W8 || MODE == kFp8
     // ---- add the four K slices: waves 1..3 park their accumulators in LDS, wave 0 sums in wave order
     using AccElem   = decltype(acc[0][0][0] + acc[0][0][0]);
     AccElem* red    = reinterpret_cast<AccElem*>(lds); // [3][NXB][2][16][64]
+    // the epilogue's operands travel while the slices are added
+    EpilogueOperands<NXB> eo;
+    if(wave == 0)
+        load_epilogue<MODE, GEMM0, NXB, true>(p, eo, expert, row0, nrows, 0, 32, n_base, 0, r32, kg, slice);
     if(wave > 0)
     {
 #pragma unroll
@@ -304,7 +323,8 @@ __global__ __launch_bounds__(kBlock, (NXB > 1 || MODE == kBf16W8 || MODE == kFp8
                     acc[i][b][v] += red[(((w * NXB + i) * 2 + b) * 16 + v) * 64 + lane];
         }
 
-    run_epilogue<MODE, GEMM0, NXB, true>(p, acc, expert, row0, nrows, 0, 32, ceil_div(nrows, 32), n_base, 0, r32, kg, slice);
+    pin_epilogue(eo);
+    apply_epilogue<MODE, GEMM0, NXB>(p, acc, eo, row0, nrows, 0, 32, ceil_div(nrows, 32), r32, kg, expert);
 }
 
 template <int MODE, bool GEMM0, int NXB, bool WPERM>
