@@ -557,6 +557,16 @@ inline bool big_tile_ok(const mi355_fused_moe_traits& t, int64_t tokens, int top
 {
     const int eb  = (t.prec_i == MI355_MOE_BF16 || t.prec_i == MI355_MOE_FP16) ? 2 : 1;
     const int y_b = y_bytes(t);
+    // 8-bit rows of an odd number of 64-byte steps run on the large tiles where that is clearly the better: layers of
+    // 2^22 weights per matrix and 160 rows per expert, or so few output columns that the down GEMM has to be cut along K,
+    // which the small tiles cannot be (fp8, small -> large tiles: 16 x 4160 x 4096 at 190 / 600 rows 385 -> 302, 724 -> 579
+    // us, at 40 rows 214 -> 222; 8 x 832 x 8192 at 90 rows 182 -> 83; 64 x 1344 x 768 at 90 rows 86 -> 110).
+    if((hidden * eb) % 128 != 0)
+    {
+        const bool few_columns = experts * ceil_div(hidden, 256) < device_info().num_cu / 2;
+        if((int64_t)hidden * inter < (1 << 22) || (tokens * topk / std::max(experts, 1) < 160 && !few_columns))
+            return false;
+    }
     return t.block_m % 16 == 0 && offsets_fit(t, tokens, topk, experts, hidden, inter) &&
            big_tile_supported(t.prec_i, hidden * eb, inter * y_b, y_b == 1);
 }

@@ -151,6 +151,10 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
     // step k then has to guarantee the data of step k+1: every transfer runs one step further ahead.
     constexpr bool kPipe  = !kW8 && !kMx;
     constexpr bool kXPair = kPipe && GEMM0; // 128-byte token stages
+    // 8-bit rows of an odd number of 64-byte steps (hidden sizes that are odd multiples of 64): the last 128-byte window
+    // has only its first half.  Lanes that would fetch the second half (the next row's bytes, past the tensor's end in its
+    // last row) fetch the first one again, and the last step has no partner, so nothing reads what they fetched.
+    constexpr bool kOddK = kXPair && (MODE == kI8 || MODE == kFp8);
     constexpr int kWS     = kXPair ? kWSlotsPair : kWSlots;
     constexpr int kXO     = kXPair ? kXOffsetPair : kXOffset;
 
@@ -281,7 +285,8 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
         if constexpr(kMx)
             ys_base += step0 * ys_step;
     }
-    const int n_wunits      = kW8 ? kt_count / 2 : kt_count; // two units (row halves) per 128 bytes of weight K
+    const bool odd_k        = kOddK && (kt_count & 1) != 0;
+    const int n_wunits      = kW8 ? kt_count / 2 : kt_count + (odd_k ? 1 : 0); // two units (row halves) per 128 bytes of weight K
 
     // weight role: unit u (half u & 1) -> ring slot u % 6
     // Weights no other row tile re-reads (the expert has a single one) are fetched non-temporal: measured
@@ -551,6 +556,49 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                     __builtin_amdgcn_sched_barrier(0);
                 });
             };
+            if constexpr(kOddK)
+            {
+                // the last window's units go out in steps kt_count - 5 and kt_count - 4 (rows of five steps or more: see
+                // big_tile_supported) and are the last to go out: from there on the lanes of the missing half fetch the
+                // other one
+                int k   = 0;
+                int end = odd_k ? kt_count - 5 : kt_count;
+                for(;;)
+                {
+                    for(; k < end; k += 2)
+                    {
+                        step(k, H0{});
+                        step(k + 1, H1{});
+                    }
+                    if(!odd_k || end == kt_count - 1)
+                        break;
+                    end = kt_count - 1;
+                    if(w_role)
+                    {
+#pragma unroll
+                        for(int j = 0; j < 4; j++)
+                        {
+                            const int rih   = (q4 + 4 * j) * 8 + (WPERM ? lane & 7 : lane >> 3);
+                            const int chunk = WPERM ? (lane >> 3) ^ (((q4 + 4 * j) >> 1) & 1) : (lane & 7) ^ weight_row_swizzle(rih);
+                            const uint32_t back = (chunk & 4) ? (WPERM ? 1024u : 64u) : 0u;
+                            doff[j] -= back;
+                            doff[4 + j] -= back;
+                        }
+                    }
+                    else
+                    {
+#pragma unroll
+                        for(int j = 0; j < 10; j++)
+                        {
+                            const int lrow = (q4 + 4 * j) * 8 + (lane >> 3);
+                            doff[j] -= (((lane & 7) ^ ((lrow >> 1) & 7)) & 4) ? 64u : 0u;
+                        }
+                    }
+                }
+                if(odd_k)
+                    step(k, H0{});
+                return;
+            }
             for(int k = 0; k < kt_count; k += 2)
             {
                 step(k, H0{});
@@ -741,9 +789,13 @@ int big_tile_rows() { return kBigXRows; }
 
 bool big_tile_supported(int prec, int k_bytes0, int k_bytes1, bool y_i8)
 {
-    // K in whole pairs of 64-byte steps; the int8 path's down GEMM with bf16 Y against int8 weights in fours
+    // K in whole pairs of 64-byte steps; the int8 path's down GEMM with bf16 Y against int8 weights in fours; the 8-bit
+    // gate+up GEMM also in odd numbers of steps, from five on (kOddK)
+    const bool k0_odd = k_bytes0 % (2 * kStepKB) == kStepKB && k_bytes0 >= 5 * kStepKB;
+    if(prec == MI355_MOE_FP8 && k0_odd)
+        return k_bytes1 % (2 * kStepKB) == 0;
     if(prec == MI355_MOE_INT8)
-        return k_bytes0 % (2 * kStepKB) == 0 && k_bytes1 % ((y_i8 ? 2 : 4) * kStepKB) == 0;
+        return (k_bytes0 % (2 * kStepKB) == 0 || k0_odd) && k_bytes1 % ((y_i8 ? 2 : 4) * kStepKB) == 0;
     return (prec == MI355_MOE_BF16 || prec == MI355_MOE_FP16 || prec == MI355_MOE_FP8) && k_bytes0 % (2 * kStepKB) == 0 &&
            k_bytes1 % (2 * kStepKB) == 0;
 }
