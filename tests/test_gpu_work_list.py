@@ -1,0 +1,39 @@
+"""The GEMMs' work list (an expert's rows without the padding behind its last token) and the one-workgroup sort that
+writes it, at the edges of row blocks, sort units, waves and the sort's capacity."""
+import numpy as np
+import pytest
+
+import oracle
+from therock_amd import inputs as mi
+from tests.test_gpu_fused_moe import TOL, oracle_out
+from tests.test_gpu_sorting import check as check_sorting
+
+pytestmark = pytest.mark.gpu
+
+COUNTS = [1, 31, 32, 33, 0, 63, 64, 65, 2]  # tokens of every expert
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp8", "int8"])
+@pytest.mark.parametrize("unit", [16, 48, 64, 128])
+def test_rows_per_expert_at_block_and_unit_edges(unit, dtype):
+    from tests.gpu_util import rel_l2, run_fused_moe
+    cfg = mi.MoeConfig("edges", sum(COUNTS), 256, 256, len(COUNTS), 1, dtype, "softmax_renorm", unit=unit)
+    inp = mi.make_inputs_np(cfg, 1)
+    ids = np.random.default_rng(2).permutation(np.repeat(np.arange(len(COUNTS)), COUNTS)).astype(np.int32)
+    inp["topk_ids"] = ids[:, None]
+    for kw in ({}, {"unfused": True}):
+        got, _ = run_fused_moe(cfg, inp, **kw)
+        ref, _ = oracle_out(cfg, inp, None, 1, 0)
+        assert np.all(np.isfinite(oracle.bf16_to_f32(got)))
+        assert rel_l2(oracle.bf16_to_f32(got), ref) <= TOL[dtype], (unit, dtype, kw)
+
+
+@pytest.mark.parametrize("tokens,experts,topk", [(1, 1, 1), (63, 2, 1), (64, 65, 1), (1023, 63, 1), (341, 256, 3), (1025, 255, 1),
+                                                 (4096, 256, 4), (16384, 3, 1), (16385, 3, 1), (4096, 257, 4)])
+def test_one_workgroup_sort_at_its_edges(tokens, experts, topk):
+    rng = np.random.default_rng(tokens + experts)
+    ids = np.argsort(rng.random((tokens, experts)), axis=1)[:, :topk].astype(np.int32)
+    check_sorting(ids, rng.random((tokens, topk), dtype=np.float32), experts, 32)
+    if experts > 1:
+        check_sorting(np.minimum(ids, 1) if topk == 1 else ids, rng.random((tokens, topk), dtype=np.float32), experts, 48,
+                      mask=(np.arange(experts) % 2 == 0).astype(np.int32))
