@@ -117,7 +117,8 @@ inline float run_timed(const stream_config& s, F&& launch)
 // One block per (device, stream): calls on different streams never share intermediates.  A block that was
 // handed out is never freed or moved - work already enqueued, or a captured graph, may still refer to it - so
 // growth allocates a new block and keeps the old one until the process ends.  Growth needs hipMalloc, which a
-// capturing stream does not allow: such callers pass their own workspace (or call once before capturing).
+// capturing stream does not allow: such callers pass their own workspace (or call once before capturing), and a
+// block that is too small for the captured call is an error of that call.
 // Calls that overlap on ONE stream's block from several host threads are the caller's to serialise.
 inline mi355_moe_workspace cached_workspace(size_t bytes, hipStream_t stream)
 {
@@ -135,7 +136,12 @@ inline mi355_moe_workspace cached_workspace(size_t bytes, hipStream_t stream)
     if(b.bytes < bytes)
     {
         hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-        if(hipStreamIsCapturing(stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone)
+        const bool capturing = hipStreamIsCapturing(stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+        // the reported size has room for options a call can do without (a down GEMM cut along K): the library says
+        // whether what is there is enough, before it launches anything
+        if(capturing && b.ptr != nullptr)
+            return mi355_moe_workspace{b.ptr, b.bytes};
+        if(capturing)
             throw std::runtime_error("mi355: the stream is capturing and the cached workspace would have to grow; "
                                      "pass a workspace of fused_moe_get_workspace_size() bytes instead");
         void* p = nullptr;

@@ -248,7 +248,9 @@ typedef struct mi355_fused_moe_args
 int mi355_fused_moe_supported(const mi355_fused_moe_traits* traits);
 
 /* bytes of the mi355_moe_workspace for mi355_fused_moe / mi355_fused_moegemm (includes the sort's own
- * workspace); 0 for unsupported traits or sizes out of range */
+ * workspace); 0 for unsupported traits or sizes out of range.  At some sizes this includes room for a down GEMM cut
+ * along K, which is faster: a workspace without that room (one sized for a larger batch that is not cut, say) is accepted
+ * and the GEMM runs uncut. */
 size_t mi355_fused_moe_workspace_size(const mi355_fused_moe_traits* traits, int32_t tokens,
                                       int32_t num_experts, int32_t topk, int32_t hidden_size,
                                       int32_t intermediate_size);
@@ -284,7 +286,7 @@ int mi355_fused_moe(const mi355_fused_moe_traits* traits, const mi355_fused_moe_
  * mi355_fused_moe_static_ws_capacity() bytes (96 MiB, enough for the decode regime: 256 tokens of a 128-expert
  * top-8 layer with hidden 4096 and intermediate 1536) that is part of the library's device image: every GPU the
  * library runs on holds it from the first use of the library until the process ends.  Nothing is allocated or
- * freed by the call.  A problem whose mi355_fused_moe_workspace_size() exceeds the capacity is rejected with
+ * freed by the call.  A problem whose intermediates exceed the capacity is rejected with
  * MI355_MOE_E_WORKSPACE.  All calls on one GPU share the buffer: calls that overlap on one GPU (two streams, two
  * threads) race; calls on one stream are ordered and safe.  The buffer's device address is looked up on the first
  * call on each device (not a stream operation; make that first call outside a capture). */
