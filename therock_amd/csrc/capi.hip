@@ -349,13 +349,12 @@ int run_fused_moe(const mi355_fused_moe_traits* traits, const mi355_fused_moe_ar
     g.topk                  = a->topk;
     g.stride_token          = a->stride_token;
     // every host-side check of both halves comes before the first launch: a rejected call has written nothing
-    rc = validate_fused_moegemm(*traits, g, ws_ptr, ws_bytes);
+    WorkspaceLayout wl{};
+    rc = validate_fused_moegemm(*traits, g, ws_ptr, ws_bytes, wl);
     if(rc != MI355_MOE_OK)
         return rc;
     if(a->num_tokens > 0 && (a->topk_ids_ptr == nullptr || a->topk_weight_ptr == nullptr))
         return fail(MI355_MOE_E_INVALID, "fused_moe: topk_ids or topk_weight is null");
-    const WorkspaceLayout wl = workspace_layout(*traits, a->num_tokens, a->num_experts, a->topk,
-                                                a->hidden_size, a->intermediate_size);
 
     // the combine writes every element of o, so the sort does not need to zero it
     mi355_moe_sorting_args s{};
@@ -376,12 +375,11 @@ int run_fused_moe(const mi355_fused_moe_traits* traits, const mi355_fused_moe_ar
     s.unit_size               = a->block_m;
     s.num_experts             = a->num_experts;
     s.topk                    = a->topk;
-    const GemmPlan plan = make_gemm_plan(*traits, ws_ptr, a->num_tokens, a->num_experts, a->topk, a->hidden_size,
-                                         a->intermediate_size);
+    const GemmPlan plan = make_gemm_plan(*traits, wl, ws_ptr, a->intermediate_size);
     rc = launch_moe_sorting(s, static_cast<hipStream_t>(stream), &plan);
     if(rc != MI355_MOE_OK)
         return rc;
-    return launch_fused_moegemm(*traits, g, ws_ptr, ws_bytes, static_cast<hipStream_t>(stream), /*prep_done=*/true);
+    return launch_fused_moegemm(*traits, g, ws_ptr, ws_bytes, static_cast<hipStream_t>(stream), &wl);
 }
 } // namespace
 

@@ -657,19 +657,20 @@ inline int64_t alt_most_active(int64_t tokens, int topk, int experts)
 
 // min_active: active experts from which the large tiles may be chosen.  A batch that cannot have as many (few tokens)
 // gets no second candidate, hence no empty launches (13 tokens of the 256-expert model: two of them, 16 us of 627).
-inline int alt_mblk(const mi355_fused_moe_traits& t, int64_t tokens, int topk, int experts, int hidden, int inter, int min_active)
+// mblk: what pick_mblk chose.
+inline int alt_mblk(const mi355_fused_moe_traits& t, int mblk, int64_t tokens, int topk, int experts, int hidden, int inter, int min_active)
 {
-    if(t.prec_i != MI355_MOE_FP8 || t.fused_quant != 0 || alt_most_active(tokens, topk, experts) < min_active ||
+    if(mblk > 4 || t.prec_i != MI355_MOE_FP8 || t.fused_quant != 0 || alt_most_active(tokens, topk, experts) < min_active ||
        !big_tile_ok(t, tokens, topk, experts, hidden, inter))
         return 0;
-    return pick_mblk(t, tokens, topk, experts, hidden, inter) <= 4 ? big_tile_rows() / 32 : 0;
+    return mblk <= 4 ? big_tile_rows() / 32 : 0;
 }
 
 // enough active experts for tiles of 256 of their weight_rows weight rows to fill the chip
 inline int alt_min_active(int weight_rows) { return ceil_div(device_info().num_cu, ceil_div(weight_rows, 256)); }
-inline int alt_mblk_fused(const mi355_fused_moe_traits& t, int64_t tokens, int topk, int experts, int hidden, int inter)
+inline int alt_mblk_fused(const mi355_fused_moe_traits& t, int mblk, int64_t tokens, int topk, int experts, int hidden, int inter)
 {
-    return alt_mblk(t, tokens, topk, experts, hidden, inter, alt_min_active((t.gate_only ? 1 : 2) * inter));
+    return alt_mblk(t, mblk, tokens, topk, experts, hidden, inter, alt_min_active((t.gate_only ? 1 : 2) * inter));
 }
 
 // The most tiles of `rows` rows that `active` experts can need for n entries between them (an expert's c rows split into
@@ -769,15 +770,14 @@ inline bool down_gemm_decode(int prec, int mblk, bool decode, bool y_i8, int exp
 //  * Large-tile kernel (one workgroup per compute unit): what a launch takes is its rounds of workgroups, each about
 //    3 us + operand bytes / 40 B/ns, and the combine's traffic at 4 TB/s, which grows with the slices (636 tokens x 3 of 7
 //    fp8 experts 5632 x 3200: 172 us, cut in two 224).  Cut where this says a tenth of it is gained.
-inline int down_gemm_slice_bytes(const mi355_fused_moe_traits& t, int64_t tokens, int topk, int experts, int hidden, int inter)
+// mblk, alt: what pick_mblk and alt_mblk chose (two candidate tile heights write one buffer: not cut).
+inline int down_gemm_slice_bytes(const mi355_fused_moe_traits& t, int mblk, int alt, int64_t tokens, int topk, int experts, int hidden, int inter)
 {
-    const int mblk    = pick_mblk(t, tokens, topk, experts, hidden, inter);
     const int64_t n   = tokens * topk;
     const bool quant  = t.prec_i != MI355_MOE_BF16 && t.prec_i != MI355_MOE_FP16;
     const bool decode = down_gemm_decode(t.prec_i, mblk, decode_tile(t, mblk), t.prec_i == MI355_MOE_INT8 && t.fused_quant != 0,
                                          experts, n, hidden);
-    // (two candidate tile heights write one buffer: not cut)
-    if(n == 0 || (!decode && mblk <= 4) || alt_mblk_fused(t, tokens, topk, experts, hidden, inter) != 0)
+    if(n == 0 || (!decode && mblk <= 4) || alt != 0)
         return 0;
     const int num_cu      = device_info().num_cu;
     const int64_t active  = std::min<int64_t>(experts, n);
@@ -852,7 +852,7 @@ int gemm_tile_rows(const mi355_fused_moe_traits& t, int32_t tokens, int32_t expe
 int gemm_alt_tile_rows(const mi355_fused_moe_traits& t, int32_t tokens, int32_t experts, int32_t topk, int32_t hidden,
                        int32_t inter)
 {
-    return alt_mblk_fused(t, tokens, topk, experts, hidden, inter) * 32;
+    return alt_mblk_fused(t, pick_mblk(t, tokens, topk, experts, hidden, inter), tokens, topk, experts, hidden, inter) * 32;
 }
 
 WorkspaceLayout workspace_layout(const mi355_fused_moe_traits& t, int32_t tokens, int32_t experts, int32_t topk,
@@ -879,7 +879,9 @@ WorkspaceLayout workspace_layout(const mi355_fused_moe_traits& t, int32_t tokens
     w.ys_off         = bump(t.prec_i == MI355_MOE_FP8 ? (size_t)w.ys_kb_stride * (inter / 32) : 0);
     w.yq_off         = bump(requant ? (size_t)round_up<int64_t>(w.max_pad, 16) * inter : 0);
     w.yrs_off        = bump(requant ? (size_t)w.max_pad * sizeof(float) : 0);
-    w.k_slice        = down_gemm_slice_bytes(t, tokens, topk, experts, hidden, inter);
+    w.mblk           = mblk;
+    w.alt            = alt_mblk_fused(t, mblk, tokens, topk, experts, hidden, inter);
+    w.k_slice        = down_gemm_slice_bytes(t, mblk, w.alt, tokens, topk, experts, hidden, inter);
     const int w_b    = t.prec_i == MI355_MOE_BF16 || t.prec_i == MI355_MOE_FP16 ? 2 : 1;
     w.p_off          = bump((size_t)w.max_pad * hidden * 2);
     w.least          = w.total;
@@ -887,18 +889,16 @@ WorkspaceLayout workspace_layout(const mi355_fused_moe_traits& t, int32_t tokens
     return w;
 }
 
-GemmPlan make_gemm_plan(const mi355_fused_moe_traits& t, void* ws_ptr, int32_t tokens, int32_t experts, int32_t topk,
-                        int32_t hidden, int32_t inter)
+GemmPlan make_gemm_plan(const mi355_fused_moe_traits& t, const WorkspaceLayout& ws, void* ws_ptr, int32_t inter)
 {
-    const WorkspaceLayout ws = workspace_layout(t, tokens, experts, topk, hidden, inter);
     unsigned char* wsb       = static_cast<unsigned char*>(ws_ptr);
     GemmPlan g{};
     g.tile_map      = reinterpret_cast<int*>(wsb + ws.map_off);
-    g.rows_per_tile = pick_mblk(t, tokens, topk, experts, hidden, inter) * 32;
+    g.rows_per_tile = ws.mblk * 32;
     g.max_tiles     = ws.max_tiles;
     g.inv           = reinterpret_cast<int*>(wsb + ws.inv_off);
     // the second candidate needs enough active experts for its gate+up tiles (256 weight rows each) to fill the chip
-    g.alt_rows_per_tile = alt_mblk_fused(t, tokens, topk, experts, hidden, inter) * 32;
+    g.alt_rows_per_tile = ws.alt * 32;
     g.alt_min_rows      = kAltMinRows;
     g.alt_min_active    = alt_min_active((t.gate_only ? 1 : 2) * inter);
     return g;
@@ -914,7 +914,7 @@ bool sizes_in_range(int32_t tokens, int32_t experts, int32_t topk, int32_t hidde
 // Everything that can be checked on the host before anything is launched: the fused entry point calls it ahead
 // of the sort, so that a rejected call leaves the caller's sort outputs and workspace untouched.
 int validate_fused_moegemm(const mi355_fused_moe_traits& t, const mi355_fused_moegemm_args& a, const void* ws_ptr,
-                           size_t ws_bytes)
+                           size_t ws_bytes, WorkspaceLayout& ws)
 {
     int rc = check_traits(t);
     if(rc != MI355_MOE_OK)
@@ -923,7 +923,7 @@ int validate_fused_moegemm(const mi355_fused_moe_traits& t, const mi355_fused_mo
     if(!sizes_in_range(T, E, K, H, I) || a.stride_token < H)
         return fail(MI355_MOE_E_INVALID, "fused_moegemm: bad sizes (H=%d I=%d T=%d E=%d K=%d stride=%d)", H, I, T, E,
                     K, a.stride_token);
-    const WorkspaceLayout ws = workspace_layout(t, T, E, K, H, I);
+    ws = workspace_layout(t, T, E, K, H, I);
     if(ws_ptr == nullptr || ws_bytes < ws.least)
         return fail(MI355_MOE_E_WORKSPACE, "fused_moegemm: workspace of %zu bytes needed, %zu given", ws.least,
                     ws_ptr ? ws_bytes : (size_t)0);
@@ -956,18 +956,23 @@ int validate_fused_moegemm(const mi355_fused_moe_traits& t, const mi355_fused_mo
                                  (int64_t)2 * I * H * eb >= ((int64_t)1 << 32)))
         return fail(MI355_MOE_E_UNSUPPORTED, "fused_moegemm: pre-shuffled weights need rows of whole 64-byte blocks and "
                                              "experts below 4 GiB (H=%d I=%d)", H, I);
-    const int mblk = pick_mblk(t, T, K, E, H, I);
     // (smooth-quant activations hold a row per (slot, token))
-    if(mblk > 4 && (int64_t)T * (t.fused_quant == 1 ? K : 1) * a.stride_token * eb >= ((int64_t)1 << 32))
+    if(ws.mblk > 4 && (int64_t)T * (t.fused_quant == 1 ? K : 1) * a.stride_token * eb >= ((int64_t)1 << 32))
         return fail(MI355_MOE_E_UNSUPPORTED, "fused_moegemm: a token buffer of 4 GiB or more (stride_token=%d) is not "
                                              "supported at this problem size", a.stride_token);
     return MI355_MOE_OK;
 }
 
 int launch_fused_moegemm(const mi355_fused_moe_traits& t, const mi355_fused_moegemm_args& a, void* ws_ptr,
-                         size_t ws_bytes, hipStream_t stream, bool prep_done)
+                         size_t ws_bytes, hipStream_t stream, const WorkspaceLayout* prepared)
 {
-    int rc = validate_fused_moegemm(t, a, ws_ptr, ws_bytes);
+    int rc               = MI355_MOE_OK;
+    const bool prep_done = prepared != nullptr;
+    WorkspaceLayout ws{};
+    if(prep_done)
+        ws = *prepared;
+    else
+        rc = validate_fused_moegemm(t, a, ws_ptr, ws_bytes, ws);
     if(rc != MI355_MOE_OK)
         return rc;
     if(a.num_tokens == 0)
@@ -975,14 +980,13 @@ int launch_fused_moegemm(const mi355_fused_moe_traits& t, const mi355_fused_moeg
     const bool quant = t.prec_i != MI355_MOE_BF16 && t.prec_i != MI355_MOE_FP16;
     const int H = a.hidden_size, I = a.intermediate_size, T = a.num_tokens, E = a.num_experts, K = a.topk;
     const int eb = quant ? 1 : 2;
-    const WorkspaceLayout ws = workspace_layout(t, T, E, K, H, I);
     unsigned char* wsb = static_cast<unsigned char*>(ws_ptr);
     int* tile_map      = reinterpret_cast<int*>(wsb + ws.map_off);
     int* inv           = reinterpret_cast<int*>(wsb + ws.inv_off);
-    const int mblk     = pick_mblk(t, T, K, E, H, I);
+    const int mblk     = ws.mblk;
     const int max_units = (int)ceil_div<int64_t>(ws.max_pad, t.block_m);
     // the sort chose between two tile heights (see alt_mblk): both kernel families are launched for each GEMM
-    const int alt     = alt_mblk_fused(t, T, K, E, H, I);
+    const int alt     = ws.alt;
     int max_tiles     = ws.max_tiles;
     int alt_max_tiles = alt ? (int)std::min<int64_t>(ws.max_tiles, E + ws.max_pad / (alt * 32) + 1) : 0;
     if(prep_done)
@@ -1204,7 +1208,7 @@ int flatmm_layout(int kind, const mi355_moe_flatmm_args& a, FlatmmLayout& L)
         L.mblk = std::min(L.mblk, 4);
     }
     // skewed decode-sized batches: the same choice between two tile heights as the fused entry points make
-    L.alt          = a.k_padded_zeros == 0 ? alt_mblk(L.traits, a.NumTokens, a.TopK, a.NumExperts, L.hidden, L.inter, alt_min_active(a.N)) : 0;
+    L.alt          = a.k_padded_zeros == 0 ? alt_mblk(L.traits, L.mblk, a.NumTokens, a.TopK, a.NumExperts, L.hidden, L.inter, alt_min_active(a.N)) : 0;
     L.max_pad      = (int64_t)a.TopK * a.NumTokens + (int64_t)a.NumExperts * a.block_m - a.TopK;
     L.max_tiles    = (int32_t)(a.NumExperts + L.max_pad / (L.mblk * 32) + 1);
     L.total        = 0;
@@ -1216,7 +1220,7 @@ int flatmm_layout(int kind, const mi355_moe_flatmm_args& a, FlatmmLayout& L)
     L.map_off = bump(sizeof(int) * (kMapHdr + (size_t)kMapEnt * L.max_tiles));
     L.inv_off = bump(sizeof(int) * (size_t)a.NumTokens * a.TopK);
     const int b_bytes = w8 || f8 ? 1 : 2;
-    L.k_slice = g1 || L.alt != 0 || a.k_padded_zeros > 0 ? 0 : down_gemm_slice_bytes(L.traits, a.NumTokens, a.TopK, a.NumExperts, L.hidden, L.inter);
+    L.k_slice = g1 || L.alt != 0 || a.k_padded_zeros > 0 ? 0 : down_gemm_slice_bytes(L.traits, L.mblk, L.alt, a.NumTokens, a.TopK, a.NumExperts, L.hidden, L.inter);
     L.p_off   = bump(g1 ? 0 : (size_t)L.max_pad * L.hidden * 2);
     // the fp8 down GEMM runs the block-scaled MFMA: its input carries one scale per row, so every block scale is 2^0
     L.ys_kb_stride = round_up<int64_t>(L.max_pad, 256) + 512;

@@ -22,6 +22,7 @@ struct WorkspaceLayout
     size_t least;      // without the room for a down GEMM cut along K: a call with less than total bytes is not cut
     int64_t max_pad;
     int32_t max_tiles; // upper bound of M tiles
+    int mblk, alt;     // tile height and the second one the sort may choose (0: none), in 32-row blocks
 };
 
 int check_traits(const mi355_fused_moe_traits& t);
@@ -39,17 +40,16 @@ int gemm_tile_rows(const mi355_fused_moe_traits& t, int32_t tokens, int32_t expe
 // true when the sizes are ones the path can index (24-bit token ids, 8-bit slots, at most 1024 experts)
 bool sizes_in_range(int32_t tokens, int32_t experts, int32_t topk, int32_t hidden, int32_t inter);
 
-// host-side checks of launch_fused_moegemm, launching nothing
+// host-side checks of launch_fused_moegemm, launching nothing; ws: the problem's layout
 int validate_fused_moegemm(const mi355_fused_moe_traits& t, const mi355_fused_moegemm_args& a, const void* ws_ptr,
-                           size_t ws_bytes);
+                           size_t ws_bytes, WorkspaceLayout& ws);
 
-// prep_done: the tile list and the inverse map were already written by the sort (GemmPlan)
+// prepared: the layout of a call that was validated and whose tile list and inverse map the sort has written (GemmPlan)
 int launch_fused_moegemm(const mi355_fused_moe_traits& t, const mi355_fused_moegemm_args& a, void* ws_ptr,
-                         size_t ws_bytes, hipStream_t stream, bool prep_done = false);
+                         size_t ws_bytes, hipStream_t stream, const WorkspaceLayout* prepared = nullptr);
 
-// the plan the sort has to fill for launch_fused_moegemm(..., prep_done = true)
-GemmPlan make_gemm_plan(const mi355_fused_moe_traits& t, void* ws_ptr, int32_t tokens, int32_t experts,
-                        int32_t topk, int32_t hidden, int32_t inter);
+// the plan the sort has to fill for launch_fused_moegemm(..., &ws)
+GemmPlan make_gemm_plan(const mi355_fused_moe_traits& t, const WorkspaceLayout& ws, void* ws_ptr, int32_t inter);
 
 namespace gemm {
 struct GemmParams;
