@@ -287,6 +287,39 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
     }
     const bool odd_k        = kOddK && (kt_count & 1) != 0;
     const int n_wunits      = kW8 ? kt_count / 2 : kt_count + (odd_k ? 1 : 0); // two units (row halves) per 128 bytes of weight K
+    // Where the walk over K begins.  The 256 weight rows of a tile lie a row pitch apart, so that with a pitch of whole
+    // 4 KiB (hidden 4096 or 2048 in 16 bits, 4096 or 8192 in 8) every row of a K window sits behind the same L2 channel,
+    // and the workgroups of an XCD, started together, walk the channels in step.  Column tile i begins a
+    // share of K further on instead, the fractional part of i * golden ratio, and wraps around: any run of consecutive
+    // tiles, the 32 an XCD runs together, spreads evenly over the row and its channels.  (Steps of 3, 5, 9, 11 and 13
+    // windows of 128 bytes measured the same; 4 windows reach 16 of the start points of an 8 KiB row and are as slow as
+    // none.  Tiles are numbered over the experts, as a narrow layer has few columns.)  Gate+up
+    // GEMM at 83 rows per expert: bf16 8 x 4096 x 16384 462 -> 350 us (4.7 -> 6.1 TB/s), fp8 / int8 16 x 4096 x 8192
+    // 255 -> 190 / 262 -> 200 us; at other pitches up to 4 % (int8, 64 x 7168 x 2048 at 84 rows: pass 713 -> 684 us).
+    // Not rotated: row tiles that share weights, which fetch each weight slice together and each token slice for eight
+    // column tiles at a time (4096 tokens x 2 of 8 bf16 experts 1598 -> 1720 us); down GEMMs without the bad pitch, whose
+    // shorter K gains up to 2 % at 145 rows and loses as much elsewhere (263 rows of 15 fp16 experts 3840 x 11008 3 %, 1000
+    // tokens x 8 of 256 fp8 experts 7168 x 2048 0.8 %).
+    constexpr uint32_t kGolden = 0x9e3779b9u; // its fractional part in units of 2^-32
+    const int n_win   = n_wunits >> 1; // 128-byte windows of weight K
+    const bool rotate = !odd_k && tile.expert_tiles == 1 && (GEMM0 || (p.w_row_bytes & 4095) == 0);
+    const uint32_t at = (uint32_t)expert * (uint32_t)p.n_ntiles + (uint32_t)tile.nt;
+    const int rot     = rotate ? (int)__umulhi(at * kGolden, (uint32_t)n_win) : 0; // < n_win
+    // the wave's stream (weights or tokens): address of the window it is in, moved on by its issue functions
+    const int w_kadv            = weight_k_advance(p, 2 * kStepKB); // bytes between the 128-byte K windows of two weight units
+    const int64_t window_bytes  = w_role ? w_kadv : (int64_t)x_step * (kW8 ? 4 : 2);
+    const int64_t stream_bytes  = window_bytes * n_win;
+    const unsigned char* stream = dbase + window_bytes * rot;
+    int windows_left            = n_win - rot; // to the end of K
+    ys_base += rot * 2 * ys_step; // (moves along with the tokens)
+    auto end_window = [&]() __attribute__((always_inline)) {
+        if(--windows_left == 0)
+        {
+            stream -= stream_bytes;
+            if constexpr(kMx)
+                ys_base -= n_win * 2 * ys_step;
+        }
+    };
 
     // weight role: unit u (half u & 1) -> ring slot u % 6
     // Weights no other row tile re-reads (the expert has a single one) are fetched non-temporal: measured
@@ -294,14 +327,13 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
     // re-reads should hit L2, and non-temporal fetches cost 3 % there.  NT is a template argument like the
     // slab-group count, for the same reason.
     const bool w_nt = tile.expert_tiles == 1;
-    const int w_kadv = weight_k_advance(p, 2 * kStepKB); // bytes between the 128-byte K windows of two weight units
     auto issue_w = [&](int u, auto half_tag, auto nt_tag) __attribute__((always_inline)) {
         constexpr int H = decltype(half_tag)::value;
         constexpr bool NT = decltype(nt_tag)::value;
         if(u >= n_wunits)
             return;
         const uint32_t sbase     = lds_base + (u % kWS) * kWUnitBytes + q4 * 1024;
-        const unsigned char* src = dbase + (u >> 1) * w_kadv;
+        const unsigned char* src = stream;
 #pragma unroll
         for(int j = 0; j < 4; j++)
         {
@@ -315,21 +347,32 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
             else
                 dma16(src, off, __builtin_amdgcn_readfirstlane(sbase + j * 4096));
         }
+        if(H < 0 ? (u & 1) : H)
+        {
+            stream += w_kadv;
+            end_window();
+        }
     };
     // token role: step x -> ring stage x % 3
     auto issue_x = [&](int x, int groups) __attribute__((always_inline)) {
         if(x >= kt_count)
             return;
         const uint32_t sbase     = lds_base + kXOffset + (x % kXStages) * kXStageBytes + q4 * 1024;
-        const unsigned char* src = dbase + x * x_step;
+        const unsigned char* src = stream;
 #pragma unroll
         for(int j = 0; j < 5; j++)
             if(j < groups)
                 dma16(src, doff[j], __builtin_amdgcn_readfirstlane(sbase + j * 4096));
         if constexpr(kMx)
-            dma4(ys_base + x * ys_step, doff[5],
+        {
+            dma4(ys_base, doff[5],
                  __builtin_amdgcn_readfirstlane(lds_base + kYsOffset + (x % kXStages) * kYsStageBytes +
                                                 (q4 >> 1) * kYsRows + (q4 & 1) * 256));
+            ys_base += ys_step;
+        }
+        stream += x_step;
+        if((x & (kW8 ? 3 : 1)) == (kW8 ? 3 : 1))
+            end_window();
     };
 
     // 128-byte token stages: pair m = steps 2 m and 2 m + 1 -> stage m & 1; two instructions per 64 rows of the tile
@@ -339,11 +382,13 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
             if(2 * m >= kt_count)
                 return;
             const uint32_t sbase     = lds_base + kXO + (m & 1) * kXPairBytes + q4 * 1024;
-            const unsigned char* src = dbase + m * (2 * kStepKB);
+            const unsigned char* src = stream;
 #pragma unroll
             for(int j = 0; j < 10; j++)
                 if(j < 2 * groups)
                     dma16(src, doff[j], __builtin_amdgcn_readfirstlane(sbase + j * 4096));
+            stream += 2 * kStepKB;
+            end_window();
         }
     };
 
