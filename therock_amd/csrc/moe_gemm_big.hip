@@ -149,12 +149,15 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
     // k, each fragment right behind the last MFMA that reads its register, so that after a barrier the MFMAs start
     // at once instead of waiting for operand fetches that all eight waves issue at the same moment.  The barrier of
     // step k then has to guarantee the data of step k+1: every transfer runs one step further ahead.
-    constexpr bool kPipe  = !kW8 && !kMx;
+    constexpr bool kPipe  = !kMx;
     constexpr bool kXPair = kPipe && GEMM0; // 128-byte token stages
     // 8-bit rows of an odd number of 64-byte steps (hidden sizes that are odd multiples of 64): the last 128-byte window
     // has only its first half.  Lanes that would fetch the second half (the next row's bytes, past the tensor's end in its
     // last row) fetch the first one again, and the last step has no partner, so nothing reads what they fetched.
     constexpr bool kOddK = kXPair && (MODE == kI8 || MODE == kFp8);
+    // Down GEMM weights of one byte a value, rows of an odd number of 64-byte pieces: the last 128-byte window begins 64 bytes
+    // earlier, inside the row, and the steps it serves read its second half.
+    constexpr bool kOddW = !GEMM0 && (MODE == kI8 || kW8);
     constexpr int kWS     = kXPair ? kWSlotsPair : kWSlots;
     constexpr int kXO     = kXPair ? kXOffsetPair : kXOffset;
 
@@ -285,8 +288,8 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
         if constexpr(kMx)
             ys_base += step0 * ys_step;
     }
-    const bool odd_k        = kOddK && (kt_count & 1) != 0;
-    const int n_wunits      = kW8 ? kt_count / 2 : kt_count + (odd_k ? 1 : 0); // two units (row halves) per 128 bytes of weight K
+    const bool odd_k        = (kOddK || kOddW) && (kt_count & (kW8 ? 2 : 1)) != 0; // (kW8: 64 bytes of weights are two steps)
+    const int n_wunits      = kW8 ? (kt_count + (odd_k ? 2 : 0)) / 2 : kt_count + (odd_k ? 1 : 0); // two units (row halves) per 128 bytes of weight K
     // Where the walk over K begins.  The 256 weight rows of a tile lie a row pitch apart, so that with a pitch of whole
     // 4 KiB (hidden 4096 or 2048 in 16 bits, 4096 or 8192 in 8) every row of a K window sits behind the same L2 channel,
     // and the workgroups of an XCD, started together, walk the channels in step.  Column tile i begins a
@@ -308,14 +311,18 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
     // the wave's stream (weights or tokens): address of the window it is in, moved on by its issue functions
     const int w_kadv            = weight_k_advance(p, 2 * kStepKB); // bytes between the 128-byte K windows of two weight units
     const int64_t window_bytes  = w_role ? w_kadv : (int64_t)x_step * (kW8 ? 4 : 2);
-    const int64_t stream_bytes  = window_bytes * n_win;
     const unsigned char* stream = dbase + window_bytes * rot;
-    int windows_left            = n_win - rot; // to the end of K
     ys_base += rot * 2 * ys_step; // (moves along with the tokens)
+    // windows until the stream goes back, and by how much: to the start of K, or (kOddW) the half window
+    const bool half_window = kOddW && odd_k && w_role;
+    int windows_left       = half_window ? n_win - 1 : n_win - rot;
+    const int64_t back     = half_window ? w_kadv / 2 : window_bytes * n_win;
+    if(half_window && windows_left == 0) // (a slice of 64 bytes: the window begins in the slice before)
+        stream -= back;
     auto end_window = [&]() __attribute__((always_inline)) {
         if(--windows_left == 0)
         {
-            stream -= stream_bytes;
+            stream -= back;
             if constexpr(kMx)
                 ys_base -= n_win * 2 * ys_step;
         }
@@ -405,29 +412,23 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
             for(int v = 0; v < 16; v++)
                 acc[i][b][v] = 0;
 
-    // prologue: weight units 0..3 (0..4 when pipelined with six slots), token steps 0 and 1 (and 2; or pairs 0 and 1)
+    // prologue: weight units 0..3 (0..4 when pipelined with six slots, unless a unit lasts four steps), token steps 0 and 1
+    // (and 2; or pairs 0 and 1)
     using H0 = std::integral_constant<int, 0>;
     using H1 = std::integral_constant<int, 1>;
     if(w_role)
     {
+        auto units = [&](auto nt_tag) __attribute__((always_inline)) {
+            static_for<(kPipe && !kXPair && !kW8) ? 5 : 4>([&](auto u_tag) __attribute__((always_inline)) {
+                constexpr int u = decltype(u_tag)::value;
+                using Half      = std::integral_constant<int, (u & 1)>;
+                issue_w(u, Half{}, nt_tag);
+            });
+        };
         if(w_nt)
-        {
-            issue_w(0, H0{}, std::true_type{});
-            issue_w(1, H1{}, std::true_type{});
-            issue_w(2, H0{}, std::true_type{});
-            issue_w(3, H1{}, std::true_type{});
-            if constexpr(kPipe && !kXPair)
-                issue_w(4, H0{}, std::true_type{});
-        }
+            units(std::true_type{});
         else
-        {
-            issue_w(0, H0{}, std::false_type{});
-            issue_w(1, H1{}, std::false_type{});
-            issue_w(2, H0{}, std::false_type{});
-            issue_w(3, H1{}, std::false_type{});
-            if constexpr(kPipe && !kXPair)
-                issue_w(4, H0{}, std::false_type{});
-        }
+            units(std::false_type{});
     }
     else if constexpr(kXPair)
     {
@@ -463,14 +464,31 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
             Frag wf[kSteps][2];
             Frag xf[kSteps][NF];
             uint32_t xs[kSteps][NF];
+            // first step of the last window where only its second half is new (kOddW)
+            [[maybe_unused]] const int half_from = kOddW && odd_k ? kt_count - (kW8 ? 2 : 1) : INT32_MAX;
             // weight fragment b of sub-step s of step kk (parity P), token fragment i of sub-step s of step kk
             auto load_wf = [&](int kk, auto p_tag, int s, int b) __attribute__((always_inline)) {
                 constexpr int P          = decltype(p_tag)::value;
                 constexpr int kh         = P * 4; // first chunk of the step inside the 128-byte weight row
-                const unsigned char* wp  = lds + (((kk & ~1) + w_h) % kWS) * kWUnitBytes + w_off + b * 32 * (2 * kStepKB);
+                const unsigned char* wp  = lds + ((big_pair_of_step(kk, kW8) + w_h) % kWS) * kWUnitBytes + w_off + b * 32 * (2 * kStepKB);
                 const int cw_lo          = kOpB == 16 ? ((kh + 2 * s + kg) ^ sw_wr) * kWChunkB : ((kh + kg) ^ sw_wr) * kWChunkB;
                 const int cw_hi          = ((kh + 2 + kg) ^ sw_wr) * kWChunkB;
                 Frag f;
+                if constexpr(kW8)
+                {
+                    // 8 int8 of this lane's K group, not converted yet: 16-byte chunk (kk & 3) * 2 + s of the row, half kg
+                    const int q   = (kk >= half_from ? kk + 2 : kk) & 3;
+                    const int c8  = (((q << 1) + s) ^ sw_wr) * kWChunkB + kg * 8;
+                    const uint2 v = *reinterpret_cast<const uint2*>(wp + c8);
+                    f.lo.x        = v.x;
+                    f.lo.y        = v.y;
+                    return f;
+                }
+                if constexpr(kOddW)
+                {
+                    f.lo = *reinterpret_cast<const uint4*>(wp + (cw_lo ^ (kk >= half_from ? 4 * kWChunkB : 0)));
+                    return f;
+                }
                 f.lo = *reinterpret_cast<const uint4*>(wp + cw_lo);
                 if constexpr(kOpB == 32)
                     f.hi = *reinterpret_cast<const uint4*>(wp + cw_hi);
@@ -504,8 +522,8 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
             };
             // own transfers of the data named `need` have landed (the instructions issued after them may be
             // pending), everyone's are visible after the barrier, and nobody reads the buffers of the step before
-            auto sync = [&](bool counted, auto w_tag, auto x_tag) __attribute__((always_inline)) {
-                if(counted)
+            auto sync = [&](bool w_counted, bool x_counted, auto w_tag, auto x_tag) __attribute__((always_inline)) {
+                if(w_role ? w_counted : x_counted)
                 {
                     if(w_role)
                         wait_vmcnt<decltype(w_tag)::value>();
@@ -521,14 +539,21 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
             constexpr int kXI = XG + (kMx ? 1 : 0); // token-role instructions of one step
             // step 0's data: weight units 0 and 1 (2, 3, 4 may be pending), token step 0 (1 and 2 pending); with
             // 128-byte token stages weight units 2 and 3 and token pair 1 may be pending
+            // (a unit of int8 weights lasts four steps: units 2 and 3)
+            const bool six = kt_count >= 6;
             if constexpr(kXPair)
-                sync(kt_count >= 6, std::integral_constant<int, 8>{}, std::integral_constant<int, 2 * XG>{});
+                sync(six, six, std::integral_constant<int, 8>{}, std::integral_constant<int, 2 * XG>{});
             else
-                sync(kt_count >= 6, std::integral_constant<int, 12>{}, std::integral_constant<int, 2 * kXI>{});
+                sync(kW8 ? n_wunits >= 4 : six, six, std::integral_constant<int, (kW8 ? 8 : 12)>{}, std::integral_constant<int, 2 * kXI>{});
             static_for<kSteps>([&](auto s_tag) __attribute__((always_inline)) {
                 constexpr int s = decltype(s_tag)::value;
                 wf[s][0]        = load_wf(0, H0{}, s, 0);
                 wf[s][1]        = load_wf(0, H0{}, s, 1);
+                if constexpr(kW8)
+                {
+                    wf[s][0].lo = int8x8_to_bf16x8(make_uint2(wf[s][0].lo.x, wf[s][0].lo.y));
+                    wf[s][1].lo = int8x8_to_bf16x8(make_uint2(wf[s][1].lo.x, wf[s][1].lo.y));
+                }
                 static_for<NB>([&](auto i_tag) __attribute__((always_inline)) {
                     constexpr int i = decltype(i_tag)::value;
                     xf[s][i]        = load_xf(0, s, i, xs[s][i]);
@@ -546,14 +571,19 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                 // k - 1) was last read before the barrier of step k - 1: the even step has no barrier.
                 // Measured: without it the bf16 and int8 GEMMs (two MFMA sub-steps per step) run 2 % faster, the fp8
                 // GEMM (one) 5 % slower, so that one keeps it.
+                // Units of int8 weights, one every other step and read for four: the pair of step k + 1 has landed once at most
+                // two units are in flight, while there are later ones (big_units_may_fly).
+                const bool counted = k + 4 < kt_count;
                 if constexpr(kXPair)
                 {
                     if constexpr(PAR == 1 || kSteps == 1)
-                        sync(k + 4 < kt_count, std::integral_constant<int, (PAR ? 4 : 8)>{},
+                        sync(counted, counted, std::integral_constant<int, (PAR ? 4 : 8)>{},
                              std::integral_constant<int, (PAR ? 0 : 2 * XG)>{});
                 }
+                else if constexpr(kW8)
+                    sync(big_units_may_fly(k + 1, kt_count, kW8), counted, std::integral_constant<int, 8>{}, std::integral_constant<int, kXI>{});
                 else
-                    sync(k + 4 < kt_count, std::integral_constant<int, (PAR ? 8 : 12)>{}, std::integral_constant<int, kXI>{});
+                    sync(counted, counted, std::integral_constant<int, (PAR ? 8 : 12)>{}, std::integral_constant<int, kXI>{});
                 // the transfers of the step go out behind the MFMAs of the second token block (measured: 1 to 2 %
                 // faster than right after the barrier, where all eight waves queue up at the address unit while the
                 // MFMA pipe has nothing to do; one instruction behind every block is 5 % slower)
@@ -568,7 +598,12 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                             issue_x_pair((k + 3) >> 1, XG);
                     }
                     else if(w_role)
-                        issue_w(k + 5, NPAR{}, nt_tag);
+                    {
+                        if constexpr(!kW8)
+                            issue_w(k + 5, NPAR{}, nt_tag);
+                        else if constexpr(PAR == 0)
+                            issue_w(big_unit_of_step(k, kW8), std::integral_constant<int, -1>{}, nt_tag);
+                    }
                     else
                         issue_x(k + 3, XG);
                 };
@@ -577,6 +612,14 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                     issue_next();
                 static_for<kSteps>([&](auto s_tag) __attribute__((always_inline)) {
                     constexpr int s = decltype(s_tag)::value;
+                    // int8 weights of the next step travel under this one's MFMAs and are converted behind them
+                    [[maybe_unused]] Frag raw[2];
+                    if constexpr(kW8)
+                    {
+                        raw[0] = load_wf(k + 1, NPAR{}, s, 0);
+                        raw[1] = load_wf(k + 1, NPAR{}, s, 1);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
                     static_for<NB>([&](auto i_tag) __attribute__((always_inline)) {
                         constexpr int i = decltype(i_tag)::value;
                         if constexpr(MODE == kFp8 && GEMM0)
@@ -596,8 +639,16 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                             issue_next();
                         __builtin_amdgcn_sched_barrier(0);
                     });
-                    wf[s][0] = load_wf(k + 1, NPAR{}, s, 0);
-                    wf[s][1] = load_wf(k + 1, NPAR{}, s, 1);
+                    if constexpr(kW8)
+                    {
+                        wf[s][0].lo = int8x8_to_bf16x8(make_uint2(raw[0].lo.x, raw[0].lo.y));
+                        wf[s][1].lo = int8x8_to_bf16x8(make_uint2(raw[1].lo.x, raw[1].lo.y));
+                    }
+                    else
+                    {
+                        wf[s][0] = load_wf(k + 1, NPAR{}, s, 0);
+                        wf[s][1] = load_wf(k + 1, NPAR{}, s, 1);
+                    }
                     __builtin_amdgcn_sched_barrier(0);
                 });
             };
@@ -644,6 +695,17 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                     step(k, H0{});
                 return;
             }
+            if constexpr(kOddW && !kW8)
+            {
+                for(int k = 0; k + 1 < kt_count; k += 2)
+                {
+                    step(k, H0{});
+                    step(k + 1, H1{});
+                }
+                if(odd_k)
+                    step(kt_count - 1, H0{});
+                return;
+            }
             for(int k = 0; k < kt_count; k += 2)
             {
                 step(k, H0{});
@@ -654,15 +716,14 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
         // one compute step; PAR = k & 1
         auto step = [&](int k, auto par_tag) __attribute__((always_inline)) {
             constexpr int PAR = decltype(par_tag)::value;
-            // Needed now: token step k and the weight units of pair k >> 1 (k >> 2 with int8 weights).  Issued after them
-            // and allowed to stay pending: token step k+1; two weight units (even k) or three (odd k), until the last
-            // pair is the one needed (big_units_may_fly).
-            if(kW8 && w_role ? big_units_may_fly(k, kt_count, kW8) : k + 3 < kt_count)
+            // Needed now: token step k and the weight units of pair k >> 1.  Issued after them and allowed to stay pending:
+            // token step k+1; two weight units (even k) or three (odd k), until the last pair is the one needed.
+            if(big_units_may_fly(k, kt_count, false))
             {
                 if(w_role)
                     wait_vmcnt<PAR ? 12 : 8>();
                 else
-                    wait_vmcnt<XG + (kMx ? 1 : 0)>(); // token-role instructions of one step
+                    wait_vmcnt<XG + 1>(); // token-role instructions of one step
             }
             else
                 wait_vmcnt<0>();
@@ -674,12 +735,7 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
             asm volatile("" ::: "memory");
             auto issue_next = [&]() __attribute__((always_inline)) {
                 if(w_role)
-                {
-                    if constexpr(!kW8)
-                        issue_w(big_unit_of_step(k, kW8), par_tag, nt_tag);
-                    else if constexpr(PAR == 0)
-                        issue_w(big_unit_of_step(k, kW8), std::integral_constant<int, -1>{}, nt_tag);
-                }
+                    issue_w(big_unit_of_step(k, false), par_tag, nt_tag);
                 else
                     issue_x(k + 2, XG);
             };
@@ -694,7 +750,7 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                 issue_next();
 
             // first unit of the pair that holds this step's weight bytes
-            const int pair0          = big_pair_of_step(k, kW8);
+            const int pair0          = big_pair_of_step(k, false);
             const unsigned char* wst = lds + ((pair0 + w_h) % kWSlots) * kWUnitBytes + w_off;
             const unsigned char* xst = lds + x_off + (k % kXStages) * kXStageBytes;
             [[maybe_unused]] const unsigned char* ysl =
@@ -714,18 +770,9 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                 for(int b = 0; b < 2; b++)
                 {
                     const unsigned char* wp = wst + b * 32 * (2 * kStepKB);
-                    if constexpr(kW8)
-                    {
-                        // 8 int8 of this lane's K group: 16-byte chunk (k & 3) * 2 + s of the row, half kg
-                        const int c8 = ((((k & 3) << 1) + s) ^ sw_wr) * kWChunkB + kg * 8;
-                        wf[b].lo     = int8x8_to_bf16x8(*reinterpret_cast<const uint2*>(wp + c8));
-                    }
-                    else
-                    {
-                        wf[b].lo = *reinterpret_cast<const uint4*>(wp + cw_lo);
-                        if constexpr(kOpB == 32)
-                            wf[b].hi = *reinterpret_cast<const uint4*>(wp + cw_hi);
-                    }
+                    wf[b].lo = *reinterpret_cast<const uint4*>(wp + cw_lo);
+                    if constexpr(kOpB == 32)
+                        wf[b].hi = *reinterpret_cast<const uint4*>(wp + cw_hi);
                 }
 #pragma unroll
                 for(int i = 0; i < NB; i++)
@@ -835,13 +882,17 @@ int big_tile_rows() { return kBigXRows; }
 
 bool big_tile_supported(int prec, int k_bytes0, int k_bytes1, bool y_i8)
 {
-    // K in whole pairs of 64-byte steps; the int8 path's down GEMM with bf16 Y against int8 weights in fours; the 8-bit
-    // gate+up GEMM also in odd numbers of steps, from five on (kOddK)
+    // K in whole pairs of 64-byte steps; the int8 path's down GEMM in whole 64-byte pieces of its weight rows, two at
+    // least (kOddW); the
+    // 8-bit gate+up GEMM also in odd numbers of steps, from five on (kOddK)
     const bool k0_odd = k_bytes0 % (2 * kStepKB) == kStepKB && k_bytes0 >= 5 * kStepKB;
     if(prec == MI355_MOE_FP8 && k0_odd)
         return k_bytes1 % (2 * kStepKB) == 0;
     if(prec == MI355_MOE_INT8)
-        return (k_bytes0 % (2 * kStepKB) == 0 || k0_odd) && k_bytes1 % ((y_i8 ? 2 : 4) * kStepKB) == 0;
+    {
+        const int kw1 = y_i8 ? k_bytes1 : k_bytes1 / 2;
+        return (k_bytes0 % (2 * kStepKB) == 0 || k0_odd) && kw1 % kStepKB == 0 && kw1 >= 2 * kStepKB;
+    }
     return (prec == MI355_MOE_BF16 || prec == MI355_MOE_FP16 || prec == MI355_MOE_FP8) && k_bytes0 % (2 * kStepKB) == 0 &&
            k_bytes1 % (2 * kStepKB) == 0;
 }

@@ -268,8 +268,8 @@ __device__ __attribute__((always_inline)) inline uint4 int8x8_to_bf16x8(uint2 v)
         const uint32_t f1 = __float_as_uint(static_cast<float>((s << 16) >> 24));
         const uint32_t f2 = __float_as_uint(static_cast<float>((s << 8) >> 24));
         const uint32_t f3 = __float_as_uint(static_cast<float>(s >> 24));
-        o[2 * h]     = (f1 & 0xffff0000u) | (f0 >> 16);
-        o[2 * h + 1] = (f3 & 0xffff0000u) | (f2 >> 16);
+        o[2 * h]     = __builtin_amdgcn_perm(f1, f0, 0x07060302u); // the upper halves of both
+        o[2 * h + 1] = __builtin_amdgcn_perm(f3, f2, 0x07060302u);
     }
     r.x = o[0];
     r.y = o[1];
