@@ -7,7 +7,7 @@
 //     workload (about 270 rows) is one tile and its weights are fetched once.
 //   * Both operands go global -> LDS with global_load_lds_dwordx4 (no staging registers).  The K loop
 //     advances in 64-byte steps.  Tokens (re-read from L2 by every column tile) arrive one 64-byte
-//     step at a time through a ring of three stages.  Weights are streamed from HBM exactly once, as
+//     step at a time through a ring of three to six stages (step_stages).  Weights are streamed from HBM exactly once, as
 //     full 128-byte lines, half of the tile's rows per unit (unit u = rows (u&1)*128.., K bytes
 //     [128*(u>>1), +128)), through a ring of six units issued four steps ahead.
 //   * The loads are issued from inline assembly so that their completion is tracked by hand:
@@ -52,22 +52,33 @@ constexpr int kMaxNB        = kBigXRows / 64; // token blocks per wave (5)
 constexpr int kWHalfRows    = kBigWRows / 2;
 constexpr int kWUnitBytes   = kWHalfRows * 2 * kStepKB; // 128 rows x 128 B
 constexpr int kWSlots       = 6;
-constexpr int kXStageBytes  = kBigXRows * kStepKB;
-constexpr int kXStages      = 3;
 constexpr int kYsRows       = 512;                      // padded rows per K block of a scale stage
 constexpr int kYsStageBytes = (kStepKB / 32) * kYsRows; // fp8 gemm1: e8m0 scales of 2 K blocks
 constexpr int kXOffset      = kWSlots * kWUnitBytes;
-constexpr int kYsOffset     = kXOffset + kXStages * kXStageBytes;
-constexpr int kLdsBytes     = kYsOffset + kXStages * kYsStageBytes;
-static_assert(kLdsBytes <= 160 * 1024, "LDS budget of a gfx950 compute unit");
+constexpr int kLdsBytes     = 160 * 1024; // of a gfx950 compute unit
 // Gate+up GEMM (token rows gathered by id): a token stage holds 128 bytes of K per row, two compute steps, so that a
 // token DMA instruction fetches eight whole 128-byte lines instead of sixteen half lines (a compute unit's address
-// path moves 100 GB/s in whole lines and 58 GB/s in halves).  Two such stages and a weight ring of five slots.
-constexpr int kXPairBytes   = kBigXRows * 2 * kStepKB;
+// path moves 100 GB/s in whole lines and 58 GB/s in halves).  Two such stages of a full tile and a weight ring of five slots.
 constexpr int kWSlotsPair   = 5;
 constexpr int kXOffsetPair  = kWSlotsPair * kWUnitBytes;
-constexpr int kLdsBytesPair = kXOffsetPair + 2 * kXPairBytes;
-static_assert(kLdsBytesPair <= 160 * 1024, "LDS budget of a gfx950 compute unit");
+
+// Token stages of a tile of `groups` 64-row token groups: as many as fit beside the weight ring.  A compute unit's requests
+// return in order, so a token stage arrives with the HBM latency of the weights ahead of it (1.4 us and more under load),
+// and a step of a tile of few rows, whose MFMAs take 0.2 .. 0.4 us, took half of that with the two stages a full tile has
+// room for (0.7 .. 0.9 us whatever the operand type or the rows).  More weight units in flight (seven slots) changed nothing.
+// Passes, two -> as many stages as fit: 900 tokens x 8 of 64 bf16 experts 2560 x 1536 363 -> 339 us, 1881 x 3 of 39 bf16 experts
+// 6976 x 2880 1080 -> 1038, 2048 x 8 of 128 int8 experts 4096 x 1536 743 -> 697, 777 x 4 of 32 fp16 experts 2880 x 2880 382 -> 372.
+constexpr int pair_stage_bytes(int groups) { return groups * 64 * 2 * kStepKB; }
+constexpr int pair_stages(int groups) { return groups <= 2 ? 4 : groups == 3 ? 3 : 2; }
+constexpr int step_stage_bytes(int groups) { return groups * 64 * kStepKB; }
+constexpr int step_stages(int groups, bool scales) { return groups <= 2 ? 6 : groups == 3 ? (scales ? 4 : 5) : groups == 4 ? (scales ? 3 : 4) : 3; }
+constexpr bool stages_fit(int groups)
+{
+    return kXOffsetPair + pair_stages(groups) * pair_stage_bytes(groups) <= kLdsBytes &&
+           kXOffset + step_stages(groups, false) * step_stage_bytes(groups) <= kLdsBytes &&
+           kXOffset + step_stages(groups, true) * (step_stage_bytes(groups) + kYsStageBytes) <= kLdsBytes;
+}
+static_assert(stages_fit(1) && stages_fit(2) && stages_fit(3) && stages_fit(4) && stages_fit(kMaxNB), "LDS budget");
 
 typedef __attribute__((address_space(3))) unsigned char lds_byte_t;
 
@@ -159,7 +170,9 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
     // earlier, inside the row, and the steps it serves read its second half.
     constexpr bool kOddW = !GEMM0 && (MODE == kI8 || kW8);
     constexpr int kWS     = kXPair ? kWSlotsPair : kWSlots;
-    constexpr int kXO     = kXPair ? kXOffsetPair : kXOffset;
+    // token stages (steps, or pairs of steps) of a tile, and the LDS offset of its scale stages
+    constexpr auto x_stages  = [](int groups) { return kXPair ? pair_stages(groups) : step_stages(groups, kMx); };
+    constexpr auto ys_offset = [](int groups) { return kXOffset + step_stages(groups, kMx) * step_stage_bytes(groups); };
 
     extern __shared__ __align__(16) unsigned char lds[];
 
@@ -319,13 +332,12 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
     const int64_t back     = half_window ? w_kadv / 2 : window_bytes * n_win;
     if(half_window && windows_left == 0) // (a slice of 64 bytes: the window begins in the slice before)
         stream -= back;
-    auto end_window = [&]() __attribute__((always_inline)) {
-        if(--windows_left == 0)
-        {
-            stream -= back;
-            if constexpr(kMx)
-                ys_base -= n_win * 2 * ys_step;
-        }
+    // (selects, not a branch: branches in the issue path cost time)
+    auto end_window = [&](int64_t bytes) __attribute__((always_inline)) {
+        const bool end = --windows_left == 0;
+        stream += bytes - (end ? back : 0);
+        if constexpr(kMx)
+            ys_base -= end ? n_win * 2 * ys_step : 0;
     };
 
     // weight role: unit u (half u & 1) -> ring slot u % 6
@@ -339,7 +351,7 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
         constexpr bool NT = decltype(nt_tag)::value;
         if(u >= n_wunits)
             return;
-        const uint32_t sbase     = lds_base + (u % kWS) * kWUnitBytes + q4 * 1024;
+        const uint32_t sbase     = lds_base + ((uint32_t)u % kWS) * kWUnitBytes + q4 * 1024;
         const unsigned char* src = stream;
 #pragma unroll
         for(int j = 0; j < 4; j++)
@@ -356,15 +368,14 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
         }
         if(H < 0 ? (u & 1) : H)
         {
-            stream += w_kadv;
-            end_window();
+            end_window(w_kadv);
         }
     };
-    // token role: step x -> ring stage x % 3
-    auto issue_x = [&](int x, int groups) __attribute__((always_inline)) {
+    // token role: step x -> ring stage x % x_stages(groups)
+    auto issue_x = [&](int x, int stage, int groups) __attribute__((always_inline)) {
         if(x >= kt_count)
             return;
-        const uint32_t sbase     = lds_base + kXOffset + (x % kXStages) * kXStageBytes + q4 * 1024;
+        const uint32_t sbase     = lds_base + kXOffset + stage * step_stage_bytes(groups) + q4 * 1024;
         const unsigned char* src = stream;
 #pragma unroll
         for(int j = 0; j < 5; j++)
@@ -373,29 +384,42 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
         if constexpr(kMx)
         {
             dma4(ys_base, doff[5],
-                 __builtin_amdgcn_readfirstlane(lds_base + kYsOffset + (x % kXStages) * kYsStageBytes +
+                 __builtin_amdgcn_readfirstlane(lds_base + ys_offset(groups) + stage * kYsStageBytes +
                                                 (q4 >> 1) * kYsRows + (q4 & 1) * 256));
             ys_base += ys_step;
         }
-        stream += x_step;
         if((x & (kW8 ? 3 : 1)) == (kW8 ? 3 : 1))
-            end_window();
+            end_window(x_step);
+        else
+            stream += x_step;
     };
 
-    // 128-byte token stages: pair m = steps 2 m and 2 m + 1 -> stage m & 1; two instructions per 64 rows of the tile
-    auto issue_x_pair = [&](int m, int groups) __attribute__((always_inline)) {
+    // 128-byte token stages: pair m = steps 2 m and 2 m + 1 -> stage m % x_stages(groups); two instructions per 64 rows of the
+    // tile
+    // (kOddK) token lanes of the half the last pair does not have fetch the other half from here on
+    auto halve_x = [&]() __attribute__((always_inline)) {
+        if constexpr(kXPair)
+        {
+#pragma unroll
+            for(int j = 0; j < 10; j++)
+            {
+                const int lrow = (q4 + 4 * j) * 8 + (lane >> 3);
+                doff[j] -= (((lane & 7) ^ ((lrow >> 1) & 7)) & 4) ? 64u : 0u;
+            }
+        }
+    };
+    auto issue_x_pair = [&](int m, int stage, int groups) __attribute__((always_inline)) {
         if constexpr(kXPair)
         {
             if(2 * m >= kt_count)
                 return;
-            const uint32_t sbase     = lds_base + kXO + (m & 1) * kXPairBytes + q4 * 1024;
+            const uint32_t sbase     = lds_base + kXOffsetPair + stage * pair_stage_bytes(groups) + q4 * 1024;
             const unsigned char* src = stream;
 #pragma unroll
             for(int j = 0; j < 10; j++)
                 if(j < 2 * groups)
                     dma16(src, doff[j], __builtin_amdgcn_readfirstlane(sbase + j * 4096));
-            stream += 2 * kStepKB;
-            end_window();
+            end_window(2 * kStepKB);
         }
     };
 
@@ -412,8 +436,8 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
             for(int v = 0; v < 16; v++)
                 acc[i][b][v] = 0;
 
-    // prologue: weight units 0..3 (0..4 when pipelined with six slots, unless a unit lasts four steps), token steps 0 and 1
-    // (and 2; or pairs 0 and 1)
+    // prologue: weight units 0..3 (0..4 when pipelined with six slots, unless a unit lasts four steps), all token
+    // stages (but one when not pipelined)
     using H0 = std::integral_constant<int, 0>;
     using H1 = std::integral_constant<int, 1>;
     if(w_role)
@@ -432,15 +456,19 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
     }
     else if constexpr(kXPair)
     {
-        issue_x_pair(0, x_groups);
-        issue_x_pair(1, x_groups);
+        const int stages = x_stages(x_groups);
+        for(int m = 0; m < stages; m++)
+        {
+            if(odd_k && m == kt_count >> 1)
+                halve_x();
+            issue_x_pair(m, m, x_groups);
+        }
     }
     else
     {
-        issue_x(0, x_groups);
-        issue_x(1, x_groups);
-        if constexpr(kPipe)
-            issue_x(2, x_groups);
+        const int stages = x_stages(x_groups) - (kPipe ? 0 : 1);
+        for(int x = 0; x < stages; x++)
+            issue_x(x, x, x_groups);
     }
 
     // per-lane LDS read offsets (swizzled chunk positions are per-lane constants)
@@ -458,6 +486,9 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
         constexpr int NB = decltype(nb_tag)::value;
         constexpr int XG = decltype(xg_tag)::value;
         constexpr int NF = NB > 0 ? NB : 1;
+        // (a weight-role wave owns blocks 0, 2, .., as many as the tile has token groups)
+        constexpr int kGroups = XG > 0 ? XG : NB > 0 ? NB : 1;
+        constexpr int kXS     = x_stages(kGroups);
         if constexpr(kPipe)
         {
             // operand registers of the step about to run
@@ -470,7 +501,7 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
             auto load_wf = [&](int kk, auto p_tag, int s, int b) __attribute__((always_inline)) {
                 constexpr int P          = decltype(p_tag)::value;
                 constexpr int kh         = P * 4; // first chunk of the step inside the 128-byte weight row
-                const unsigned char* wp  = lds + ((big_pair_of_step(kk, kW8) + w_h) % kWS) * kWUnitBytes + w_off + b * 32 * (2 * kStepKB);
+                const unsigned char* wp  = lds + ((uint32_t)(big_pair_of_step(kk, kW8) + w_h) % kWS) * kWUnitBytes + w_off + b * 32 * (2 * kStepKB);
                 const int cw_lo          = kOpB == 16 ? ((kh + 2 * s + kg) ^ sw_wr) * kWChunkB : ((kh + kg) ^ sw_wr) * kWChunkB;
                 const int cw_hi          = ((kh + 2 + kg) ^ sw_wr) * kWChunkB;
                 Frag f;
@@ -499,7 +530,7 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                 scale = 127;
                 if constexpr(kXPair)
                 {
-                    const unsigned char* xp = lds + kXO + ((kk >> 1) & 1) * kXPairBytes + (wt * 32 + r32 + i * 64) * (2 * kStepKB);
+                    const unsigned char* xp = lds + kXOffsetPair + ((uint32_t)(kk >> 1) % kXS) * pair_stage_bytes(kGroups) + (wt * 32 + r32 + i * 64) * (2 * kStepKB);
                     const int kh            = (kk & 1) * 4;
                     const int cx_lo         = kOpB == 16 ? ((kh + 2 * s + kg) ^ sw_w) * 16 : ((kh + kg) ^ sw_w) * 16;
                     const int cx_hi         = ((kh + 2 + kg) ^ sw_w) * 16;
@@ -509,14 +540,14 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                 }
                 else
                 {
-                    const unsigned char* xp = lds + x_off + (kk % kXStages) * kXStageBytes + i * 64 * kStepKB;
+                    const unsigned char* xp = lds + x_off + ((uint32_t)kk % kXS) * step_stage_bytes(kGroups) + i * 64 * kStepKB;
                     const int cx_lo         = kOpB == 16 ? ((2 * s + kg) ^ sw_x) * 16 : (kg ^ sw_x) * 16;
                     const int cx_hi         = ((2 + kg) ^ sw_x) * 16;
                     f.lo                    = *reinterpret_cast<const uint4*>(xp + cx_lo);
                     if constexpr(kOpB == 32)
                         f.hi = *reinterpret_cast<const uint4*>(xp + cx_hi);
                     if constexpr(kMx)
-                        scale = lds[kYsOffset + (kk % kXStages) * kYsStageBytes + kg * kYsRows + wt * 32 + r32 + i * 64];
+                        scale = lds[ys_offset(kGroups) + ((uint32_t)kk % kXS) * kYsStageBytes + kg * kYsRows + wt * 32 + r32 + i * 64];
                 }
                 return f;
             };
@@ -537,14 +568,14 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                 asm volatile("" ::: "memory");
             };
             constexpr int kXI = XG + (kMx ? 1 : 0); // token-role instructions of one step
-            // step 0's data: weight units 0 and 1 (2, 3, 4 may be pending), token step 0 (1 and 2 pending); with
-            // 128-byte token stages weight units 2 and 3 and token pair 1 may be pending
-            // (a unit of int8 weights lasts four steps: units 2 and 3)
+            // step 0's data: weight units 0 and 1 (2, 3, 4 may be pending; with 128-byte token stages, or where a unit lasts
+            // four steps, 2 and 3) and the first token stage (the others may be pending)
             const bool six = kt_count >= 6;
             if constexpr(kXPair)
-                sync(six, six, std::integral_constant<int, 8>{}, std::integral_constant<int, 2 * XG>{});
+                sync(six, kt_count >= 2 * kXS, std::integral_constant<int, 8>{}, std::integral_constant<int, 2 * XG * (kXS - 1)>{});
             else
-                sync(kW8 ? n_wunits >= 4 : six, six, std::integral_constant<int, (kW8 ? 8 : 12)>{}, std::integral_constant<int, 2 * kXI>{});
+                sync(kW8 ? n_wunits >= 4 : six, kt_count >= kXS, std::integral_constant<int, (kW8 ? 8 : 12)>{},
+                     std::integral_constant<int, kXI * (kXS - 1)>{});
             static_for<kSteps>([&](auto s_tag) __attribute__((always_inline)) {
                 constexpr int s = decltype(s_tag)::value;
                 wf[s][0]        = load_wf(0, H0{}, s, 0);
@@ -562,10 +593,11 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
             auto step = [&](int k, auto par_tag) __attribute__((always_inline)) {
                 constexpr int PAR = decltype(par_tag)::value;
                 using NPAR        = std::integral_constant<int, 1 - PAR>;
-                // The barrier of step k guarantees step k+1: token step k+1 (k+2 may be pending) and the weight pair
-                // of step k+1, that is units up to k+1 for even k (k+2 .. k+4 pending) or up to k+2 for odd k.
+                // The barrier of step k guarantees step k+1: token step k+1 (the kXS - 2 after it may be pending) and the
+                // weight pair of step k+1, that is units up to k+1 for even k (k+2 .. k+4 pending) or up to k+2 for odd k.
                 // 128-byte token stages: a weight unit less is in flight (unit k+3 may be pending at odd k), and the
-                // token pair of steps k+1 and k+2 is due at odd k, where it is the wave's only transfer.
+                // token pair of steps k+1 and k+2 is due at odd k (the kXS - 2 after it may be pending; at even k one more,
+                // its pair was due the step before).
                 // Steps 2 m and 2 m + 1 read the same weight pair and the same token stage, so only the barrier of
                 // the odd step has anything to guarantee, and what the even step overwrites (the slot of weight unit
                 // k - 1) was last read before the barrier of step k - 1: the even step has no barrier.
@@ -576,26 +608,29 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                 const bool counted = k + 4 < kt_count;
                 if constexpr(kXPair)
                 {
+                    // (all of them have been issued if the last step is further off)
                     if constexpr(PAR == 1 || kSteps == 1)
-                        sync(counted, counted, std::integral_constant<int, (PAR ? 4 : 8)>{},
-                             std::integral_constant<int, (PAR ? 0 : 2 * XG)>{});
+                        sync(counted, k + 2 * kXS - 2 < kt_count, std::integral_constant<int, (PAR ? 4 : 8)>{},
+                             std::integral_constant<int, 2 * XG * (kXS - (PAR ? 2 : 1))>{});
                 }
                 else if constexpr(kW8)
-                    sync(big_units_may_fly(k + 1, kt_count, kW8), counted, std::integral_constant<int, 8>{}, std::integral_constant<int, kXI>{});
+                    sync(big_units_may_fly(k + 1, kt_count, kW8), k + kXS <= kt_count, std::integral_constant<int, 8>{},
+                         std::integral_constant<int, kXI * (kXS - 2)>{});
                 else
-                    sync(counted, counted, std::integral_constant<int, (PAR ? 8 : 12)>{}, std::integral_constant<int, kXI>{});
+                    sync(counted, k + kXS <= kt_count, std::integral_constant<int, (PAR ? 8 : 12)>{},
+                         std::integral_constant<int, kXI * (kXS - 2)>{});
                 // the transfers of the step go out behind the MFMAs of the second token block (measured: 1 to 2 %
                 // faster than right after the barrier, where all eight waves queue up at the address unit while the
                 // MFMA pipe has nothing to do; one instruction behind every block is 5 % slower)
                 auto issue_next = [&]() __attribute__((always_inline)) {
                     if constexpr(kXPair)
                     {
-                        // slot (k + 4) % 5 held unit k - 1, stage ((k + 3) / 2) & 1 held the pair of steps k - 1 and
-                        // k - 2: both were last read during step k - 1, into registers, before this step's barrier
+                        // slot (k + 4) % 5 held unit k - 1, the stage of pair (k - 1) / 2 the tokens of steps k - 1 and k:
+                        // both were last read during step k - 1, into registers, before this step's barrier
                         if(w_role)
                             issue_w(k + 4, par_tag, nt_tag);
                         else if constexpr(PAR == 1)
-                            issue_x_pair((k + 3) >> 1, XG);
+                            issue_x_pair(((k - 1) >> 1) + kXS, (uint32_t)((k - 1) >> 1) % kXS, XG);
                     }
                     else if(w_role)
                     {
@@ -605,7 +640,7 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                             issue_w(big_unit_of_step(k, kW8), std::integral_constant<int, -1>{}, nt_tag);
                     }
                     else
-                        issue_x(k + 3, XG);
+                        issue_x(k + kXS, (uint32_t)k % kXS, XG);
                 };
                 constexpr int kIssueAfter = 1;
                 if constexpr(NB <= kIssueAfter)
@@ -655,10 +690,10 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
             if constexpr(kOddK)
             {
                 // the last window's units go out in steps kt_count - 5 and kt_count - 4 (rows of five steps or more: see
-                // big_tile_supported) and are the last to go out: from there on the lanes of the missing half fetch the
-                // other one
+                // big_tile_supported) and its tokens in step kt_count - 2 kXS, each the wave's last: from there on the lanes of
+                // the missing half fetch the other one
                 int k   = 0;
-                int end = odd_k ? kt_count - 5 : kt_count;
+                int end = !odd_k ? kt_count : kt_count - (w_role ? 5 : 2 * kXS + 1);
                 for(;;)
                 {
                     for(; k < end; k += 2)
@@ -681,15 +716,8 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                             doff[4 + j] -= back;
                         }
                     }
-                    else
-                    {
-#pragma unroll
-                        for(int j = 0; j < 10; j++)
-                        {
-                            const int lrow = (q4 + 4 * j) * 8 + (lane >> 3);
-                            doff[j] -= (((lane & 7) ^ ((lrow >> 1) & 7)) & 4) ? 64u : 0u;
-                        }
-                    }
+                    else if(kt_count > 2 * kXS) // (otherwise the last pair has gone out already)
+                        halve_x();
                 }
                 if(odd_k)
                     step(k, H0{});
@@ -717,13 +745,13 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
         auto step = [&](int k, auto par_tag) __attribute__((always_inline)) {
             constexpr int PAR = decltype(par_tag)::value;
             // Needed now: token step k and the weight units of pair k >> 1.  Issued after them and allowed to stay pending:
-            // token step k+1; two weight units (even k) or three (odd k), until the last pair is the one needed.
-            if(big_units_may_fly(k, kt_count, false))
+            // kXS - 2 token steps; two weight units (even k) or three (odd k), until the last pair is the one needed.
+            if(w_role ? big_units_may_fly(k, kt_count, false) : k + kXS - 2 < kt_count)
             {
                 if(w_role)
                     wait_vmcnt<PAR ? 12 : 8>();
                 else
-                    wait_vmcnt<XG + 1>(); // token-role instructions of one step
+                    wait_vmcnt<(XG + 1) * (kXS - 2)>(); // token-role instructions of the steps after it
             }
             else
                 wait_vmcnt<0>();
@@ -737,7 +765,7 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                 if(w_role)
                     issue_w(big_unit_of_step(k, false), par_tag, nt_tag);
                 else
-                    issue_x(k + 2, XG);
+                    issue_x(k + kXS - 1, (uint32_t)(k + kXS - 1) % kXS, XG);
             };
             // Where in the step the transfers go out: right here, or after the MFMAs of token block kIssueAfter.  The
             // buffers they write are free from the barrier on either way, but issued here the handful of scalar and
@@ -751,10 +779,10 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
 
             // first unit of the pair that holds this step's weight bytes
             const int pair0          = big_pair_of_step(k, false);
-            const unsigned char* wst = lds + ((pair0 + w_h) % kWSlots) * kWUnitBytes + w_off;
-            const unsigned char* xst = lds + x_off + (k % kXStages) * kXStageBytes;
+            const unsigned char* wst = lds + ((uint32_t)(pair0 + w_h) % kWSlots) * kWUnitBytes + w_off;
+            const unsigned char* xst = lds + x_off + ((uint32_t)k % kXS) * step_stage_bytes(kGroups);
             [[maybe_unused]] const unsigned char* ysl =
-                lds + kYsOffset + (k % kXStages) * kYsStageBytes + kg * kYsRows + wt * 32 + r32;
+                lds + ys_offset(kGroups) + ((uint32_t)k % kXS) * kYsStageBytes + kg * kYsRows + wt * 32 + r32;
             constexpr int kh = PAR * 4; // first chunk of this step inside the 128-byte weight row
 #pragma unroll
             for(int s = 0; s < kSteps; s++)
@@ -844,8 +872,7 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
 template <int MODE, bool GEMM0, bool WPERM>
 int launch_big_w(const GemmParams& p, int max_tiles, hipStream_t stream)
 {
-    constexpr bool kMx  = MODE == kFp8 && !GEMM0;
-    const size_t lds    = (GEMM0 && MODE != kBf16W8) ? kLdsBytesPair : kMx ? kLdsBytes : kYsOffset;
+    const size_t lds    = kLdsBytes;
     // the dynamic LDS limit is an attribute of the function on one device: set once per device, whichever host
     // thread gets there first (the others wait for it)
     static std::once_flag attr_once[64];
