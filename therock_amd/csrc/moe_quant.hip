@@ -4,6 +4,7 @@
 #include "moe_gemm_device.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace mi355 {
 using namespace gemm;
@@ -26,38 +27,103 @@ __device__ inline unsigned char quantise_one(float v)
     }
 }
 
-// eight quotients o[i] * (1 / s) -> eight codes in two dwords.  e4m3: the conversion instruction packs two codes
-// into a chosen half of a dword, so four of them fill both dwords with no masking or shifting.
-template <bool FP8>
-__device__ inline uint2 quantise_8(const float (&o)[8], double s_rcp)
+// Four integers -> their low bytes in one dword.
+__device__ inline uint32_t pack_low_bytes(int a, int b, int c, int d)
 {
+    const uint32_t ab = __builtin_amdgcn_perm(static_cast<uint32_t>(b), static_cast<uint32_t>(a), 0x0c0c0400u);
+    const uint32_t cd = __builtin_amdgcn_perm(static_cast<uint32_t>(d), static_cast<uint32_t>(c), 0x04000c0cu);
+    return ab | cd;
+}
+
+// A row's quantisation by its largest magnitude.  scale() is what the codes stand for: amax / qmax, 1 for a row of zeros.
+// lo and hi bracket its reciprocal: v_rcp_f32 is within 1 ulp and the roundings that follow (of the scale itself, the two
+// products here and the one with the element) add 2^-22 at most, so that x * lo and x * hi enclose fp32(x / scale()), and with
+// them every monotone conversion of it.  Outside the range where none of these can overflow or lose bits to subnormals
+// (rows of zeros and infinities among them) both are NaN.
+template <bool FP8>
+struct RowScale
+{
+    static constexpr float kMax = FP8 ? 448.0f : 127.0f;
+    float amax, lo, hi;
+    __device__ explicit RowScale(float m) : amax(m)
+    {
+        const float r = m >= 0x1p-100f && m <= 0x1p100f ? kMax * __builtin_amdgcn_rcpf(m) : __builtin_nanf("");
+        lo            = r * (1.0f - 0x1p-20f);
+        hi            = r * (1.0f + 0x1p-20f);
+    }
+    __device__ float scale() const { return amax > 0.f ? amax / kMax : 1.0f; }
+};
+
+// Eight quotients o[i] / scale -> eight codes in two dwords; NEAREST: int8 codes rounded to nearest even instead of toward
+// zero.  A code is right where both ends of the bracket give it, which fails for one quotient in some 2^14 (those within
+// 2^-20 of a code's boundary): one piece of eight in 2000 is done again with the fp64 product that rounds like the
+// division.  That product, two conversions at a quarter of the fp32 rate, was most of these kernels' instructions.
+// A NaN becomes -128 and -127 (e4m3: -448 and NaN) at the two ends, so it goes to the exact form too.
+// 3001 x 8 smooth-quantised int8 rows of 4096: 62 -> 50 us (with half the registers, see the launch); 24008 rows of 1536
+// re-quantised between the GEMMs 30 -> 25 us.
+template <bool FP8, bool NEAREST = false>
+__device__ inline uint2 quantise_8(const float (&o)[8], const RowScale<FP8>& row)
+{
+    uint2 lo, hi;
+    auto fp8x4 = [](float a, float b, float c, float d) {
+        const int w = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false);
+        return static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(c, d, w, true));
+    };
     if constexpr(FP8)
     {
-        float c[8];
+        float l[8], h[8];
 #pragma unroll
         for(int i = 0; i < 8; i++)
-            c[i] = fminf(fmaxf(div_by_row_scale(o[i], s_rcp), -448.f), 448.f);
-        int w0 = __builtin_amdgcn_cvt_pk_fp8_f32(c[0], c[1], 0, false);
-        w0     = __builtin_amdgcn_cvt_pk_fp8_f32(c[2], c[3], w0, true);
-        int w1 = __builtin_amdgcn_cvt_pk_fp8_f32(c[4], c[5], 0, false);
-        w1     = __builtin_amdgcn_cvt_pk_fp8_f32(c[6], c[7], w1, true);
-        return make_uint2(static_cast<uint32_t>(w0), static_cast<uint32_t>(w1));
+        {
+            l[i] = __builtin_amdgcn_fmed3f(o[i] * row.lo, -448.f, 448.f);
+            h[i] = o[i] * row.hi;
+        }
+        lo = make_uint2(fp8x4(l[0], l[1], l[2], l[3]), fp8x4(l[4], l[5], l[6], l[7]));
+        hi = make_uint2(fp8x4(h[0], h[1], h[2], h[3]), fp8x4(h[4], h[5], h[6], h[7]));
     }
     else
     {
-        uint32_t w[2] = {0u, 0u};
+        int l[8], h[8];
 #pragma unroll
         for(int i = 0; i < 8; i++)
-            w[i >> 2] |= static_cast<uint32_t>(quantise_one<false>(div_by_row_scale(o[i], s_rcp))) << (8 * (i & 3));
-        return make_uint2(w[0], w[1]);
+        {
+            const float a = __builtin_amdgcn_fmed3f(o[i] * row.lo, -128.f, 127.f);
+            const float b = __builtin_amdgcn_fmed3f(o[i] * row.hi, -127.f, 127.f);
+            l[i]          = static_cast<int>(NEAREST ? __builtin_rintf(a) : a);
+            h[i]          = static_cast<int>(NEAREST ? __builtin_rintf(b) : b);
+        }
+        lo = make_uint2(pack_low_bytes(l[0], l[1], l[2], l[3]), pack_low_bytes(l[4], l[5], l[6], l[7]));
+        hi = make_uint2(pack_low_bytes(h[0], h[1], h[2], h[3]), pack_low_bytes(h[4], h[5], h[6], h[7]));
     }
+    if(((lo.x ^ hi.x) | (lo.y ^ hi.y)) != 0)
+    {
+        const double s_rcp = row_reciprocal(row.scale());
+        float q[8];
+#pragma unroll
+        for(int i = 0; i < 8; i++)
+            q[i] = div_by_row_scale(o[i], s_rcp);
+        if constexpr(FP8)
+        {
+#pragma unroll
+            for(int i = 0; i < 8; i++)
+                q[i] = fminf(fmaxf(q[i], -448.f), 448.f);
+            lo = make_uint2(fp8x4(q[0], q[1], q[2], q[3]), fp8x4(q[4], q[5], q[6], q[7]));
+        }
+        else
+        {
+            int c[8];
+#pragma unroll
+            for(int i = 0; i < 8; i++)
+                c[i] = NEAREST ? static_cast<int>(__builtin_rintf(q[i])) : static_cast<int>(static_cast<signed char>(quantise_one<false>(q[i])));
+            lo = make_uint2(pack_low_bytes(c[0], c[1], c[2], c[3]), pack_low_bytes(c[4], c[5], c[6], c[7]));
+        }
+    }
+    return lo;
 }
 
 __device__ inline float block_max_256(float v, float* s_red)
 {
-#pragma unroll
-    for(int d = 32; d > 0; d >>= 1)
-        v = fmaxf(v, __shfl_xor(v, d));
+    v = wave_reduce_max(v, 0.f);
     if((threadIdx.x & 63) == 0)
         s_red[threadIdx.x >> 6] = v;
     __syncthreads();
@@ -119,12 +185,10 @@ __device__ inline float quantise_row(const uint16_t* __restrict__ xr, const floa
         amax          = block_max_256(amax, s_red);
         // a row of zeros: the scale written is 1 (row-wise quant) or 0 (smooth-quant, as amax / qmax gives);
         // either way the row's codes are 0, never the 0 / 0 the plain formula would convert
-        const float s_out = (amax > 0.f || !unit_scale_when_zero) ? amax / qmx : 1.0f;
-        const float s     = amax > 0.f ? s_out : 1.0f;
         if(threadIdx.x == 0)
-            *scale_out = s_out;
-        const double s_rcp = row_reciprocal(s);
-        auto store = [&](int c, const float (&o)[8]) { *reinterpret_cast<uint2*>(qr + c * 8) = quantise_8<FP8>(o, s_rcp); };
+            *scale_out = (amax > 0.f || !unit_scale_when_zero) ? amax / qmx : 1.0f;
+        const RowScale<FP8> row(amax);
+        auto store = [&](int c, const float (&o)[8]) { *reinterpret_cast<uint2*>(qr + c * 8) = quantise_8<FP8>(o, row); };
 #pragma unroll
         for(int j = 0; j < kQuantCache; j++)
         {
@@ -192,7 +256,7 @@ __global__ __launch_bounds__(256) void moe_smoothquant_kernel(const uint16_t* __
 // Vector form (hidden % 8 == 0, aligned rows): one workgroup per token walks its slots, so the token's row is
 // read once (its first kQuantCache pieces per thread stay in registers) and only the experts' smooth scales and
 // the quantised rows move per slot.
-template <bool FP8>
+template <bool FP8, int PIECES>
 __global__ __launch_bounds__(256) void moe_smoothquant_vec_kernel(const uint16_t* __restrict__ x,
                                                                    const float* __restrict__ smscale,
                                                                    const int* __restrict__ topk_ids, int tokens,
@@ -227,19 +291,19 @@ __global__ __launch_bounds__(256) void moe_smoothquant_vec_kernel(const uint16_t
     };
     // the smooth scales of the cached pieces, for the slot about to be processed: fetched one slot ahead, so that
     // their latency passes under the previous slot's reduction, conversions and stores
-    float4 sm[kQuantCache][2];
+    float4 sm[PIECES][2];
     auto fetch_scales = [&](const float* sr) {
 #pragma unroll
-        for(int j = 0; j < kQuantCache; j++)
+        for(int j = 0; j < PIECES; j++)
             if(threadIdx.x + 256 * j < chunks)
             {
                 sm[j][0] = *reinterpret_cast<const float4*>(sr + (threadIdx.x + 256 * j) * 8);
                 sm[j][1] = *reinterpret_cast<const float4*>(sr + (threadIdx.x + 256 * j) * 8 + 4);
             }
     };
-    float xv[kQuantCache][8];
+    float xv[PIECES][8];
 #pragma unroll
-    for(int j = 0; j < kQuantCache; j++)
+    for(int j = 0; j < PIECES; j++)
         if(threadIdx.x + 256 * j < chunks)
             load_x(threadIdx.x + 256 * j, xv[j]);
     if(topk > 0)
@@ -247,10 +311,10 @@ __global__ __launch_bounds__(256) void moe_smoothquant_vec_kernel(const uint16_t
     for(int k = 0; k < topk; k++)
     {
         const float* sr = scales_of_slot(k);
-        float v[kQuantCache][8];
+        float v[PIECES][8];
         float amax = 0.f;
 #pragma unroll
-        for(int j = 0; j < kQuantCache; j++)
+        for(int j = 0; j < PIECES; j++)
         {
             const int c = threadIdx.x + 256 * j;
             if(c < chunks)
@@ -265,7 +329,7 @@ __global__ __launch_bounds__(256) void moe_smoothquant_vec_kernel(const uint16_t
         }
         if(k + 1 < topk)
             fetch_scales(scales_of_slot(k + 1));
-        for(int c = threadIdx.x + 256 * kQuantCache; c < chunks; c += 256)
+        for(int c = threadIdx.x + 256 * PIECES; PIECES == kQuantCache && c < chunks; c += 256)
         {
             float a[8], b[8];
             load_x(c, a);
@@ -275,24 +339,22 @@ __global__ __launch_bounds__(256) void moe_smoothquant_vec_kernel(const uint16_t
                 amax = fmaxf(amax, fabsf(b[i]));
         }
         amax            = block_max_256(amax, s_red[k & 1]); // two buffers: one barrier per slot suffices
-        const float ys_out = amax / qmx;
-        const float ys     = amax > 0.f ? ys_out : 1.0f; // a row of zeros: scale 0, codes 0 (not 0 / 0)
-        const int64_t r    = (int64_t)k * tokens + t;
+        const int64_t r = (int64_t)k * tokens + t;
         if(threadIdx.x == 0)
-            yscale[r] = ys_out;
+            yscale[r] = amax / qmx; // (a row of zeros: scale 0, codes 0)
         unsigned char* qr = qy + r * y_stride;
-        const double ys_rcp = row_reciprocal(ys);
+        const RowScale<FP8> row(amax);
         // (streaming stores: the quantised rows are written once and should not push the experts' scales out of L2)
         auto store = [&](int c, const float (&o)[8]) {
             typedef __attribute__((ext_vector_type(2))) unsigned u32x2_t;
-            const uint2 q = quantise_8<FP8>(o, ys_rcp);
+            const uint2 q = quantise_8<FP8>(o, row);
             __builtin_nontemporal_store(u32x2_t{q.x, q.y}, reinterpret_cast<u32x2_t*>(qr + c * 8));
         };
 #pragma unroll
-        for(int j = 0; j < kQuantCache; j++)
+        for(int j = 0; j < PIECES; j++)
             if(threadIdx.x + 256 * j < chunks)
                 store(threadIdx.x + 256 * j, v[j]);
-        for(int c = threadIdx.x + 256 * kQuantCache; c < chunks; c += 256)
+        for(int c = threadIdx.x + 256 * PIECES; PIECES == kQuantCache && c < chunks; c += 256)
         {
             float a[8], b[8];
             load_x(c, a);
@@ -312,7 +374,7 @@ __global__ __launch_bounds__(256) void moe_smoothquant_vec_kernel(const uint16_t
 // is computed by the same expressions as in the per-token form: the results are the same bits.
 constexpr int kSqRange   = 128;  // tokens per range
 constexpr int kSqMaxList = 8192; // routing entries of a range (kSqRange x topk)
-template <bool FP8>
+template <bool FP8, int PIECES>
 __global__ __launch_bounds__(256) void moe_smoothquant_grouped_kernel(const uint16_t* __restrict__ x,
                                                                        const float* __restrict__ smscale,
                                                                        const int* __restrict__ topk_ids, int tokens,
@@ -345,9 +407,9 @@ __global__ __launch_bounds__(256) void moe_smoothquant_grouped_kernel(const uint
     if(n == 0)
         return;
     const float* sr = smscale + (int64_t)e * hidden;
-    float4 sm[kQuantCache][2];
+    float4 sm[PIECES][2];
 #pragma unroll
-    for(int j = 0; j < kQuantCache; j++)
+    for(int j = 0; j < PIECES; j++)
         if(threadIdx.x + 256 * j < chunks)
         {
             sm[j][0] = *reinterpret_cast<const float4*>(sr + (threadIdx.x + 256 * j) * 8);
@@ -368,11 +430,11 @@ __global__ __launch_bounds__(256) void moe_smoothquant_grouped_kernel(const uint
         o[0] = in[0] * s0.x; o[1] = in[1] * s0.y; o[2] = in[2] * s0.z; o[3] = in[3] * s0.w;
         o[4] = in[4] * s1.x; o[5] = in[5] * s1.y; o[6] = in[6] * s1.z; o[7] = in[7] * s1.w;
     };
-    uint4 raw[kQuantCache];
+    uint4 raw[PIECES];
     auto fetch_row = [&](int entry) {
         const uint16_t* xr = x + (int64_t)(t0 + entry / topk) * x_stride;
 #pragma unroll
-        for(int j = 0; j < kQuantCache; j++)
+        for(int j = 0; j < PIECES; j++)
             if(threadIdx.x + 256 * j < chunks)
                 raw[j] = *reinterpret_cast<const uint4*>(xr + (threadIdx.x + 256 * j) * 8);
     };
@@ -383,10 +445,10 @@ __global__ __launch_bounds__(256) void moe_smoothquant_grouped_kernel(const uint
         const int t        = t0 + entry / topk;
         const int k        = entry - (entry / topk) * topk;
         const uint16_t* xr = x + (int64_t)t * x_stride;
-        float v[kQuantCache][8];
+        float v[PIECES][8];
         float amax = 0.f;
 #pragma unroll
-        for(int j = 0; j < kQuantCache; j++)
+        for(int j = 0; j < PIECES; j++)
             if(threadIdx.x + 256 * j < chunks)
             {
                 float xv[8];
@@ -400,7 +462,7 @@ __global__ __launch_bounds__(256) void moe_smoothquant_grouped_kernel(const uint
             }
         if(m + 1 < n)
             fetch_row(s_list[m + 1]);
-        for(int c = threadIdx.x + 256 * kQuantCache; c < chunks; c += 256)
+        for(int c = threadIdx.x + 256 * PIECES; PIECES == kQuantCache && c < chunks; c += 256)
         {
             float a[8], b[8];
             unpack(*reinterpret_cast<const uint4*>(xr + c * 8), a);
@@ -410,23 +472,21 @@ __global__ __launch_bounds__(256) void moe_smoothquant_grouped_kernel(const uint
                 amax = fmaxf(amax, fabsf(b[i]));
         }
         amax               = block_max_256(amax, s_red[m & 1]); // two buffers: one barrier per row suffices
-        const float ys_out = amax / qmx;
-        const float ys     = amax > 0.f ? ys_out : 1.0f; // a row of zeros: scale 0, codes 0 (not 0 / 0)
-        const int64_t r    = (int64_t)k * tokens + t;
+        const int64_t r = (int64_t)k * tokens + t;
         if(threadIdx.x == 0)
-            yscale[r] = ys_out;
+            yscale[r] = amax / qmx; // (a row of zeros: scale 0, codes 0)
         unsigned char* qr   = qy + r * y_stride;
-        const double ys_rcp = row_reciprocal(ys);
+        const RowScale<FP8> row(amax);
         auto store = [&](int c, const float (&o)[8]) {
             typedef __attribute__((ext_vector_type(2))) unsigned u32x2_t;
-            const uint2 q = quantise_8<FP8>(o, ys_rcp);
+            const uint2 q = quantise_8<FP8>(o, row);
             __builtin_nontemporal_store(u32x2_t{q.x, q.y}, reinterpret_cast<u32x2_t*>(qr + c * 8));
         };
 #pragma unroll
-        for(int j = 0; j < kQuantCache; j++)
+        for(int j = 0; j < PIECES; j++)
             if(threadIdx.x + 256 * j < chunks)
                 store(threadIdx.x + 256 * j, v[j]);
-        for(int c = threadIdx.x + 256 * kQuantCache; c < chunks; c += 256)
+        for(int c = threadIdx.x + 256 * PIECES; PIECES == kQuantCache && c < chunks; c += 256)
         {
             float a[8], b[8];
             unpack(*reinterpret_cast<const uint4*>(xr + c * 8), a);
@@ -507,26 +567,11 @@ __global__ __launch_bounds__(256) void moe_requant_y_kernel(const uint16_t* __re
         for(int i = 0; i < 8; i++)
             amax = fmaxf(amax, fabsf(t[i]));
     }
-#pragma unroll
-    for(int d = 32; d > 0; d >>= 1)
-        amax = fmaxf(amax, __shfl_xor(amax, d));
-    const float ys_out = amax / (FP8 ? 448.0f : 127.0f);
-    const float ys     = amax > 0.f ? ys_out : 1.0f; // a row of zeros: scale 0, codes 0
+    amax = wave_reduce_max(amax, 0.f);
     if(lane == 0)
-        yscale[row] = ys_out;
-    const double ys_rcp = row_reciprocal(ys);
-    auto store = [&](int c, const float (&o)[8]) {
-        if constexpr(FP8)
-            *reinterpret_cast<uint2*>(dst(c)) = quantise_8<true>(o, ys_rcp);
-        else
-        {
-            uint32_t w[2] = {0u, 0u};
-#pragma unroll
-            for(int i = 0; i < 8; i++)
-                w[i >> 2] |= (static_cast<uint32_t>(static_cast<int>(__builtin_rintf(div_by_row_scale(o[i], ys_rcp)))) & 0xffu) << (8 * (i & 3));
-            *reinterpret_cast<uint2*>(dst(c)) = make_uint2(w[0], w[1]);
-        }
-    };
+        yscale[row] = amax / (FP8 ? 448.0f : 127.0f); // (a row of zeros: scale 0, codes 0)
+    const RowScale<FP8> rs(amax);
+    auto store = [&](int c, const float (&o)[8]) { *reinterpret_cast<uint2*>(dst(c)) = quantise_8<FP8, !FP8>(o, rs); };
 #pragma unroll
     for(int j = 0; j < kQuantCache; j++)
         if(lane + 64 * j < chunks)
@@ -624,16 +669,22 @@ int launch_moe_smoothquant(const mi355_moe_smoothquant_args& a, int32_t q_dtype,
     const int64_t ranges8 = ceil_div<int64_t>(ceil_div(a.tokens, kSqRange), 8);
     const bool grouped    = vec && (int64_t)a.experts * a.hidden_size * (int64_t)sizeof(float) > (3ll << 20) &&
                          kSqRange * a.topk <= kSqMaxList && ranges8 * a.experts * 8 < (1ll << 31);
-    if(grouped)
-    {
-        const dim3 grid((unsigned)(ranges8 * a.experts * 8));
-        q_dtype == MI355_MOE_FP8 ? launch(moe_smoothquant_grouped_kernel<true>, grid)
-                                 : launch(moe_smoothquant_grouped_kernel<false>, grid);
-    }
-    else if(q_dtype == MI355_MOE_FP8)
-        vec ? launch(moe_smoothquant_vec_kernel<true>, per_token) : launch(moe_smoothquant_kernel<true>, per_row);
-    else
-        vec ? launch(moe_smoothquant_vec_kernel<false>, per_token) : launch(moe_smoothquant_kernel<false>, per_row);
+    auto of_type = [&](auto fp8_tag, auto pieces_tag) {
+        constexpr bool FP8   = decltype(fp8_tag)::value;
+        constexpr int PIECES = decltype(pieces_tag)::value;
+        if(grouped)
+            launch(moe_smoothquant_grouped_kernel<FP8, PIECES>, dim3((unsigned)(ranges8 * a.experts * 8)));
+        else if(vec)
+            launch(moe_smoothquant_vec_kernel<FP8, PIECES>, per_token);
+        else
+            launch(moe_smoothquant_kernel<FP8>, per_row);
+    };
+    // rows of up to 4096 columns need half the registers: twice the waves per compute unit
+    auto pieces = [&](auto fp8_tag) {
+        a.hidden_size <= 2 * 256 * 8 ? of_type(fp8_tag, std::integral_constant<int, 2>{})
+                                     : of_type(fp8_tag, std::integral_constant<int, kQuantCache>{});
+    };
+    q_dtype == MI355_MOE_FP8 ? pieces(std::true_type{}) : pieces(std::false_type{});
     MI355_HIP_TRY(hipGetLastError());
     return MI355_MOE_OK;
 }
