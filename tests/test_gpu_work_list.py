@@ -37,3 +37,22 @@ def test_one_workgroup_sort_at_its_edges(tokens, experts, topk):
     if experts > 1:
         check_sorting(np.minimum(ids, 1) if topk == 1 else ids, rng.random((tokens, topk), dtype=np.float32), experts, 48,
                       mask=(np.arange(experts) % 2 == 0).astype(np.int32))
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "int8"])
+@pytest.mark.parametrize("masked", [False, True])
+def test_scan_pass_lists_experts_of_many_tiles(masked, dtype):
+    # more entries than the one-workgroup sort takes: one expert of hundreds of tiles, empty and masked ones between and last
+    from tests.gpu_util import rel_l2, run_fused_moe
+    counts = [0, 12001, 0, 33, 4000, 1, 500, 0]
+    cfg = mi.MoeConfig("many_tiles", sum(counts), 128, 128, len(counts), 1, dtype, "softmax_renorm", unit=32)
+    assert cfg.tokens > 16384  # kOneShotMaxEntries
+    inp = mi.make_inputs_np(cfg, 3)
+    inp["topk_ids"] = np.random.default_rng(4).permutation(np.repeat(np.arange(len(counts)), counts)).astype(np.int32)[:, None]
+    mask = np.array([1, 1, 0, 1, 1, 1, 0, 1], np.int32) if masked else None
+    if masked:  # weights of the local experts only
+        for k in ("g", "d", "g_scale", "d_scale"):
+            inp[k] = None if inp[k] is None else inp[k][:int(mask.sum())]
+    got, _ = run_fused_moe(cfg, inp, mask=mask)
+    ref, _ = oracle_out(cfg, inp, mask)
+    assert rel_l2(oracle.bf16_to_f32(got), ref) <= TOL[dtype]

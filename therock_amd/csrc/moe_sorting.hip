@@ -138,6 +138,22 @@ struct ScanShared
     int wave4[4][kScanWaves + 1];
 };
 
+// last expert whose base[] is at or before t (experts that own nothing share their base with the next one that does,
+// and come before it)
+__device__ inline int expert_of(const int* base, int E, int t)
+{
+    int lo = 0, hi = E; // first expert with base > t
+    while(lo < hi)
+    {
+        const int mid = (lo + hi) >> 1;
+        if(base[mid] <= t)
+            lo = mid + 1;
+        else
+            hi = mid;
+    }
+    return lo - 1;
+}
+
 // Pass 2, run by one 1024-thread block.  counts is [nseg][E] (global or LDS): on entry the
 // per-segment histogram, on exit the output position of each segment's first entry per expert
 // (-1 for experts that produce no output).
@@ -263,21 +279,8 @@ __device__ inline void scan_phase(ScanShared& s, int* counts, int nseg, int E, i
                 sorted_w[pos]   = 0.f;
             }
         }
-        // the expert of output tile t: the last one whose first tile is at or before t (experts without tiles share
-        // their first-tile index with the next expert that has some, and come before it)
         for(int t = tid; t < total_tiles; t += kScanBlock)
-        {
-            int lo = 0, hi = E; // first expert with tbase > t
-            while(lo < hi)
-            {
-                const int mid = (lo + hi) >> 1;
-                if(s.tbase[mid] <= t)
-                    lo = mid + 1;
-                else
-                    hi = mid;
-            }
-            sorted_eid[t] = s.oeid[lo - 1];
-        }
+            sorted_eid[t] = s.oeid[expert_of(s.tbase, E, t)];
     }
     else
     for(int ex = wave; ex < E; ex += kScanWaves)
@@ -304,7 +307,6 @@ __device__ inline void scan_phase(ScanShared& s, int* counts, int nseg, int E, i
     // work list of the grouped GEMMs: the rows of an expert (without its padding) split evenly into tiles
     if(plan.tile_map != nullptr)
     {
-        const int rows    = my_rows;
         int rows_per_tile = plan.rows_per_tile;
         if(plan.alt_rows_per_tile > 0) // (uniform: every thread takes this branch or none)
         {
@@ -313,23 +315,27 @@ __device__ inline void scan_phase(ScanShared& s, int* counts, int nseg, int E, i
         }
         if(tid == 0)
             plan.tile_map[1] = rows_per_tile;
-        const int nt   = ceil_div(rows, rows_per_tile);
+        // All of the block's threads share the experts' tiles: one that holds a sixth of the entries has a hundred, and a
+        // single thread writing them was almost half of the pass (32768 tokens x 6 of 64 experts, Zipf: 23.9 -> 15.3 us).  A
+        // thread per tile that searches its expert costs experts of a few tiles 1 us.
+        int* mbase = s.part; // first tile of the expert (the walks over the segments' sums end before the scan's barriers)
         int n_tiles;
-        const int tb = block_exclusive_scan<kScanWaves>(nt, s.wave, n_tiles);
+        const int tb = block_exclusive_scan<kScanWaves>(ceil_div(my_rows, rows_per_tile), s.wave, n_tiles);
+        if(tid < E)
+            mbase[tid] = tb;
+        __syncthreads();
+        const int rows = e < E && s.tiles[e] > 0 ? s.cnt[e] : 0;
+        const int nt   = ceil_div(rows, rows_per_tile);
         if(nt > 0)
         {
-            const int per = round_up(ceil_div(rows, nt), 32);
-            for(int j = 0; j < nt && tb + j < plan.max_tiles; j++)
+            const int first = mbase[e];
+            const int per   = round_up(ceil_div(rows, nt), 32);
+            const int r0    = s.tbase[e] * U;
+            for(int j = part; j < nt && first + j < plan.max_tiles; j += kScanBlock / Ep)
             {
-                int* ent = plan.tile_map + kMapHdr + (tb + j) * kMapEnt;
-                ent[0]   = s.oeid[tid];
-                ent[1]   = s.tbase[tid] * U + j * per;
-                ent[2]   = min(per, rows - j * per);
-                ent[3]   = tb;
-                ent[4]   = nt;
-                ent[5]   = s.tbase[tid] * U;
-                ent[6]   = rows;
-                ent[7]   = per;
+                int4* ent = reinterpret_cast<int4*>(plan.tile_map + kMapHdr + (first + j) * kMapEnt);
+                ent[0]    = make_int4(s.oeid[e], r0 + j * per, min(per, rows - j * per), first);
+                ent[1]    = make_int4(nt, r0, rows, per);
             }
         }
         if(tid == 0)
@@ -373,22 +379,6 @@ struct OneShotShared
     int mbase[kOneShotMaxExperts];  // first GEMM tile
     int wsum[6][kOneShotMaxExperts / kWave];
 };
-
-// last expert whose base[] is at or before t (experts that own nothing share their base with the next one that does,
-// and come before it)
-__device__ inline int expert_of(const int* base, int E, int t)
-{
-    int lo = 0, hi = E; // first expert with base > t
-    while(lo < hi)
-    {
-        const int mid = (lo + hi) >> 1;
-        if(base[mid] <= t)
-            lo = mid + 1;
-        else
-            hi = mid;
-    }
-    return lo - 1;
-}
 
 // ---- whole sort in one workgroup (block 0); the other blocks zero moe_buf.
 // Up to STEPS x 1024 entries and 256 experts.  A chain of latencies in one workgroup, so what counts is its length:
