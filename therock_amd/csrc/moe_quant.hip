@@ -54,9 +54,40 @@ struct RowScale
     __device__ float scale() const { return amax > 0.f ? amax / kMax : 1.0f; }
 };
 
-// Eight quotients o[i] / scale -> eight codes in two dwords; NEAREST: int8 codes rounded to nearest even instead of toward
-// zero.  A code is right where both ends of the bracket give it, which fails for one quotient in some 2^14 (those within
-// 2^-20 of a code's boundary): one piece of eight in 2000 is done again with the fp64 product that rounds like the
+__device__ inline uint32_t fp8x4(float a, float b, float c, float d)
+{
+    const int w = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false);
+    return static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(c, d, w, true));
+}
+
+// Eight codes in two dwords, each from the quotient rounded like the division; NEAREST: int8 codes rounded to nearest even
+// instead of toward zero.
+template <bool FP8, bool NEAREST>
+__device__ inline uint2 exact_codes_8(const float (&o)[8], double s_rcp)
+{
+    float q[8];
+#pragma unroll
+    for(int i = 0; i < 8; i++)
+        q[i] = div_by_row_scale(o[i], s_rcp);
+    if constexpr(FP8)
+    {
+#pragma unroll
+        for(int i = 0; i < 8; i++)
+            q[i] = fminf(fmaxf(q[i], -448.f), 448.f);
+        return make_uint2(fp8x4(q[0], q[1], q[2], q[3]), fp8x4(q[4], q[5], q[6], q[7]));
+    }
+    else
+    {
+        int c[8];
+#pragma unroll
+        for(int i = 0; i < 8; i++)
+            c[i] = NEAREST ? static_cast<int>(__builtin_rintf(q[i])) : static_cast<int>(static_cast<signed char>(quantise_one<false>(q[i])));
+        return make_uint2(pack_low_bytes(c[0], c[1], c[2], c[3]), pack_low_bytes(c[4], c[5], c[6], c[7]));
+    }
+}
+
+// The same codes.  A code is right where both ends of the bracket give it, which fails for one quotient in some 2^14 (those
+// within 2^-20 of a code's boundary): one piece of eight in 2000 is done again with the fp64 product that rounds like the
 // division.  That product, two conversions at a quarter of the fp32 rate, was most of these kernels' instructions.
 // A NaN becomes -128 and -127 (e4m3: -448 and NaN) at the two ends, so it goes to the exact form too.
 // 3001 x 8 smooth-quantised int8 rows of 4096: 62 -> 50 us (with half the registers, see the launch); 24008 rows of 1536
@@ -65,10 +96,6 @@ template <bool FP8, bool NEAREST = false>
 __device__ inline uint2 quantise_8(const float (&o)[8], const RowScale<FP8>& row)
 {
     uint2 lo, hi;
-    auto fp8x4 = [](float a, float b, float c, float d) {
-        const int w = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false);
-        return static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(c, d, w, true));
-    };
     if constexpr(FP8)
     {
         float l[8], h[8];
@@ -96,28 +123,7 @@ __device__ inline uint2 quantise_8(const float (&o)[8], const RowScale<FP8>& row
         hi = make_uint2(pack_low_bytes(h[0], h[1], h[2], h[3]), pack_low_bytes(h[4], h[5], h[6], h[7]));
     }
     if(((lo.x ^ hi.x) | (lo.y ^ hi.y)) != 0)
-    {
-        const double s_rcp = row_reciprocal(row.scale());
-        float q[8];
-#pragma unroll
-        for(int i = 0; i < 8; i++)
-            q[i] = div_by_row_scale(o[i], s_rcp);
-        if constexpr(FP8)
-        {
-#pragma unroll
-            for(int i = 0; i < 8; i++)
-                q[i] = fminf(fmaxf(q[i], -448.f), 448.f);
-            lo = make_uint2(fp8x4(q[0], q[1], q[2], q[3]), fp8x4(q[4], q[5], q[6], q[7]));
-        }
-        else
-        {
-            int c[8];
-#pragma unroll
-            for(int i = 0; i < 8; i++)
-                c[i] = NEAREST ? static_cast<int>(__builtin_rintf(q[i])) : static_cast<int>(static_cast<signed char>(quantise_one<false>(q[i])));
-            lo = make_uint2(pack_low_bytes(c[0], c[1], c[2], c[3]), pack_low_bytes(c[4], c[5], c[6], c[7]));
-        }
-    }
+        lo = exact_codes_8<FP8, NEAREST>(o, row_reciprocal(row.scale()));
     return lo;
 }
 
@@ -507,7 +513,9 @@ __global__ __launch_bounds__(256) void moe_smoothquant_grouped_kernel(const uint
 // alone.
 // FP8 (the fp8 path with fused_quant): e4m3 codes instead, scale = amax / 448, rounded to nearest even by the
 // conversion instruction.
-template <bool SMOOTH, bool FP8>
+// LONG: rows of more pieces than a lane keeps take the exact quotients.  The pieces a lane fetches again come one at a time,
+// and with the bracket's branch in that loop 28 rows of 8320 took 13.2 us instead of 11.4, 8612 rows of 2496 18.8 instead of 17.9.
+template <bool SMOOTH, bool FP8, bool LONG>
 __global__ __launch_bounds__(256) void moe_requant_y_kernel(const uint16_t* __restrict__ y, int inter,
                                                              const float* __restrict__ smooth,
                                                              const int* __restrict__ sorted_ids,
@@ -571,7 +579,13 @@ __global__ __launch_bounds__(256) void moe_requant_y_kernel(const uint16_t* __re
     if(lane == 0)
         yscale[row] = amax / (FP8 ? 448.0f : 127.0f); // (a row of zeros: scale 0, codes 0)
     const RowScale<FP8> rs(amax);
-    auto store = [&](int c, const float (&o)[8]) { *reinterpret_cast<uint2*>(dst(c)) = quantise_8<FP8, !FP8>(o, rs); };
+    [[maybe_unused]] const double s_rcp = LONG ? row_reciprocal(rs.scale()) : 0.0;
+    auto store = [&](int c, const float (&o)[8]) {
+        if constexpr(LONG)
+            *reinterpret_cast<uint2*>(dst(c)) = exact_codes_8<FP8, !FP8>(o, s_rcp);
+        else
+            *reinterpret_cast<uint2*>(dst(c)) = quantise_8<FP8, !FP8>(o, rs);
+    };
 #pragma unroll
     for(int j = 0; j < kQuantCache; j++)
         if(lane + 64 * j < chunks)
@@ -727,10 +741,15 @@ int launch_requant_y(const void* y, int32_t inter, const float* smooth, const in
         hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, static_cast<const uint16_t*>(y), inter, smooth, sorted_ids,
                            sorted_expert_ids, total, unit, tokens, topk, segs, static_cast<unsigned char*>(yq), yscale);
     };
+    const bool is_long = inter > 8 * 64 * kQuantCache;
+    auto of_type       = [&](auto smooth_tag, auto fp8_tag) {
+        constexpr bool S = decltype(smooth_tag)::value, F = decltype(fp8_tag)::value;
+        is_long ? launch(moe_requant_y_kernel<S, F, true>) : launch(moe_requant_y_kernel<S, F, false>);
+    };
     if(fp8)
-        smooth != nullptr ? launch(moe_requant_y_kernel<true, true>) : launch(moe_requant_y_kernel<false, true>);
+        smooth != nullptr ? of_type(std::true_type{}, std::true_type{}) : of_type(std::false_type{}, std::true_type{});
     else
-        smooth != nullptr ? launch(moe_requant_y_kernel<true, false>) : launch(moe_requant_y_kernel<false, false>);
+        smooth != nullptr ? of_type(std::true_type{}, std::false_type{}) : of_type(std::false_type{}, std::false_type{});
     MI355_HIP_TRY(hipGetLastError());
     return MI355_MOE_OK;
 }
