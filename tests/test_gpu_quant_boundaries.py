@@ -70,3 +70,14 @@ def test_smoothquant_codes_at_boundaries(hidden, experts, kind):
     rq, rs = oracle.smoothquant(np.ones((tokens, hidden), np.float32), sm, ids, oracle.DT_I8 if kind == "int8" else oracle.DT_E4M3)
     assert np.array_equal(ys.cpu().numpy(), rs)
     assert np.array_equal(qy.view(torch.uint8).cpu().numpy(), rq.view(np.uint8))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fq", [1, 2])
+@pytest.mark.parametrize("dtype", ["int8", "fp8"])
+@pytest.mark.parametrize("inter", [2048, 2176, 4224])
+def test_requantised_rows_around_a_lanes_registers(inter, dtype, fq):
+    # up to 2048 columns a lane keeps its pieces and codes come from the bracket; longer rows take the exact quotients
+    from therock_amd import inputs as mi
+    from tests.test_gpu_fused_quant import run
+    run(mi.MoeConfig("fq_long_rows", 48, 256, inter, 4, 2, dtype, "softmax_renorm"), fq)
