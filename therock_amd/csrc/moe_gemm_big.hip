@@ -312,13 +312,12 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
     // none.  Tiles are numbered over the experts, as a narrow layer has few columns.)  Gate+up
     // GEMM at 83 rows per expert: bf16 8 x 4096 x 16384 462 -> 350 us (4.7 -> 6.1 TB/s), fp8 / int8 16 x 4096 x 8192
     // 255 -> 190 / 262 -> 200 us; at other pitches up to 4 % (int8, 64 x 7168 x 2048 at 84 rows: pass 713 -> 684 us).
-    // Not rotated: row tiles that share weights, which fetch each weight slice together and each token slice for eight
-    // column tiles at a time (4096 tokens x 2 of 8 bf16 experts 1598 -> 1720 us); down GEMMs without the bad pitch, whose
-    // shorter K gains up to 2 % at 145 rows and loses as much elsewhere (263 rows of 15 fp16 experts 3840 x 11008 3 %, 1000
-    // tokens x 8 of 256 fp8 experts 7168 x 2048 0.8 %).
+    // Which layers do: big_k_spread, by sizes alone, so that the order of a token's sums does not depend on how many rows other
+    // tokens bring its expert.  (int8 sums are exact in any order: there experts of several row tiles, which fetch each
+    // weight slice together and each token slice for eight column tiles at a time, keep one place to begin at.)
     constexpr uint32_t kGolden = 0x9e3779b9u; // its fractional part in units of 2^-32
     const int n_win   = n_wunits >> 1; // 128-byte windows of weight K
-    const bool rotate = !odd_k && tile.expert_tiles == 1 && (GEMM0 || (p.w_row_bytes & 4095) == 0);
+    const bool rotate = !odd_k && p.k_spread != 0 && (MODE != kI8 || tile.expert_tiles == 1);
     const uint32_t at = (uint32_t)expert * (uint32_t)p.n_ntiles + (uint32_t)tile.nt;
     const int rot     = rotate ? (int)__umulhi(at * kGolden, (uint32_t)n_win) : 0; // < n_win
     // the wave's stream (weights or tokens): address of the window it is in, moved on by its issue functions

@@ -90,6 +90,7 @@ struct GemmParams
     int k_cols;
     int k_slice;
     int topk; // slots per token
+    int k_spread; // large tiles: column tiles begin K at different places (see big_k_spread)
 };
 
 // row of the gate+up GEMM's activations (and index of its per-row scale) a sorted id refers to (here and below: an id
