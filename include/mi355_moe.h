@@ -272,7 +272,7 @@ int32_t mi355_fused_moe_k_slices(const mi355_fused_moe_traits* traits, int32_t t
                                  int32_t hidden_size, int32_t intermediate_size, size_t ws_bytes);
 
 /* sorted rows one GEMM workgroup owns at this problem size: 32, 64 or 128 (moe_gemm_kernel) or 320
- * (moe_gemm_big_kernel); 0 for unsupported traits.  The counterpart of Block_M0 of the instance
+ * (moe_gemm_big_kernel; not for token rows so far apart that they span 4 GiB or more: 128 at most); 0 for unsupported traits.  The counterpart of Block_M0 of the instance
  * ck_tile's dispatcher selects (fused_moegemm_shape.hpp:43-64); here it is chosen per problem size. */
 int32_t mi355_fused_moe_tile_rows(const mi355_fused_moe_traits* traits, int32_t tokens, int32_t num_experts,
                                   int32_t topk, int32_t hidden_size, int32_t intermediate_size);

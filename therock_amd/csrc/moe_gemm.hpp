@@ -9,7 +9,7 @@ namespace mi355 {
 struct WorkspaceLayout
 {
     size_t sort_off;   // moe_sorting segment counters
-    size_t map_off;    // int32 [4 + 8 * max_tiles]: live tile count, then one entry per M tile
+    size_t map_off;    // int32 [4 + 8 * max_tiles, more for far rows]: live tile count, then one entry per M tile
     size_t inv_off;    // int32 [tokens * topk]: sorted position of the (token, slot) entry, -1 when dropped
     size_t y_off;      // intermediate activations Y [max_pad, inter] (bf16 or e4m3)
     size_t ys_off;     // e8m0 block scales of Y [inter / 32][ys_kb_stride] (fp8 path only)
@@ -27,8 +27,10 @@ struct WorkspaceLayout
 
 int check_traits(const mi355_fused_moe_traits& t);
 
+// far_rows: of a call whose token rows do not all lie within 4 GiB (it runs without the kernels that address them with
+// 32-bit offsets, on more and smaller tiles, and its down GEMM is not cut; least is the same)
 WorkspaceLayout workspace_layout(const mi355_fused_moe_traits& t, int32_t tokens, int32_t experts,
-                                 int32_t topk, int32_t hidden, int32_t inter);
+                                 int32_t topk, int32_t hidden, int32_t inter, bool far_rows = false);
 
 // the second tile height the sort may choose on the device for this problem (0: none)
 int gemm_alt_tile_rows(const mi355_fused_moe_traits& t, int32_t tokens, int32_t experts, int32_t topk, int32_t hidden,
