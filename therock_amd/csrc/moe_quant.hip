@@ -88,10 +88,12 @@ __device__ inline uint2 exact_codes_8(const float (&o)[8], double s_rcp)
 
 // The same codes.  A code is right where both ends of the bracket give it, which fails for one quotient in some 2^14 (those
 // within 2^-20 of a code's boundary): one piece of eight in 2000 is done again with the fp64 product that rounds like the
-// division.  That product, two conversions at a quarter of the fp32 rate, was most of these kernels' instructions.
+// division, and, with codes rounded toward zero, the piece that holds the row's maximum, whose quotient is 127 itself.
+// That product, two conversions at a quarter of the fp32 rate, was most of these kernels' instructions.
 // A NaN becomes -128 and -127 (e4m3: -448 and NaN) at the two ends, so it goes to the exact form too.
-// 3001 x 8 smooth-quantised int8 rows of 4096: 62 -> 50 us (with half the registers, see the launch); 24008 rows of 1536
-// re-quantised between the GEMMs 30 -> 25 us.
+// Used where a thread has one or two pieces (a wave's lane up to four in the re-quantisation), which are then in registers
+// for the exact form as well; with more, the branch costs more than it saves (see kBracketCols).  24008 rows of 1536
+// re-quantised between the GEMMs: 30 -> 25 us.
 template <bool FP8, bool NEAREST = false>
 __device__ inline uint2 quantise_8(const float (&o)[8], const RowScale<FP8>& row)
 {
@@ -141,7 +143,12 @@ __device__ inline float block_max_256(float v, float* s_red)
 // (cols % 8 == 0, 16-byte aligned rows); the first kCache pieces of every thread stay in registers between the
 // two passes, so rows of up to 8192 columns are read once.  Returns the row's amax to every thread.
 constexpr int kQuantCache = 4;
-template <bool FP8, bool SMOOTH, bool VEC>
+// Rows of up to two pieces a thread take their codes from the bracket, longer ones the exact quotients.  Exact -> bracket, us:
+// 32768 rows of 1024 / 4096, int8 37.0 -> 32.6 / 77.1 -> 67.8, e4m3 35.2 -> 26.6 / 75.8 -> 67.4; 8192 rows of 7168, int8 28.1 -> 29.3, e4m3
+// 27.5 -> 28.8; 3001 x 8 smooth-quantised rows of 7168 grouped by expert, int8 80 -> 92, e4m3 72 -> 83 (fewer registers, too: four
+// waves per SIMD instead of three).
+constexpr int kBracketCols = 2 * 256 * 8;
+template <bool FP8, bool SMOOTH, bool VEC, bool BRACKET>
 __device__ inline float quantise_row(const uint16_t* __restrict__ xr, const float* __restrict__ sr, int cols,
                                      unsigned char* __restrict__ qr, float* s_red, bool unit_scale_when_zero, float* scale_out)
 {
@@ -194,7 +201,10 @@ __device__ inline float quantise_row(const uint16_t* __restrict__ xr, const floa
         if(threadIdx.x == 0)
             *scale_out = (amax > 0.f || !unit_scale_when_zero) ? amax / qmx : 1.0f;
         const RowScale<FP8> row(amax);
-        auto store = [&](int c, const float (&o)[8]) { *reinterpret_cast<uint2*>(qr + c * 8) = quantise_8<FP8>(o, row); };
+        const double s_rcp = row_reciprocal(row.scale());
+        auto store = [&](int c, const float (&o)[8]) {
+            *reinterpret_cast<uint2*>(qr + c * 8) = BRACKET ? quantise_8<FP8>(o, row) : exact_codes_8<FP8, false>(o, s_rcp);
+        };
 #pragma unroll
         for(int j = 0; j < kQuantCache; j++)
         {
@@ -230,14 +240,14 @@ __device__ inline float quantise_row(const uint16_t* __restrict__ xr, const floa
 }
 
 // per-row dynamic quantisation bf16 -> e4m3 / int8
-template <bool FP8, bool VEC>
+template <bool FP8, bool VEC, bool BRACKET>
 __global__ __launch_bounds__(256) void rowwise_quant_kernel(const uint16_t* __restrict__ x, int cols,
                                                              int64_t stride_x, unsigned char* __restrict__ q,
                                                              float* __restrict__ scale)
 {
     __shared__ float s_red[4];
     const int64_t row = blockIdx.x;
-    quantise_row<FP8, false, VEC>(x + row * stride_x, nullptr, cols, q + row * cols, s_red, true, scale + row);
+    quantise_row<FP8, false, VEC, BRACKET>(x + row * stride_x, nullptr, cols, q + row * cols, s_red, true, scale + row);
 }
 
 // MoE smooth-quant: row (slot k, token t) = x[t, :] * smscale[expert(t, k), :], per-row dynamic quantisation.
@@ -255,7 +265,7 @@ __global__ __launch_bounds__(256) void moe_smoothquant_kernel(const uint16_t* __
     int e       = topk_ids[(int64_t)t * topk + k];
     e           = min(max(e, 0), experts - 1);
     const int64_t r = (int64_t)k * tokens + t;
-    quantise_row<FP8, true, false>(x + (int64_t)t * x_stride, smscale + (int64_t)e * hidden, hidden, qy + r * y_stride, s_red,
+    quantise_row<FP8, true, false, false>(x + (int64_t)t * x_stride, smscale + (int64_t)e * hidden, hidden, qy + r * y_stride, s_red,
                                    false, yscale + r);
 }
 
@@ -350,10 +360,15 @@ __global__ __launch_bounds__(256) void moe_smoothquant_vec_kernel(const uint16_t
             yscale[r] = amax / qmx; // (a row of zeros: scale 0, codes 0)
         unsigned char* qr = qy + r * y_stride;
         const RowScale<FP8> row(amax);
+        [[maybe_unused]] const double s_rcp = row_reciprocal(row.scale());
         // (streaming stores: the quantised rows are written once and should not push the experts' scales out of L2)
         auto store = [&](int c, const float (&o)[8]) {
             typedef __attribute__((ext_vector_type(2))) unsigned u32x2_t;
-            const uint2 q = quantise_8<FP8>(o, row);
+            uint2 q;
+            if constexpr(PIECES == kQuantCache)
+                q = exact_codes_8<FP8, false>(o, s_rcp);
+            else
+                q = quantise_8<FP8>(o, row);
             __builtin_nontemporal_store(u32x2_t{q.x, q.y}, reinterpret_cast<u32x2_t*>(qr + c * 8));
         };
 #pragma unroll
@@ -483,9 +498,14 @@ __global__ __launch_bounds__(256) void moe_smoothquant_grouped_kernel(const uint
             yscale[r] = amax / qmx; // (a row of zeros: scale 0, codes 0)
         unsigned char* qr   = qy + r * y_stride;
         const RowScale<FP8> row(amax);
+        [[maybe_unused]] const double s_rcp = row_reciprocal(row.scale());
         auto store = [&](int c, const float (&o)[8]) {
             typedef __attribute__((ext_vector_type(2))) unsigned u32x2_t;
-            const uint2 q = quantise_8<FP8>(o, row);
+            uint2 q;
+            if constexpr(PIECES == kQuantCache)
+                q = exact_codes_8<FP8, false>(o, s_rcp);
+            else
+                q = quantise_8<FP8>(o, row);
             __builtin_nontemporal_store(u32x2_t{q.x, q.y}, reinterpret_cast<u32x2_t*>(qr + c * 8));
         };
 #pragma unroll
@@ -672,8 +692,8 @@ int launch_moe_smoothquant(const mi355_moe_smoothquant_args& a, int32_t q_dtype,
     const bool vec = a.hidden_size % 8 == 0 && a.x_stride % 8 == 0 && a.y_stride % 8 == 0 &&
                      reinterpret_cast<uintptr_t>(a.p_x) % 16 == 0 && reinterpret_cast<uintptr_t>(a.p_smscale) % 16 == 0 &&
                      reinterpret_cast<uintptr_t>(a.p_qy) % 8 == 0;
-    auto launch = [&](auto kernel, dim3 grid) {
-        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, static_cast<const uint16_t*>(a.p_x),
+    auto launch = [&](auto kernel, dim3 grid, unsigned lds = 0) {
+        hipLaunchKernelGGL(kernel, grid, dim3(256), lds, stream, static_cast<const uint16_t*>(a.p_x),
                            static_cast<const float*>(a.p_smscale), static_cast<const int*>(a.p_topk_ids), a.tokens,
                            a.hidden_size, a.experts, a.topk, (int64_t)a.x_stride, (int64_t)a.y_stride,
                            static_cast<unsigned char*>(a.p_qy), static_cast<float*>(a.p_yscale));
@@ -683,19 +703,23 @@ int launch_moe_smoothquant(const mi355_moe_smoothquant_args& a, int32_t q_dtype,
     const int64_t ranges8 = ceil_div<int64_t>(ceil_div(a.tokens, kSqRange), 8);
     const bool grouped    = vec && (int64_t)a.experts * a.hidden_size * (int64_t)sizeof(float) > (3ll << 20) &&
                          kSqRange * a.topk <= kSqMaxList && ranges8 * a.experts * 8 < (1ll << 31);
+    // Columns past a thread's registers are fetched again, 6 bytes each, from L2 while the workgroups of an XCD (32 compute
+    // units x 4) need no more than it holds; with longer rows 12 KB of LDS more leave three per compute unit: 2048 x 8 int8
+    // rows of 13312 129 us with four, 133 with three; of 14336 158, 147; of 16384 242, 210.
+    const unsigned grouped_lds = 32 * 4 * 6 * (int64_t)(a.hidden_size - 8 * 256 * kQuantCache) > (4 << 20) ? 12 << 10 : 0;
     auto of_type = [&](auto fp8_tag, auto pieces_tag) {
         constexpr bool FP8   = decltype(fp8_tag)::value;
         constexpr int PIECES = decltype(pieces_tag)::value;
         if(grouped)
-            launch(moe_smoothquant_grouped_kernel<FP8, PIECES>, dim3((unsigned)(ranges8 * a.experts * 8)));
+            launch(moe_smoothquant_grouped_kernel<FP8, PIECES>, dim3((unsigned)(ranges8 * a.experts * 8)), grouped_lds);
         else if(vec)
             launch(moe_smoothquant_vec_kernel<FP8, PIECES>, per_token);
         else
             launch(moe_smoothquant_kernel<FP8>, per_row);
     };
-    // rows of up to 4096 columns need half the registers: twice the waves per compute unit
+    // rows of up to 4096 columns need half the registers: six waves per SIMD instead of three (grouped: four, by its list in LDS)
     auto pieces = [&](auto fp8_tag) {
-        a.hidden_size <= 2 * 256 * 8 ? of_type(fp8_tag, std::integral_constant<int, 2>{})
+        a.hidden_size <= kBracketCols ? of_type(fp8_tag, std::integral_constant<int, 2>{})
                                      : of_type(fp8_tag, std::integral_constant<int, kQuantCache>{});
     };
     q_dtype == MI355_MOE_FP8 ? pieces(std::true_type{}) : pieces(std::false_type{});
@@ -721,10 +745,14 @@ int launch_rowwise_quant(const void* x, int64_t rows, int32_t cols, int64_t stri
         hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3(256), 0, stream, static_cast<const uint16_t*>(x), cols,
                            stride_x, static_cast<unsigned char*>(q), static_cast<float*>(scale));
     };
-    if(q_dtype == MI355_MOE_FP8)
-        vec ? launch(rowwise_quant_kernel<true, true>) : launch(rowwise_quant_kernel<true, false>);
-    else
-        vec ? launch(rowwise_quant_kernel<false, true>) : launch(rowwise_quant_kernel<false, false>);
+    auto of_type = [&](auto fp8_tag) {
+        constexpr bool FP8 = decltype(fp8_tag)::value;
+        if(!vec)
+            launch(rowwise_quant_kernel<FP8, false, false>);
+        else
+            cols <= kBracketCols ? launch(rowwise_quant_kernel<FP8, true, true>) : launch(rowwise_quant_kernel<FP8, true, false>);
+    };
+    q_dtype == MI355_MOE_FP8 ? of_type(std::true_type{}) : of_type(std::false_type{});
     MI355_HIP_TRY(hipGetLastError());
     return MI355_MOE_OK;
 }
