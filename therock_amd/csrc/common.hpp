@@ -141,11 +141,12 @@ __host__ __device__ inline void blocked_tile_of(int rel, int rows, int cols, int
     }
 }
 
-// Transfer schedule of the large-tile kernel's K loop where operands are not pipelined (the fp8 and the int8 x bf16 down
-// GEMM).  A weight-role wave has issued units 0 .. 3 before the loop and one more in every step (w8: in every even step,
-// as a unit then lasts four steps), as far as there are any; the barrier of step k has to guarantee the unit pair it reads.
-// How many of the last issued units may be in flight at that barrier: 2 in even and 3 in odd steps while units are still
-// being issued; at the end the last issued units are the ones that are needed, and all have to land.
+// Transfer schedule of the large-tile kernel's K loop in the fp8 down GEMM, whose operands are not pipelined, and with int8
+// weights against bf16 tokens (w8), pipelined, whose weight units last four steps.  A weight-role wave has issued units 0 .. 3
+// before the loop and one more in every step (w8: in every even step), as far as there are any.  The barrier of step k has to
+// guarantee the unit pair that step k reads (w8: the pair of step k + 1, whose operands step k fetches).  How many of the last
+// issued units may be in flight at the barrier that guarantees step k: 2 in even and 3 in odd steps (w8: 2) while units are
+// still being issued; at the end the last issued units are the ones that are needed, and all have to land.
 __host__ __device__ constexpr int big_unit_of_step(int k, bool w8) { return w8 ? (k >> 1) + 4 : k + 4; } // issued in step k
 __host__ __device__ constexpr int big_pair_of_step(int k, bool w8) { return w8 ? (k >> 2) << 1 : k & ~1; } // first unit it reads
 __host__ __device__ constexpr bool big_units_may_fly(int k, int kt_count, bool w8)

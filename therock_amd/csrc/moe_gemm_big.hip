@@ -288,8 +288,8 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
     const int x_step      = (!GEMM0 && p.y_slab > 0) ? 1024 : kStepKB; // bytes between token steps
 
     const uint32_t lds_base = lds_offset(lds);
-    // compute steps (even; a multiple of four with int8 weights): this workgroup's slice of K, whose first bytes the
-    // base addresses point at (a slice is a multiple of 512 weight bytes)
+    // compute steps of this workgroup's slice of K, whose first bytes the base addresses point at (a slice is a multiple of
+    // 512 weight bytes): even, but for 8-bit rows of an odd number of 64-byte steps (kOddK, kOddW)
     int kt_count = p.k_bytes_x / kStepKB;
     const unsigned char* ys_base = p.y_scale;
     if(!GEMM0 && p.k_cols > 0)
@@ -393,8 +393,6 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
             stream += x_step;
     };
 
-    // 128-byte token stages: pair m = steps 2 m and 2 m + 1 -> stage m % x_stages(groups); two instructions per 64 rows of the
-    // tile
     // (kOddK) token lanes of the half the last pair does not have fetch the other half from here on
     auto halve_x = [&]() __attribute__((always_inline)) {
         if constexpr(kXPair)
@@ -407,6 +405,8 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
             }
         }
     };
+    // 128-byte token stages: pair m = steps 2 m and 2 m + 1 -> stage m % x_stages(groups); two instructions per 64 rows of the
+    // tile
     auto issue_x_pair = [&](int m, int stage, int groups) __attribute__((always_inline)) {
         if constexpr(kXPair)
         {
@@ -493,7 +493,6 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
             // operand registers of the step about to run
             Frag wf[kSteps][2];
             Frag xf[kSteps][NF];
-            uint32_t xs[kSteps][NF];
             // first step of the last window where only its second half is new (kOddW)
             [[maybe_unused]] const int half_from = kOddW && odd_k ? kt_count - (kW8 ? 2 : 1) : INT32_MAX;
             // weight fragment b of sub-step s of step kk (parity P), token fragment i of sub-step s of step kk
@@ -524,9 +523,8 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                     f.hi = *reinterpret_cast<const uint4*>(wp + cw_hi);
                 return f;
             };
-            auto load_xf = [&](int kk, int s, int i, uint32_t& scale) __attribute__((always_inline)) {
+            auto load_xf = [&](int kk, int s, int i) __attribute__((always_inline)) {
                 Frag f;
-                scale = 127;
                 if constexpr(kXPair)
                 {
                     const unsigned char* xp = lds + kXOffsetPair + ((uint32_t)(kk >> 1) % kXS) * pair_stage_bytes(kGroups) + (wt * 32 + r32 + i * 64) * (2 * kStepKB);
@@ -545,8 +543,6 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                     f.lo                    = *reinterpret_cast<const uint4*>(xp + cx_lo);
                     if constexpr(kOpB == 32)
                         f.hi = *reinterpret_cast<const uint4*>(xp + cx_hi);
-                    if constexpr(kMx)
-                        scale = lds[ys_offset(kGroups) + ((uint32_t)kk % kXS) * kYsStageBytes + kg * kYsRows + wt * 32 + r32 + i * 64];
                 }
                 return f;
             };
@@ -566,7 +562,6 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");
             };
-            constexpr int kXI = XG + (kMx ? 1 : 0); // token-role instructions of one step
             // step 0's data: weight units 0 and 1 (2, 3, 4 may be pending; with 128-byte token stages, or where a unit lasts
             // four steps, 2 and 3) and the first token stage (the others may be pending)
             const bool six = kt_count >= 6;
@@ -574,7 +569,7 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                 sync(six, kt_count >= 2 * kXS, std::integral_constant<int, 8>{}, std::integral_constant<int, 2 * XG * (kXS - 1)>{});
             else
                 sync(kW8 ? n_wunits >= 4 : six, kt_count >= kXS, std::integral_constant<int, (kW8 ? 8 : 12)>{},
-                     std::integral_constant<int, kXI * (kXS - 1)>{});
+                     std::integral_constant<int, XG * (kXS - 1)>{});
             static_for<kSteps>([&](auto s_tag) __attribute__((always_inline)) {
                 constexpr int s = decltype(s_tag)::value;
                 wf[s][0]        = load_wf(0, H0{}, s, 0);
@@ -586,7 +581,7 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                 }
                 static_for<NB>([&](auto i_tag) __attribute__((always_inline)) {
                     constexpr int i = decltype(i_tag)::value;
-                    xf[s][i]        = load_xf(0, s, i, xs[s][i]);
+                    xf[s][i]        = load_xf(0, s, i);
                 });
             });
             auto step = [&](int k, auto par_tag) __attribute__((always_inline)) {
@@ -614,10 +609,10 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                 }
                 else if constexpr(kW8)
                     sync(big_units_may_fly(k + 1, kt_count, kW8), k + kXS <= kt_count, std::integral_constant<int, 8>{},
-                         std::integral_constant<int, kXI * (kXS - 2)>{});
+                         std::integral_constant<int, XG * (kXS - 2)>{});
                 else
                     sync(counted, k + kXS <= kt_count, std::integral_constant<int, (PAR ? 8 : 12)>{},
-                         std::integral_constant<int, kXI * (kXS - 2)>{});
+                         std::integral_constant<int, XG * (kXS - 2)>{});
                 // the transfers of the step go out behind the MFMAs of the second token block (measured: 1 to 2 %
                 // faster than right after the barrier, where all eight waves queue up at the address unit while the
                 // MFMA pipe has nothing to do; one instruction behind every block is 5 % slower)
@@ -663,12 +658,12 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                         }
                         else
                         {
-                            acc[i][0] = mfma<MODE>(wf[s][0], xf[s][i], xs[s][i], acc[i][0]);
-                            acc[i][1] = mfma<MODE>(wf[s][1], xf[s][i], xs[s][i], acc[i][1]);
+                            acc[i][0] = mfma<MODE>(wf[s][0], xf[s][i], 0u, acc[i][0]);
+                            acc[i][1] = mfma<MODE>(wf[s][1], xf[s][i], 0u, acc[i][1]);
                         }
                         // the fragment's registers are free: fetch its successor (stale data after the last step)
                         __builtin_amdgcn_sched_barrier(0);
-                        xf[s][i] = load_xf(k + 1, s, i, xs[s][i]);
+                        xf[s][i] = load_xf(k + 1, s, i);
                         if constexpr(NB > kIssueAfter && s == 0 && i == kIssueAfter)
                             issue_next();
                         __builtin_amdgcn_sched_barrier(0);
@@ -738,106 +733,72 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                 step(k, H0{});
                 step(k + 1, H1{});
             }
-            return;
         }
-        // one compute step; PAR = k & 1
-        auto step = [&](int k, auto par_tag) __attribute__((always_inline)) {
-            constexpr int PAR = decltype(par_tag)::value;
-            // Needed now: token step k and the weight units of pair k >> 1.  Issued after them and allowed to stay pending:
-            // kXS - 2 token steps; two weight units (even k) or three (odd k), until the last pair is the one needed.
-            if(w_role ? big_units_may_fly(k, kt_count, false) : k + kXS - 2 < kt_count)
-            {
-                if(w_role)
-                    wait_vmcnt<PAR ? 12 : 8>();
+        else
+        {
+            // fp8 down GEMM.  One compute step; PAR = k & 1
+            auto step = [&](int k, auto par_tag) __attribute__((always_inline)) {
+                constexpr int PAR = decltype(par_tag)::value;
+                // Needed now: token step k and the weight units of pair k >> 1.  Issued after them and allowed to stay pending:
+                // kXS - 2 token steps; two weight units (even k) or three (odd k), until the last pair is the one needed.
+                if(w_role ? big_units_may_fly(k, kt_count, false) : k + kXS - 2 < kt_count)
+                {
+                    if(w_role)
+                        wait_vmcnt<PAR ? 12 : 8>();
+                    else
+                        wait_vmcnt<(XG + 1) * (kXS - 2)>(); // token-role instructions of the steps after it
+                }
                 else
-                    wait_vmcnt<(XG + 1) * (kXS - 2)>(); // token-role instructions of the steps after it
-            }
-            else
-                wait_vmcnt<0>();
-            // data of step k visible to all waves; everyone is done reading step k-1 (a bare barrier:
-            // the DMA completion was awaited above and LDS reads are consumed by MFMAs before a
-            // wave gets here)
-            asm volatile("" ::: "memory");
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-            auto issue_next = [&]() __attribute__((always_inline)) {
+                    wait_vmcnt<0>();
+                // data of step k visible to all waves; everyone is done reading step k-1 (a bare barrier:
+                // the DMA completion was awaited above and LDS reads are consumed by MFMAs before a
+                // wave gets here)
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                // The transfers of the step, whose buffers are free from the barrier on (behind the first MFMAs, as in the
+                // pipelined loop, needs a scheduling fence for which there is no register to spare)
                 if(w_role)
                     issue_w(big_unit_of_step(k, false), par_tag, nt_tag);
                 else
                     issue_x(k + kXS - 1, (uint32_t)(k + kXS - 1) % kXS, XG);
-            };
-            // Where in the step the transfers go out: right here, or after the MFMAs of token block kIssueAfter.  The
-            // buffers they write are free from the barrier on either way, but issued here the handful of scalar and
-            // DMA instructions sits between the barrier and the first operand fetch, on every wave's critical path;
-            // issued behind the first MFMAs it runs while the matrix pipe is busy (measured -2 % fp8, -4 % bf16 on the
-            // gate+up GEMM).  After all MFMAs is too late (the transfers then start up to a step later), and the fp8
-            // down GEMM has no register to spare for the scheduling fence this needs.
-            constexpr int kIssueAfter = kMx ? -1 : 1;
-            if constexpr(kIssueAfter < 0 || NB <= kIssueAfter)
-                issue_next();
 
-            // first unit of the pair that holds this step's weight bytes
-            const int pair0          = big_pair_of_step(k, false);
-            const unsigned char* wst = lds + ((uint32_t)(pair0 + w_h) % kWSlots) * kWUnitBytes + w_off;
-            const unsigned char* xst = lds + x_off + ((uint32_t)k % kXS) * step_stage_bytes(kGroups);
-            [[maybe_unused]] const unsigned char* ysl =
-                lds + ys_offset(kGroups) + ((uint32_t)k % kXS) * kYsStageBytes + kg * kYsRows + wt * 32 + r32;
-            constexpr int kh = PAR * 4; // first chunk of this step inside the 128-byte weight row
-#pragma unroll
-            for(int s = 0; s < kSteps; s++)
-            {
+                // first unit of the pair that holds this step's weight bytes
+                const int pair0          = big_pair_of_step(k, false);
+                const unsigned char* wst = lds + ((uint32_t)(pair0 + w_h) % kWSlots) * kWUnitBytes + w_off;
+                const unsigned char* xst = lds + x_off + ((uint32_t)k % kXS) * step_stage_bytes(kGroups);
+                const unsigned char* ysl = lds + ys_offset(kGroups) + ((uint32_t)k % kXS) * kYsStageBytes + kg * kYsRows + wt * 32 + r32;
+                constexpr int kh         = PAR * 4; // first chunk of this step inside the 128-byte weight row
                 Frag wf[2];
                 Frag xf[NF];
                 uint32_t xs[NF];
-                const int cx_lo = kOpB == 16 ? ((2 * s + kg) ^ sw_x) * 16 : (kg ^ sw_x) * 16;
-                const int cx_hi = ((2 + kg) ^ sw_x) * 16;
-                const int cw_lo = kOpB == 16 ? ((kh + 2 * s + kg) ^ sw_wr) * kWChunkB : ((kh + kg) ^ sw_wr) * kWChunkB;
-                const int cw_hi = ((kh + 2 + kg) ^ sw_wr) * kWChunkB;
 #pragma unroll
                 for(int b = 0; b < 2; b++)
                 {
                     const unsigned char* wp = wst + b * 32 * (2 * kStepKB);
-                    wf[b].lo = *reinterpret_cast<const uint4*>(wp + cw_lo);
-                    if constexpr(kOpB == 32)
-                        wf[b].hi = *reinterpret_cast<const uint4*>(wp + cw_hi);
+                    wf[b].lo                = *reinterpret_cast<const uint4*>(wp + ((kh + kg) ^ sw_wr) * kWChunkB);
+                    wf[b].hi                = *reinterpret_cast<const uint4*>(wp + ((kh + 2 + kg) ^ sw_wr) * kWChunkB);
                 }
 #pragma unroll
                 for(int i = 0; i < NB; i++)
                 {
                     const unsigned char* xp = xst + i * 64 * kStepKB;
-                    xf[i].lo                = *reinterpret_cast<const uint4*>(xp + cx_lo);
-                    if constexpr(kOpB == 32)
-                        xf[i].hi = *reinterpret_cast<const uint4*>(xp + cx_hi);
-                    xs[i] = 127;
-                    if constexpr(kMx)
-                        xs[i] = ysl[i * 64];
+                    xf[i].lo                = *reinterpret_cast<const uint4*>(xp + (kg ^ sw_x) * 16);
+                    xf[i].hi                = *reinterpret_cast<const uint4*>(xp + ((2 + kg) ^ sw_x) * 16);
+                    xs[i]                   = ysl[i * 64];
                 }
 #pragma unroll
                 for(int i = 0; i < NB; i++)
                 {
-                    if constexpr(MODE == kFp8 && GEMM0)
-                    {
-                        acc[i][0] = mfma_fp8_unscaled(wf[0], xf[i], acc[i][0]);
-                        acc[i][1] = mfma_fp8_unscaled(wf[1], xf[i], acc[i][1]);
-                    }
-                    else
-                    {
-                        acc[i][0] = mfma<MODE>(wf[0], xf[i], xs[i], acc[i][0]);
-                        acc[i][1] = mfma<MODE>(wf[1], xf[i], xs[i], acc[i][1]);
-                    }
-                    if(kIssueAfter >= 0 && NB > kIssueAfter && s == 0 && i == kIssueAfter)
-                    {
-                        __builtin_amdgcn_sched_barrier(0);
-                        issue_next();
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
+                    acc[i][0] = mfma<MODE>(wf[0], xf[i], xs[i], acc[i][0]);
+                    acc[i][1] = mfma<MODE>(wf[1], xf[i], xs[i], acc[i][1]);
                 }
+            };
+            for(int k = 0; k < kt_count; k += 2)
+            {
+                step(k, H0{});
+                step(k + 1, H1{});
             }
-        };
-        for(int k = 0; k < kt_count; k += 2)
-        {
-            step(k, H0{});
-            step(k + 1, H1{});
         }
     };
     // weight-role waves own blocks 0, 2, .. (ceil(nmb / 2) of them), token-role waves blocks 1, 3, ..
