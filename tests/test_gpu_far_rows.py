@@ -71,6 +71,18 @@ def test_far_rows_are_accepted():
     assert lib.mi355_moe_flatmm(2, C.byref(a), C.byref(ws), None) == _lib.E_HIP, lib.mi355_moe_last_error()
 
 
+def test_library_workspace_holds_what_it_held():
+    """The list's room for far rows does not push a call over the library-owned workspace: layers that fill 96 MiB without it."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("calls without operands: only where nothing can be launched")
+    lib = _lib.load()
+    for dtype, T, E, K, H, I in (("fp8", 48033, 8, 1, 512, 1024), ("bf16", 32465, 8, 1, 512, 1024), ("int8", 15449, 16, 2, 576, 1024)):
+        t = traits(dtype).pod()
+        a = _lib.FusedMoeArgs(num_tokens=T, num_experts=E, topk=K, hidden_size=H, intermediate_size=I)
+        assert lib.mi355_fused_moe_static_ws(C.byref(t), C.byref(a), None) == _lib.E_HIP, lib.mi355_moe_last_error()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", FUSED, ids=lambda c: f"{c[0]}-{c[1]}-{c[2]}")
 def test_fused_moe_of_far_rows(case):

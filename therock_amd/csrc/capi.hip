@@ -2,6 +2,7 @@
 #include "common.hpp"
 #include "moe_gemm.hpp"
 
+#include <algorithm>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -107,7 +108,10 @@ using namespace mi355;
 // hipGetSymbolAddress: the address kernels and copies use is the one that call returns, and every device has its own
 // copy of the array at its own address.
 constexpr size_t kStaticWsBytes = (size_t)96 << 20;
-static __device__ __align__(256) unsigned char scratch[kStaticWsBytes];
+// what the work list of a large-tile layout holds in case the token rows lie far apart comes on top: less than a byte per sorted
+// row, which takes 256 bytes and more of the other buffers
+constexpr size_t kStaticListRoom = (size_t)512 << 10;
+static __device__ __align__(256) unsigned char scratch[kStaticWsBytes + kStaticListRoom];
 
 namespace {
 // device address of `scratch` on the current device, resolved once per device; nullptr (and the error text) on failure
@@ -417,16 +421,17 @@ mi355_fused_moe_static_ws(const mi355_fused_moe_traits* traits, const mi355_fuse
     if(!sizes_in_range(a->num_tokens, a->num_experts, a->topk, a->hidden_size, a->intermediate_size))
         return fail(MI355_MOE_E_INVALID, "fused_moe_static_ws: bad sizes (H=%d I=%d T=%d E=%d K=%d)", a->hidden_size,
                     a->intermediate_size, a->num_tokens, a->num_experts, a->topk);
-    const size_t need = workspace_layout(*traits, a->num_tokens, a->num_experts, a->topk, a->hidden_size,
-                                         a->intermediate_size).least;
-    if(need > kStaticWsBytes)
+    const WorkspaceLayout ws = workspace_layout(*traits, a->num_tokens, a->num_experts, a->topk, a->hidden_size, a->intermediate_size);
+    const size_t need        = ws.least;
+    const size_t held        = kStaticWsBytes + std::min(ws.list_room, kStaticListRoom);
+    if(need > held)
         return fail(MI355_MOE_E_WORKSPACE,
                     "fused_moe_static_ws: this problem needs a workspace of %zu bytes, the library-owned one holds %zu; "
-                    "call mi355_fused_moe with a workspace of your own", need, kStaticWsBytes);
+                    "call mi355_fused_moe with a workspace of your own", need, held);
     void* ws_ptr = static_workspace();
     if(ws_ptr == nullptr)
         return MI355_MOE_E_HIP;
-    return run_fused_moe(traits, a, ws_ptr, kStaticWsBytes, stream);
+    return run_fused_moe(traits, a, ws_ptr, held, stream);
 }
 
 __attribute__((visibility("default"))) size_t

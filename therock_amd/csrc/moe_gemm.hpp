@@ -10,6 +10,7 @@ struct WorkspaceLayout
 {
     size_t sort_off;   // moe_sorting segment counters
     size_t map_off;    // int32 [4 + 8 * max_tiles, more for far rows]: live tile count, then one entry per M tile
+    size_t list_room;  // bytes of it that only calls with far rows use
     size_t inv_off;    // int32 [tokens * topk]: sorted position of the (token, slot) entry, -1 when dropped
     size_t y_off;      // intermediate activations Y [max_pad, inter] (bf16 or e4m3)
     size_t ys_off;     // e8m0 block scales of Y [inter / 32][ys_kb_stride] (fp8 path only)
