@@ -145,8 +145,9 @@ __device__ inline float block_max_256(float v, float* s_red)
 constexpr int kQuantCache = 4;
 // Rows of up to two pieces a thread take their codes from the bracket, longer ones the exact quotients.  Exact -> bracket, us:
 // 32768 rows of 1024 / 4096, int8 37.0 -> 32.6 / 77.1 -> 67.8, e4m3 35.2 -> 26.6 / 75.8 -> 67.4; 8192 rows of 7168, int8 28.1 -> 29.3, e4m3
-// 27.5 -> 28.8; 3001 x 8 smooth-quantised rows of 7168 grouped by expert, int8 80 -> 92, e4m3 72 -> 83 (fewer registers, too: four
-// waves per SIMD instead of three).
+// 27.5 -> 28.8; 3001 x 8 smooth-quantised rows of 7168 grouped by expert, int8 80 -> 92, e4m3 72 -> 83 (with the exact ones
+// fewer registers, too: four waves per SIMD instead of three).  These are of calls repeated on one input; within a pass over more
+// data than the caches hold, the 8192 e4m3 rows of 7168 take 37.7 -> 35.3 (0.07 % of that pass).
 constexpr int kBracketCols = 2 * 256 * 8;
 template <bool FP8, bool SMOOTH, bool VEC, bool BRACKET>
 __device__ inline float quantise_row(const uint16_t* __restrict__ xr, const float* __restrict__ sr, int cols,
