@@ -83,10 +83,11 @@ int launch_permute_weights(const void* src, void* dst, int32_t experts, int32_t 
 int launch_moe_smoothquant(const mi355_moe_smoothquant_args& a, int32_t q_dtype, hipStream_t stream);
 
 // int8 re-quantisation of the sorted rows of Y between the two GEMMs (smooth: [experts, inter] or null;
-// total[0] = rows of the sorted prefix; segs > 0: slab-major output)
+// total[0] = rows of the sorted prefix, at most max_rows; segs > 0: slab-major output; fp8: e4m3 codes, and the ones_bytes,
+// rounded up to 16, of block scales at `ones` set to 2^0)
 int launch_requant_y(const void* y, int32_t inter, const float* smooth, const int* sorted_ids, const int* sorted_expert_ids,
                      const int* total, int32_t unit, int32_t tokens, int32_t topk, int32_t segs, int64_t max_rows, void* yq, float* yscale,
-                     hipStream_t stream, bool fp8 = false);
+                     hipStream_t stream, bool fp8 = false, void* ones = nullptr, int64_t ones_bytes = 0);
 
 int launch_rowwise_quant(const void* x, int64_t rows, int32_t cols, int64_t stride_x, int32_t q_dtype,
                          void* q, void* scale, hipStream_t stream);

@@ -529,24 +529,41 @@ __global__ __launch_bounds__(256) void moe_smoothquant_grouped_kernel(const uint
 // scale = amax / 127, codes rounded to nearest even (|value / scale| <= 127 needs no clamp).  ck_tile has no
 // instance of these variants to match bit for bit, so the rounding is chosen for accuracy: truncation, which the
 // stand-alone smooth-quant kernel above has to use to match ck_tile's, doubles the error of the down GEMM's
-// input.  One wave per row; a row of up to 2048 columns is read once.
+// input.  FORM: who holds a row.  0: a wave, up to 2048 columns; 1: a wave that fetches the columns past those twice, one
+// piece at a time; 2: a workgroup, which has up to 8192 columns in flight together.  Form 2 for few rows, whose latency is what
+// the pass takes, and for rows long enough to keep its threads busy: 2 x 3 tokens of int8 experts 2624 x 8192, form 1 -> 2,
+// 76.3 -> 70.6 us a pass, 64 x 4 of 16 experts 1024 x 4352 69.8 -> 66.9, 3000 x 4 of 8192 529 -> 509, 1000 x 4 of 12288
+// 295 -> 287; 4000 x 4 of 4352 383 -> 387, of 5120 433 -> 437.
 // Output row-major, or slab-major when segs > 0 (y_slab_offset); padding rows and rows past the sorted prefix are left
 // alone.
 // FP8 (the fp8 path with fused_quant): e4m3 codes instead, scale = amax / 448, rounded to nearest even by the
-// conversion instruction.
-// LONG: rows of more pieces than a lane keeps take the exact quotients.  The pieces a lane fetches again come one at a time,
-// and with the bracket's branch in that loop 28 rows of 8320 took 13.2 us instead of 11.4, 8612 rows of 2496 18.8 instead of 17.9.
-template <bool SMOOTH, bool FP8, bool LONG>
+// conversion instruction; the workgroups from row_blocks on set the block scales the down GEMM reads (n_ones 16-byte
+// pieces) to 2^0, which as a launch of its own took 4.7 us.
+// Forms 1 and 2 take the exact quotients: with the bracket's branch in the loop over pieces fetched again 28 rows of 8320 took
+// 13.2 us instead of 11.4, 8612 rows of 2496 18.8 instead of 17.9 (form 1).
+template <bool SMOOTH, bool FP8, int FORM>
 __global__ __launch_bounds__(256) void moe_requant_y_kernel(const uint16_t* __restrict__ y, int inter,
                                                              const float* __restrict__ smooth,
                                                              const int* __restrict__ sorted_ids,
                                                              const int* __restrict__ sorted_expert_ids,
                                                              const int* __restrict__ total, int unit, int tokens, int topk,
                                                              int segs,
-                                                             unsigned char* __restrict__ yq, float* __restrict__ yscale)
+                                                             unsigned char* __restrict__ yq, float* __restrict__ yscale,
+                                                             int row_blocks, uint4* __restrict__ ones, int64_t n_ones)
 {
-    const int lane    = threadIdx.x & 63;
-    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    constexpr int kLanes  = FORM == 2 ? 256 : 64; // of a row
+    constexpr bool kExact = FORM > 0;
+    if constexpr(FP8)
+    {
+        if((int)blockIdx.x >= row_blocks)
+        {
+            for(int64_t i = (int64_t)(blockIdx.x - row_blocks) * 256 + threadIdx.x; i < n_ones; i += (int64_t)(gridDim.x - row_blocks) * 256)
+                ones[i] = make_uint4(0x7f7f7f7fu, 0x7f7f7f7fu, 0x7f7f7f7fu, 0x7f7f7f7fu);
+            return;
+        }
+    }
+    const int lane    = threadIdx.x & (kLanes - 1);
+    const int64_t row = FORM == 2 ? blockIdx.x : (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if(row >= total[0])
         return;
     const int chunks = inter >> 3;
@@ -579,7 +596,7 @@ __global__ __launch_bounds__(256) void moe_requant_y_kernel(const uint16_t* __re
 #pragma unroll
     for(int j = 0; j < kQuantCache; j++)
     {
-        const int c = lane + 64 * j;
+        const int c = lane + kLanes * j;
         if(c < chunks)
         {
             load(c, v[j]);
@@ -588,7 +605,7 @@ __global__ __launch_bounds__(256) void moe_requant_y_kernel(const uint16_t* __re
                 amax = fmaxf(amax, fabsf(v[j][i]));
         }
     }
-    for(int c = lane + 64 * kQuantCache; c < chunks; c += 64)
+    for(int c = lane + kLanes * kQuantCache; FORM > 0 && c < chunks; c += kLanes)
     {
         float t[8];
         load(c, t);
@@ -596,22 +613,28 @@ __global__ __launch_bounds__(256) void moe_requant_y_kernel(const uint16_t* __re
         for(int i = 0; i < 8; i++)
             amax = fmaxf(amax, fabsf(t[i]));
     }
-    amax = wave_reduce_max(amax, 0.f);
+    if constexpr(FORM == 2)
+    {
+        __shared__ float s_red[4];
+        amax = block_max_256(amax, s_red);
+    }
+    else
+        amax = wave_reduce_max(amax, 0.f);
     if(lane == 0)
         yscale[row] = amax / (FP8 ? 448.0f : 127.0f); // (a row of zeros: scale 0, codes 0)
     const RowScale<FP8> rs(amax);
-    [[maybe_unused]] const double s_rcp = LONG ? row_reciprocal(rs.scale()) : 0.0;
+    [[maybe_unused]] const double s_rcp = kExact ? row_reciprocal(rs.scale()) : 0.0;
     auto store = [&](int c, const float (&o)[8]) {
-        if constexpr(LONG)
+        if constexpr(kExact)
             *reinterpret_cast<uint2*>(dst(c)) = exact_codes_8<FP8, !FP8>(o, s_rcp);
         else
             *reinterpret_cast<uint2*>(dst(c)) = quantise_8<FP8, !FP8>(o, rs);
     };
 #pragma unroll
     for(int j = 0; j < kQuantCache; j++)
-        if(lane + 64 * j < chunks)
-            store(lane + 64 * j, v[j]);
-    for(int c = lane + 64 * kQuantCache; c < chunks; c += 64)
+        if(lane + kLanes * j < chunks)
+            store(lane + kLanes * j, v[j]);
+    for(int c = lane + kLanes * kQuantCache; FORM > 0 && c < chunks; c += kLanes)
     {
         float t[8];
         load(c, t);
@@ -760,20 +783,23 @@ int launch_rowwise_quant(const void* x, int64_t rows, int32_t cols, int64_t stri
 
 int launch_requant_y(const void* y, int32_t inter, const float* smooth, const int* sorted_ids, const int* sorted_expert_ids,
                      const int* total, int32_t unit, int32_t tokens, int32_t topk, int32_t segs, int64_t max_rows, void* yq, float* yscale,
-                     hipStream_t stream, bool fp8)
+                     hipStream_t stream, bool fp8, void* ones, int64_t ones_bytes)
 {
     if(max_rows <= 0)
         return MI355_MOE_OK;
     KernelTimer timer(MI355_MOE_K_QUANT, stream);
-    const dim3 grid((unsigned)ceil_div<int64_t>(max_rows, 4));
+    const int form       = inter <= 8 * 64 * kQuantCache ? 0 : max_rows <= 2048 || inter > 6144 ? 2 : 1; // (see the kernel)
+    const int row_blocks = (int)ceil_div<int64_t>(max_rows, form == 2 ? 1 : 4);
+    const int64_t n_ones = fp8 ? (ones_bytes + 15) / 16 : 0;
+    const dim3 grid((unsigned)(row_blocks + std::min<int64_t>(ceil_div<int64_t>(n_ones, 256), 4096)));
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, static_cast<const uint16_t*>(y), inter, smooth, sorted_ids,
-                           sorted_expert_ids, total, unit, tokens, topk, segs, static_cast<unsigned char*>(yq), yscale);
+                           sorted_expert_ids, total, unit, tokens, topk, segs, static_cast<unsigned char*>(yq), yscale, row_blocks,
+                           static_cast<uint4*>(ones), n_ones);
     };
-    const bool is_long = inter > 8 * 64 * kQuantCache;
     auto of_type       = [&](auto smooth_tag, auto fp8_tag) {
         constexpr bool S = decltype(smooth_tag)::value, F = decltype(fp8_tag)::value;
-        is_long ? launch(moe_requant_y_kernel<S, F, true>) : launch(moe_requant_y_kernel<S, F, false>);
+        form == 0 ? launch(moe_requant_y_kernel<S, F, 0>) : form == 1 ? launch(moe_requant_y_kernel<S, F, 1>) : launch(moe_requant_y_kernel<S, F, 2>);
     };
     if(fp8)
         smooth != nullptr ? of_type(std::true_type{}, std::true_type{}) : of_type(std::false_type{}, std::true_type{});
