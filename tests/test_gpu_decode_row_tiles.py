@@ -1,0 +1,61 @@
+"""Decode-sized batches in which one expert's rows fill several 32-row tiles and the others' one: the tiles' weights are then
+fetched as data read again by other workgroups, respectively read once.  All operand types and both weight layouts, sizes whose
+K ends inside a step, the down GEMM on the decode tiles and on the 256-column ones, against plain fp32 products."""
+import pytest
+
+from therock_amd import inputs as mi
+
+# (tokens, experts, topk, hidden, inter): rows of the popular expert are about half of tokens * topk
+SHAPES = [(70, 8, 1, 320, 384), (90, 16, 2, 832, 256), (130, 64, 2, 1088, 128)]
+
+
+def batch(T, E, K, H, I, dtype):
+    import numpy as np
+    inp = mi.make_inputs_np(mi.MoeConfig("row tiles", T, H, I, E, K, dtype, "softmax_renorm"), 5)
+    ids = inp["topk_ids"]
+    for t in range(0, T, 2):  # every second token also goes to expert 1
+        if 1 not in ids[t]:
+            ids[t, 0] = 1
+    for t in range(1, T, 2):
+        if 1 in ids[t] and t > 3:
+            ids[t, list(ids[t]).index(1)] = next(e for e in range(E) if e not in ids[t])
+    rows = np.bincount(ids.ravel(), minlength=E)
+    return inp, rows
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_the_batches_have_both_kinds_of_experts(shape):
+    T, E, K, H, I = shape
+    _, rows = batch(*shape, "bf16")
+    assert rows[1] > 32 and ((rows > 0) & (rows <= 32)).sum() > 3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["bf16", "fp16", "fp8", "int8"])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_experts_of_one_and_of_several_row_tiles(shape, dtype):
+    import numpy as np
+    import torch
+    import therock_amd as ta
+    from tests.gpu_reference import fused_moe_fp32
+    from tests.gpu_util import TORCH_DT, dev, run_fused_moe
+    T, E, K, H, I = shape
+    cfg = mi.MoeConfig("row tiles", T, H, I, E, K, dtype, "softmax_renorm")
+    traits = ta.fused_moe_traits(prec_i=dtype, prec_w=dtype, prec_o="fp16" if dtype == "fp16" else "bf16")
+    assert ta.fused_moe_tile_rows(traits, T, E, K, H, I) == 32
+    inp, _ = batch(*shape, dtype)
+    on = {k: None if v is None else dev(v) for k, v in inp.items()}
+    for k in ("a", "g", "d"):
+        on[k] = on[k].view(TORCH_DT[dtype])
+    ref = fused_moe_fp32(cfg, on)
+    plain, _ = run_fused_moe(cfg, inp)
+    got = torch.from_numpy(plain.astype(np.int16)).cuda().view(TORCH_DT["fp16" if dtype == "fp16" else "bf16"]).float()
+    err = float((got - ref).norm() / ref.norm())
+    print(f"row tiles {cfg}: rel-L2 = {err:.3e}", flush=True)
+    # the rounding of the intermediate rows: to 8 bits of mantissa and fewer (measured elsewhere: 3.3e-3, 2.7e-2 for fp8)
+    assert err <= (3e-2 if dtype == "fp8" else 1e-2)
+    per_row = (got - ref).norm(dim=1) / ref.norm(dim=1).clamp_min(1e-30)
+    assert float(per_row.max()) <= 6e-2  # a wrong tile or step would show in whole rows
+    if (H * (2 if dtype in ("bf16", "fp16") else 1)) % 64 == 0:
+        shuffled, _ = run_fused_moe(cfg, inp, weight_permute=1)
+        assert np.array_equal(plain, shuffled)

@@ -9,7 +9,7 @@
 // partial accumulators are added through LDS at the end (in wave order, so the result is
 // deterministic).  Same MFMA orientation (weight rows on the M side), operand layouts and epilogues
 // as moe_gemm_kernel; operand tiles are staged through LDS with the next step prefetched into
-// registers, weights with non-temporal loads.  NXB = 2 multiplies every weight tile with two token
+// registers, weights with non-temporal loads where the expert has a single row tile.  NXB = 2 multiplies every weight tile with two token
 // blocks (tiles of up to 64 sorted rows), so that experts with 33 .. 64 rows still stream their
 // weights once.
 #include "moe_gemm_device.hpp"
@@ -114,6 +114,7 @@ __global__ __launch_bounds__(kBlock, (NXB > 1 || MODE == kBf16W8 || MODE == kFp8
         else
             grow = min(n_base + blk * 32 + c, p.n_total - 1);
         woff[j] = weight_offset(p, grow, w_chunk0 + w_chunk_add(j));
+        asm volatile("" : "+v"(woff[j])); // (the upper half of the 64-bit multiply-add it comes from would stay alive beside it)
     }
 
     const int w_kadv = weight_k_advance(p, kDecWKB); // bytes between the K windows of two steps
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(kBlock, (NXB > 1 || MODE == kBf16W8 || MODE == kFp8
         ys_next_[0][i] = ys_next_[1][i] = ys_cur[i] = 0x7f7f7f7fu;
     const uint4 zero4 = {0u, 0u, 0u, 0u};
 
-    auto load_w = [&](int kt, auto buf_tag) __attribute__((always_inline)) {
+    auto load_w = [&](int kt, auto buf_tag, auto once_tag) __attribute__((always_inline)) {
         constexpr int B   = decltype(buf_tag)::value;
         auto& wv          = wv_[B];
         const int kw = kt * kDecWKB + w_chunk0 * 16;
@@ -138,8 +139,9 @@ __global__ __launch_bounds__(kBlock, (NXB > 1 || MODE == kBf16W8 || MODE == kFp8
             if(kw + w_chunk_add(j) * 16 < p.k_bytes_w)
             {
                 typedef __attribute__((ext_vector_type(4))) unsigned u32x4_t;
-                const u32x4_t t = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(wbase + (woff[j] + (uint32_t)(kt * w_kadv))));
-                wv[j]           = make_uint4(t[0], t[1], t[2], t[3]);
+                const u32x4_t* src = reinterpret_cast<const u32x4_t*>(wbase + (woff[j] + (uint32_t)(kt * w_kadv)));
+                const u32x4_t t    = decltype(once_tag)::value ? __builtin_nontemporal_load(src) : *src;
+                wv[j]              = make_uint4(t[0], t[1], t[2], t[3]);
             }
         }
     };
@@ -151,24 +153,23 @@ __global__ __launch_bounds__(kBlock, (NXB > 1 || MODE == kBf16W8 || MODE == kFp8
     const int kt_count = min(kt_all, kt_first + kt_slice);
     using B0 = std::integral_constant<int, 0>;
     using B1 = std::integral_constant<int, 1>;
-    load_w(kt_first, B0{});
-    __builtin_amdgcn_sched_barrier(0); // (the scheduler would put the ids' wait first)
-
     // addresses are a uniform base plus a 32-bit byte offset (the launcher checks that this suffices)
     uint32_t xoff[kXLoads];
     bool xvalid[kXLoads];
+    auto resolve_x = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for(int j = 0; j < kXLoads; j++)
-    {
-        const int r   = xrow + kXRowsPerPass * j;
-        xvalid[j]     = r < nrows && (!by_id || real_id(sid[j], p.tokens, GEMM0 ? p.topk : p.slot_rows));
-        uint32_t src  = row0 + r;
-        if constexpr(GEMM0)
-            src = token_row(p, sid[j]);
-        else if(p.slot_rows > 0)
-            src = (uint32_t)slot_row(sid[j], p.slot_rows);
-        xoff[j] = (xvalid[j] ? src : 0u) * (uint32_t)p.x_row_bytes + xchunk * 16;
-    }
+        for(int j = 0; j < kXLoads; j++)
+        {
+            const int r   = xrow + kXRowsPerPass * j;
+            xvalid[j]     = r < nrows && (!by_id || real_id(sid[j], p.tokens, GEMM0 ? p.topk : p.slot_rows));
+            uint32_t src  = row0 + r;
+            if constexpr(GEMM0)
+                src = token_row(p, sid[j]);
+            else if(p.slot_rows > 0)
+                src = (uint32_t)slot_row(sid[j], p.slot_rows);
+            xoff[j] = (xvalid[j] ? src : 0u) * (uint32_t)p.x_row_bytes + xchunk * 16;
+        }
+    };
     auto load_x = [&](int kt, auto buf_tag) __attribute__((always_inline)) {
         constexpr int B   = decltype(buf_tag)::value;
         auto& xv          = xv_[B];
@@ -208,7 +209,7 @@ __global__ __launch_bounds__(kBlock, (NXB > 1 || MODE == kBf16W8 || MODE == kFp8
             for(int v = 0; v < 16; v++)
                 acc[i][b][v] = 0;
 
-    auto k_step = [&](int kt, auto buf_tag) __attribute__((always_inline)) {
+    auto k_step = [&](int kt, auto buf_tag, auto once_tag) __attribute__((always_inline)) {
         constexpr int B = decltype(buf_tag)::value;
         auto& xv        = xv_[B];
         auto& wv        = wv_[B];
@@ -226,7 +227,7 @@ __global__ __launch_bounds__(kBlock, (NXB > 1 || MODE == kBf16W8 || MODE == kFp8
         if(kt + 2 < kt_count)
         {
             load_x(kt + 2, buf_tag);
-            load_w(kt + 2, buf_tag);
+            load_w(kt + 2, buf_tag, once_tag);
         }
         const unsigned char* xp = lds_x + r32 * kXStride + wave * kWaveWB * kXMul;
 #pragma unroll
@@ -270,17 +271,38 @@ __global__ __launch_bounds__(kBlock, (NXB > 1 || MODE == kBf16W8 || MODE == kFp8
         }
         __syncthreads();
     };
-    load_x(kt_first, B0{});
-    if(kt_first + 1 < kt_count)
+    auto walk = [&](auto once_tag) __attribute__((always_inline)) {
+        load_w(kt_first, B0{}, once_tag);
+        __builtin_amdgcn_sched_barrier(0); // (the scheduler would put the ids' wait first)
+        resolve_x();
+        load_x(kt_first, B0{});
+        if(kt_first + 1 < kt_count)
+        {
+            load_x(kt_first + 1, B1{});
+            load_w(kt_first + 1, B1{}, once_tag);
+        }
+        for(int kt = kt_first; kt < kt_count; kt += 2)
+        {
+            k_step(kt, B0{}, once_tag);
+            if(kt + 1 < kt_count)
+                k_step(kt + 1, B1{}, once_tag);
+        }
+    };
+    // Weights that only this workgroup reads are fetched non-temporal: 64 evenly routed tokens of 128 int8 experts 4096 x 1536
+    // 371 us, with plain loads 420.  Those of an expert with several row tiles are read by as many workgroups at about the same
+    // time, and with the hint each goes past L2 again: plain loads there take Zipf-routed batches from 250 to 221 us (256 tokens
+    // of that layer), 470 to 403 (the same in bf16), 352 to 324 (393 x 3 of 53 fp8 experts 6464 x 2560).  The walk stands here
+    // twice because a choice at each load makes the compiler wait for more loads than it has to (decode 1 to 3 % slower); the
+    // asm statements differ so that it does not fold the two walks' first loads into one and drop the hint.
+    if(tile.expert_tiles == 1)
     {
-        load_x(kt_first + 1, B1{});
-        load_w(kt_first + 1, B1{});
+        asm volatile("; weights read once");
+        walk(std::true_type{});
     }
-    for(int kt = kt_first; kt < kt_count; kt += 2)
+    else
     {
-        k_step(kt, B0{});
-        if(kt + 1 < kt_count)
-            k_step(kt + 1, B1{});
+        asm volatile("; weights read by several row tiles");
+        walk(std::false_type{});
     }
 
     // ---- add the four K slices: waves 1..3 park their accumulators in LDS, wave 0 sums in wave order
