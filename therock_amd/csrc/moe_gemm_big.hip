@@ -343,8 +343,11 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
     // Weights no other row tile re-reads (the expert has a single one) are fetched non-temporal: measured
     // -8 % on the gate+up GEMM at 32 rows per expert, -2 % at 256; with several row tiles per expert the
     // re-reads should hit L2, and non-temporal fetches cost 3 % there.  NT is a template argument like the
-    // slab-group count, for the same reason.
-    const bool w_nt = tile.expert_tiles == 1;
+    // slab-group count, for the same reason.  8-bit rows of an odd number of 64-byte pieces are left out: a 128-byte piece of
+    // every second row lies in two lines there, the pieces before and after in the same two, and with the hint each is fetched
+    // twice.  Passes, with -> without it: 1600 tokens x 8 of 64 int8 experts 4160 x 3008 870 -> 786 us, 1150 x 4 of 20 fp8 experts
+    // 6336 x 9344 1054 -> 995, 680 x 4 of 16 int8 experts 2112 x 14272 580 -> 542; at 90 rows per expert no difference.
+    const bool w_nt = tile.expert_tiles == 1 && (WPERM || p.w_row_bytes % 128 == 0);
     auto issue_w = [&](int u, auto half_tag, auto nt_tag) __attribute__((always_inline)) {
         constexpr int H = decltype(half_tag)::value;
         constexpr bool NT = decltype(nt_tag)::value;
