@@ -60,6 +60,14 @@ __device__ inline uint32_t fp8x4(float a, float b, float c, float d)
     return static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(c, d, w, true));
 }
 
+// v_cvt_i32_f32: toward zero, saturating, 0 for a NaN (which the language leaves undefined)
+__device__ inline int float_to_int(float v)
+{
+    int r;
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(r) : "v"(v));
+    return r;
+}
+
 // Eight codes in two dwords, each from the quotient rounded like the division; NEAREST: int8 codes rounded to nearest even
 // instead of toward zero.
 template <bool FP8, bool NEAREST>
@@ -90,14 +98,16 @@ __device__ inline uint2 exact_codes_8(const float (&o)[8], double s_rcp)
 // within 2^-20 of a code's boundary): one piece of eight in 2000 is done again with the fp64 product that rounds like the
 // division, and, with codes rounded toward zero, the piece that holds the row's maximum, whose quotient is 127 itself.
 // That product, two conversions at a quarter of the fp32 rate, was most of these kernels' instructions.
-// A NaN becomes -128 and -127 (e4m3: -448 and NaN) at the two ends, so it goes to the exact form too.
-// Used where a thread has one or two pieces (a wave's lane up to four in the re-quantisation), which are then in registers
-// for the exact form as well; with more, the branch costs more than it saves (see kBracketCols).  24008 rows of 1536
-// re-quantised between the GEMMs: 30 -> 25 us.
+// A NaN becomes -128 and 0 (e4m3: -448 and NaN) at the two ends, so it goes to the exact form too.  Codes rounded to nearest
+// are the low bytes of x * lo + 1.5 * 2^23, one fused instruction that rounds the product to an integer; a NaN, or a row whose
+// bracket is one, shows in the sum of x * 0 there.
+// Used where a thread has one or two pieces (up to four in the re-quantisation), which are then in registers for the exact
+// form as well; with more, the branch costs more than it saves (see kBracketCols).
 template <bool FP8, bool NEAREST = false>
 __device__ inline uint2 quantise_8(const float (&o)[8], const RowScale<FP8>& row)
 {
     uint2 lo, hi;
+    float bad = !FP8 && NEAREST ? row.lo : 0.0f;
     if constexpr(FP8)
     {
         float l[8], h[8];
@@ -116,26 +126,38 @@ __device__ inline uint2 quantise_8(const float (&o)[8], const RowScale<FP8>& row
 #pragma unroll
         for(int i = 0; i < 8; i++)
         {
-            const float a = __builtin_amdgcn_fmed3f(o[i] * row.lo, -128.f, 127.f);
-            const float b = __builtin_amdgcn_fmed3f(o[i] * row.hi, -127.f, 127.f);
-            l[i]          = static_cast<int>(NEAREST ? __builtin_rintf(a) : a);
-            h[i]          = static_cast<int>(NEAREST ? __builtin_rintf(b) : b);
+            if constexpr(NEAREST)
+            {
+                l[i] = __float_as_int(fmaf(o[i], row.lo, 0x1.8p23f));
+                h[i] = __float_as_int(fmaf(o[i], row.hi, 0x1.8p23f));
+                bad  = fmaf(o[i], 0.0f, bad);
+            }
+            else
+            {
+                l[i] = static_cast<int>(__builtin_amdgcn_fmed3f(o[i] * row.lo, -128.f, 127.f));
+                h[i] = float_to_int(o[i] * row.hi);
+            }
         }
         lo = make_uint2(pack_low_bytes(l[0], l[1], l[2], l[3]), pack_low_bytes(l[4], l[5], l[6], l[7]));
         hi = make_uint2(pack_low_bytes(h[0], h[1], h[2], h[3]), pack_low_bytes(h[4], h[5], h[6], h[7]));
     }
-    if(((lo.x ^ hi.x) | (lo.y ^ hi.y)) != 0)
+    if(((lo.x ^ hi.x) | (lo.y ^ hi.y)) != 0 || bad != bad)
         lo = exact_codes_8<FP8, NEAREST>(o, row_reciprocal(row.scale()));
     return lo;
 }
 
-__device__ inline float block_max_256(float v, float* s_red)
+template <int WAVES = 4>
+__device__ inline float block_max(float v, float* s_red)
 {
     v = wave_reduce_max(v, 0.f);
     if((threadIdx.x & 63) == 0)
         s_red[threadIdx.x >> 6] = v;
     __syncthreads();
-    return fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
+    float m = s_red[0];
+#pragma unroll
+    for(int w = 1; w < WAVES; w++)
+        m = fmaxf(m, s_red[w]);
+    return m;
 }
 
 // Per-row dynamic quantisation of one row by one 256-thread workgroup: xr bf16 (times sr fp32 when SMOOTH),
@@ -196,7 +218,7 @@ __device__ inline float quantise_row(const uint16_t* __restrict__ xr, const floa
             for(int i = 0; i < 8; i++)
                 amax = fmaxf(amax, fabsf(t[i]));
         }
-        amax          = block_max_256(amax, s_red);
+        amax          = block_max(amax, s_red);
         // a row of zeros: the scale written is 1 (row-wise quant) or 0 (smooth-quant, as amax / qmax gives);
         // either way the row's codes are 0, never the 0 / 0 the plain formula would convert
         if(threadIdx.x == 0)
@@ -226,7 +248,7 @@ __device__ inline float quantise_row(const uint16_t* __restrict__ xr, const floa
         float amax = 0.f;
         for(int c = threadIdx.x; c < cols; c += 256)
             amax = fmaxf(amax, fabsf(bf16_bits_to_float(xr[c]) * (SMOOTH ? sr[c] : 1.0f)));
-        amax          = block_max_256(amax, s_red);
+        amax          = block_max(amax, s_red);
         // a row of zeros: the scale written is 1 (row-wise quant) or 0 (smooth-quant, as amax / qmax gives);
         // either way the row's codes are 0, never the 0 / 0 the plain formula would convert
         const float s_out = (amax > 0.f || !unit_scale_when_zero) ? amax / qmx : 1.0f;
@@ -355,7 +377,7 @@ __global__ __launch_bounds__(256) void moe_smoothquant_vec_kernel(const uint16_t
             for(int i = 0; i < 8; i++)
                 amax = fmaxf(amax, fabsf(b[i]));
         }
-        amax            = block_max_256(amax, s_red[k & 1]); // two buffers: one barrier per slot suffices
+        amax            = block_max(amax, s_red[k & 1]); // two buffers: one barrier per slot suffices
         const int64_t r = (int64_t)k * tokens + t;
         if(threadIdx.x == 0)
             yscale[r] = amax / qmx; // (a row of zeros: scale 0, codes 0)
@@ -493,7 +515,7 @@ __global__ __launch_bounds__(256) void moe_smoothquant_grouped_kernel(const uint
             for(int i = 0; i < 8; i++)
                 amax = fmaxf(amax, fabsf(b[i]));
         }
-        amax               = block_max_256(amax, s_red[m & 1]); // two buffers: one barrier per row suffices
+        amax               = block_max(amax, s_red[m & 1]); // two buffers: one barrier per row suffices
         const int64_t r = (int64_t)k * tokens + t;
         if(threadIdx.x == 0)
             yscale[r] = amax / qmx; // (a row of zeros: scale 0, codes 0)
@@ -529,20 +551,18 @@ __global__ __launch_bounds__(256) void moe_smoothquant_grouped_kernel(const uint
 // scale = amax / 127, codes rounded to nearest even (|value / scale| <= 127 needs no clamp).  ck_tile has no
 // instance of these variants to match bit for bit, so the rounding is chosen for accuracy: truncation, which the
 // stand-alone smooth-quant kernel above has to use to match ck_tile's, doubles the error of the down GEMM's
-// input.  FORM: who holds a row.  0: a wave, up to 2048 columns; 1: a wave that fetches the columns past those twice, one
-// piece at a time; 2: a workgroup, which has up to 8192 columns in flight together.  Form 2 for few rows, whose latency is what
-// the pass takes, and for rows long enough to keep its threads busy: 2 x 3 tokens of int8 experts 2624 x 8192, form 1 -> 2,
-// 76.3 -> 70.6 us a pass, 64 x 4 of 16 experts 1024 x 4352 69.8 -> 66.9, 3000 x 4 of 8192 529 -> 509, 1000 x 4 of 12288
-// 295 -> 287; 4000 x 4 of 4352 383 -> 387, of 5120 433 -> 437.
+// input.  LANES: the threads that hold a row, so that it is read once: a wave up to 2048 columns, a workgroup of 256 up to
+// 8192, of 512 up to 16384 (the columns past those are fetched twice, a piece at a time, and take the exact quotients).
+// Bound by memory: 59787 rows of 12544 with smooth scales 700 us when 256 threads fetched a third of each row twice and every
+// code took its exact quotient, 616 without these, 522 (4.3 TB/s) with a slab's rows on one XCD; 23878 rows of 3904 (a wave each,
+// half of it fetched twice) 79 -> 62, 24008 of 1536 28 -> 22.
 // Output row-major, or slab-major when segs > 0 (y_slab_offset); padding rows and rows past the sorted prefix are left
 // alone.
 // FP8 (the fp8 path with fused_quant): e4m3 codes instead, scale = amax / 448, rounded to nearest even by the
 // conversion instruction; the workgroups from row_blocks on set the block scales the down GEMM reads (n_ones 16-byte
 // pieces) to 2^0, which as a launch of its own took 4.7 us.
-// Forms 1 and 2 take the exact quotients: with the bracket's branch in the loop over pieces fetched again 28 rows of 8320 took
-// 13.2 us instead of 11.4, 8612 rows of 2496 18.8 instead of 17.9 (form 1).
-template <bool SMOOTH, bool FP8, int FORM>
-__global__ __launch_bounds__(256) void moe_requant_y_kernel(const uint16_t* __restrict__ y, int inter,
+template <bool SMOOTH, bool FP8, int LANES>
+__global__ __launch_bounds__(LANES < 256 ? 256 : LANES) void moe_requant_y_kernel(const uint16_t* __restrict__ y, int inter,
                                                              const float* __restrict__ smooth,
                                                              const int* __restrict__ sorted_ids,
                                                              const int* __restrict__ sorted_expert_ids,
@@ -551,19 +571,25 @@ __global__ __launch_bounds__(256) void moe_requant_y_kernel(const uint16_t* __re
                                                              unsigned char* __restrict__ yq, float* __restrict__ yscale,
                                                              int row_blocks, uint4* __restrict__ ones, int64_t n_ones)
 {
-    constexpr int kLanes  = FORM == 2 ? 256 : 64; // of a row
-    constexpr bool kExact = FORM > 0;
+    constexpr int kThreads = LANES < 256 ? 256 : LANES;
+    constexpr bool kMore   = LANES == 512; // a row may have more columns than its threads hold
     if constexpr(FP8)
     {
         if((int)blockIdx.x >= row_blocks)
         {
-            for(int64_t i = (int64_t)(blockIdx.x - row_blocks) * 256 + threadIdx.x; i < n_ones; i += (int64_t)(gridDim.x - row_blocks) * 256)
+            for(int64_t i = (int64_t)(blockIdx.x - row_blocks) * kThreads + threadIdx.x; i < n_ones; i += (int64_t)(gridDim.x - row_blocks) * kThreads)
                 ones[i] = make_uint4(0x7f7f7f7fu, 0x7f7f7f7fu, 0x7f7f7f7fu, 0x7f7f7f7fu);
             return;
         }
     }
-    const int lane    = threadIdx.x & (kLanes - 1);
-    const int64_t row = FORM == 2 ? blockIdx.x : (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane    = threadIdx.x & (LANES - 1);
+    // Workgroup ids go round the eight XCDs: the rows of a 16-row slab, whose 64-byte pieces share lines, to one of them.  (Each
+    // round of slabs begins one XCD further on, as an expert's padding may leave the same slabs of every round empty.)
+    constexpr int kPerSlab = LANES > 64 ? 16 : 4; // workgroups
+    const int slot         = blockIdx.x >> 3;
+    const int round        = slot / kPerSlab;
+    const int64_t group    = (int64_t)(round * 8 + ((blockIdx.x + round) & 7)) * kPerSlab + slot % kPerSlab;
+    const int64_t row      = LANES > 64 ? group : group * 4 + (threadIdx.x >> 6);
     if(row >= total[0])
         return;
     const int chunks = inter >> 3;
@@ -596,7 +622,7 @@ __global__ __launch_bounds__(256) void moe_requant_y_kernel(const uint16_t* __re
 #pragma unroll
     for(int j = 0; j < kQuantCache; j++)
     {
-        const int c = lane + kLanes * j;
+        const int c = lane + LANES * j;
         if(c < chunks)
         {
             load(c, v[j]);
@@ -605,7 +631,7 @@ __global__ __launch_bounds__(256) void moe_requant_y_kernel(const uint16_t* __re
                 amax = fmaxf(amax, fabsf(v[j][i]));
         }
     }
-    for(int c = lane + kLanes * kQuantCache; FORM > 0 && c < chunks; c += kLanes)
+    for(int c = lane + LANES * kQuantCache; kMore && c < chunks; c += LANES)
     {
         float t[8];
         load(c, t);
@@ -613,32 +639,25 @@ __global__ __launch_bounds__(256) void moe_requant_y_kernel(const uint16_t* __re
         for(int i = 0; i < 8; i++)
             amax = fmaxf(amax, fabsf(t[i]));
     }
-    if constexpr(FORM == 2)
+    if constexpr(LANES > 64)
     {
-        __shared__ float s_red[4];
-        amax = block_max_256(amax, s_red);
+        __shared__ float s_red[LANES / 64];
+        amax = block_max<LANES / 64>(amax, s_red);
     }
     else
         amax = wave_reduce_max(amax, 0.f);
     if(lane == 0)
         yscale[row] = amax / (FP8 ? 448.0f : 127.0f); // (a row of zeros: scale 0, codes 0)
     const RowScale<FP8> rs(amax);
-    [[maybe_unused]] const double s_rcp = kExact ? row_reciprocal(rs.scale()) : 0.0;
-    auto store = [&](int c, const float (&o)[8]) {
-        if constexpr(kExact)
-            *reinterpret_cast<uint2*>(dst(c)) = exact_codes_8<FP8, !FP8>(o, s_rcp);
-        else
-            *reinterpret_cast<uint2*>(dst(c)) = quantise_8<FP8, !FP8>(o, rs);
-    };
 #pragma unroll
     for(int j = 0; j < kQuantCache; j++)
-        if(lane + kLanes * j < chunks)
-            store(lane + kLanes * j, v[j]);
-    for(int c = lane + kLanes * kQuantCache; FORM > 0 && c < chunks; c += kLanes)
+        if(lane + LANES * j < chunks)
+            *reinterpret_cast<uint2*>(dst(lane + LANES * j)) = quantise_8<FP8, !FP8>(v[j], rs);
+    for(int c = lane + LANES * kQuantCache; kMore && c < chunks; c += LANES)
     {
         float t[8];
         load(c, t);
-        store(c, t);
+        *reinterpret_cast<uint2*>(dst(c)) = exact_codes_8<FP8, !FP8>(t, row_reciprocal(rs.scale()));
     }
 }
 
@@ -788,18 +807,19 @@ int launch_requant_y(const void* y, int32_t inter, const float* smooth, const in
     if(max_rows <= 0)
         return MI355_MOE_OK;
     KernelTimer timer(MI355_MOE_K_QUANT, stream);
-    const int form       = inter <= 8 * 64 * kQuantCache ? 0 : max_rows <= 2048 || inter > 6144 ? 2 : 1; // (see the kernel)
-    const int row_blocks = (int)ceil_div<int64_t>(max_rows, form == 2 ? 1 : 4);
+    const int lanes      = inter <= 8 * 64 * kQuantCache ? 64 : inter <= 8 * 256 * kQuantCache ? 256 : 512; // (see the kernel)
+    const int threads    = std::max(lanes, 256);
+    const int row_blocks = (int)round_up<int64_t>(ceil_div<int64_t>(max_rows, threads / lanes), lanes > 64 ? 128 : 32); // whole rounds
     const int64_t n_ones = fp8 ? (ones_bytes + 15) / 16 : 0;
-    const dim3 grid((unsigned)(row_blocks + std::min<int64_t>(ceil_div<int64_t>(n_ones, 256), 4096)));
+    const dim3 grid((unsigned)(row_blocks + std::min<int64_t>(ceil_div<int64_t>(n_ones, threads), 4096)));
     auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, static_cast<const uint16_t*>(y), inter, smooth, sorted_ids,
+        hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, stream, static_cast<const uint16_t*>(y), inter, smooth, sorted_ids,
                            sorted_expert_ids, total, unit, tokens, topk, segs, static_cast<unsigned char*>(yq), yscale, row_blocks,
                            static_cast<uint4*>(ones), n_ones);
     };
     auto of_type       = [&](auto smooth_tag, auto fp8_tag) {
         constexpr bool S = decltype(smooth_tag)::value, F = decltype(fp8_tag)::value;
-        form == 0 ? launch(moe_requant_y_kernel<S, F, 0>) : form == 1 ? launch(moe_requant_y_kernel<S, F, 1>) : launch(moe_requant_y_kernel<S, F, 2>);
+        lanes == 64 ? launch(moe_requant_y_kernel<S, F, 64>) : lanes == 256 ? launch(moe_requant_y_kernel<S, F, 256>) : launch(moe_requant_y_kernel<S, F, 512>);
     };
     if(fp8)
         smooth != nullptr ? of_type(std::true_type{}, std::true_type{}) : of_type(std::false_type{}, std::true_type{});
