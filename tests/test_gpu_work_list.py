@@ -56,3 +56,23 @@ def test_scan_pass_lists_experts_of_many_tiles(masked, dtype):
     got, _ = run_fused_moe(cfg, inp, mask=mask)
     ref, _ = oracle_out(cfg, inp, mask)
     assert rel_l2(oracle.bf16_to_f32(got), ref) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("tokens,experts,topk", [(10240, 8, 1), (10241, 8, 1), (5123, 256, 2), (8192, 60, 2)])
+def test_both_sorts_of_the_fused_call(tokens, experts, topk, masked):
+    # around the size from which the fused call sorts in three launches: the stand-alone sort, in one workgroup up to here, and
+    # the GEMMs on its arrays give the same bits
+    from tests.gpu_util import run_fused_moe
+    cfg = mi.MoeConfig("sorts", tokens, 128, 128, experts, topk, "bf16", "softmax_renorm", unit=32)
+    inp = mi.make_inputs_np(cfg, 5)
+    mask = (np.arange(experts) % 3 != 1).astype(np.int32) if masked else None
+    if masked:
+        for k in ("g", "d"):
+            inp[k] = inp[k][:int(mask.sum())]
+    (fused, a), (apart, b) = run_fused_moe(cfg, inp, mask=mask), run_fused_moe(cfg, inp, mask=mask, unfused=True)
+    n = int(a.total[0])
+    assert n == int(b.total[0]) and n > 0
+    for x, y, m in ((a.sorted_ids, b.sorted_ids, n), (a.sorted_w, b.sorted_w, n), (a.sorted_eid, b.sorted_eid, n // 32)):
+        assert np.array_equal(x[:m].cpu().numpy(), y[:m].cpu().numpy())
+    assert np.array_equal(fused, apart)
