@@ -80,6 +80,19 @@ constexpr bool stages_fit(int groups)
 }
 static_assert(stages_fit(1) && stages_fit(2) && stages_fit(3) && stages_fit(4) && stages_fit(kMaxNB), "LDS budget");
 
+// Epilogue operands of a gate+up tile of 8-bit operands, fetched into LDS ahead of the first stages, where a tile of up to four
+// token groups leaves room: the 256 weight rows' scales, the token rows' scales and their sorted ids, 1 KiB each.  Loaded behind
+// the K loop they were two dependent round trips, one past L2, with nothing else of the compute unit in flight (4300 clocks
+// of a tile's 35000 where K is 640 bytes).  Passes: 8541 tokens x 7 of 166 int8 experts 640 x 12544 3310 -> 3139 us, 3526 x 5 of 111
+// int8 experts 512 x 1792 194 -> 189, 4054 x 8 of 47 int8 experts 3072 x 896 499 -> 484.
+constexpr int kEpiGroups   = 4;
+constexpr int kEpiRows     = kEpiGroups * 64;
+constexpr int kEpiOffset   = kLdsBytes - 3 * 1024;
+constexpr int kEpiChannels = kEpiOffset, kEpiScales = kEpiOffset + 1024, kEpiIds = kEpiOffset + 2048;
+constexpr bool epilogue_fits(int groups) { return kXOffsetPair + pair_stages(groups) * pair_stage_bytes(groups) <= kEpiOffset; }
+static_assert(epilogue_fits(1) && epilogue_fits(2) && epilogue_fits(3) && epilogue_fits(kEpiGroups) && kBigWRows * 4 <= 1024 && kEpiRows * 4 <= 1024,
+              "LDS budget of the epilogue's operands");
+
 typedef __attribute__((address_space(3))) unsigned char lds_byte_t;
 
 // Chunk swizzle of the 128-byte weight rows in LDS.  The 16 lanes that a ds_read_b128 serves together read the rows
@@ -428,6 +441,30 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
     // token blocks of this wave (blocks wt, wt + 2, ..) and 64-row slab groups that hold rows of the tile
     const int nb_w     = __builtin_amdgcn_readfirstlane(max(0, min(kMaxNB, (nmb - wt + 1) / 2)));
     const int x_groups = __builtin_amdgcn_readfirstlane(max(1, (nmb + 1) / 2));
+
+    // the epilogue's operands: ahead of all other transfers of these waves, so that the first wait covers them
+    constexpr bool kEpi = kXPair && (MODE == kI8 || MODE == kFp8);
+    const bool epi_lds  = kEpi && x_groups <= kEpiGroups && p.w_scale != nullptr && p.x_scale != nullptr;
+    if constexpr(kEpi)
+    {
+        if(epi_lds && w_role)
+        {
+            // scale of weight row i of the tile, 64 a wave
+            const int i   = q4 * 64 + lane;
+            const int row = paired ? (i >> 7) * p.n_out + min(n_base + (i & 127), p.n_out - 1) : min(n_base + i, p.n_total - 1);
+            dma4(reinterpret_cast<const unsigned char*>(p.w_scale + (int64_t)expert * p.n_total), (uint32_t)row * 4u,
+                 __builtin_amdgcn_readfirstlane(lds_base + kEpiChannels + q4 * 256));
+        }
+        else if(epi_lds)
+        {
+            const int r   = min(q4 * 64 + lane, nrows - 1);
+            const int sid = p.sorted_ids[row0 + r];
+            dma4(reinterpret_cast<const unsigned char*>(p.sorted_ids + row0), (uint32_t)r * 4u,
+                 __builtin_amdgcn_readfirstlane(lds_base + kEpiIds + q4 * 256));
+            dma4(reinterpret_cast<const unsigned char*>(p.x_scale), real_id(sid, p.tokens, p.topk) ? token_row(p, sid) * 4u : 0u,
+                 __builtin_amdgcn_readfirstlane(lds_base + kEpiScales + q4 * 256));
+        }
+    }
 
     Acc acc[kMaxNB][2];
 #pragma unroll
@@ -829,7 +866,34 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
     }
 
     // ---- epilogue
-    run_epilogue<MODE, GEMM0, kMaxNB>(p, acc, expert, row0, nrows, wt * 32, 64, nb_w, n_base, ww, r32, kg, slice);
+    if constexpr(kEpi)
+    {
+        EpilogueOperands<kMaxNB> o;
+        if(epi_lds)
+        {
+            o.cols = epilogue_columns<GEMM0>(p, n_base, ww, kg);
+            // (rows of a column group the tile does not have hold another row's scale; nothing is stored for them)
+            const float* sc = reinterpret_cast<const float*>(lds + kEpiChannels) + (paired ? ww * 32 : ww * 64) + 16 * kg;
+            load_channel_scales(sc, o.sc0);
+            load_channel_scales(sc + (paired ? 128 : 32), o.sc1);
+#pragma unroll
+            for(int i = 0; i < kMaxNB; i++)
+            {
+                const int r      = wt * 32 + i * 64 + r32;
+                const int at     = min(min(r, nrows - 1), kEpiRows - 1);
+                const int sid    = reinterpret_cast<const int*>(lds + kEpiIds)[at];
+                o.rows.real[i]   = real_id(sid, p.tokens, p.topk);
+                o.rows.sa[i]     = o.rows.real[i] ? reinterpret_cast<const float*>(lds + kEpiScales)[at] : 0.0f;
+                o.rows.orow[i]   = p.slot_rows <= 0 ? row0 + r : o.rows.real[i] ? (int)slot_row(sid, p.slot_rows) : 0;
+            }
+        }
+        else
+            load_epilogue<MODE, GEMM0, kMaxNB>(p, o, expert, row0, nrows, wt * 32, 64, n_base, ww, r32, kg, slice);
+        pin_epilogue(o);
+        apply_epilogue<MODE, GEMM0, kMaxNB>(p, acc, o, row0, nrows, wt * 32, 64, nb_w, r32, kg, expert);
+    }
+    else
+        run_epilogue<MODE, GEMM0, kMaxNB>(p, acc, expert, row0, nrows, wt * 32, 64, nb_w, n_base, ww, r32, kg, slice);
 }
 
 template <int MODE, bool GEMM0, bool WPERM>
