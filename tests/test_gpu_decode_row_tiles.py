@@ -7,7 +7,8 @@ import pytest
 from therock_amd import inputs as mi
 
 # (tokens, experts, topk, hidden, inter): rows of the popular expert are about half of tokens * topk
-SHAPES = [(70, 8, 1, 320, 384), (90, 16, 2, 832, 256), (130, 64, 2, 1088, 128), (130, 64, 2, 1088, 192), (1100, 64, 2, 1088, 256)]
+SHAPES = [(70, 8, 1, 320, 384), (90, 16, 2, 832, 256), (130, 64, 2, 1088, 128), (130, 64, 2, 1088, 192), (1100, 64, 2, 1088, 256),
+          (130, 64, 2, 1856, 128), (130, 64, 2, 1856, 192), (300, 256, 2, 2048, 128)]
 
 
 def batch(T, E, K, H, I, dtype):
