@@ -249,7 +249,7 @@ __global__ __launch_bounds__(kBigThreads) void moe_gemm_big_kernel(const GemmPar
                     grow = (blk & 1) * p.n_out + min(n_base + (blk >> 1) * 32 + c, p.n_out - 1);
                 else
                     grow = min(n_base + blk * 32 + c, p.n_total - 1);
-                doff[h * 4 + j] = weight_offset(p, grow, cchunk);
+                doff[h * 4 + j] = weight_offset(p, p.w_permuted != 0, grow, cchunk);
             }
     }
     else

@@ -117,9 +117,9 @@ __host__ __device__ __attribute__((always_inline)) inline int64_t slot_row(int s
 // into a window of K that begins on a multiple of 64 bytes; and what moving that window by `bytes` (a multiple of
 // 64) adds to it.  Row-major: row * row_bytes + 16 * chunk16, + bytes.  Pre-shuffled: the row's block row, the block
 // (chunk16 / 4) of the window, the piece inside the block; a window 64 bytes further on is the next 1 KiB block.
-__device__ __attribute__((always_inline)) inline uint32_t weight_offset(const GemmParams& p, int row, int chunk16)
+__device__ __attribute__((always_inline)) inline uint32_t weight_offset(const GemmParams& p, bool permuted, int row, int chunk16)
 {
-    if(p.w_permuted == 0)
+    if(!permuted)
         return (uint32_t)row * (uint32_t)p.w_row_bytes + chunk16 * 16;
     return (uint32_t)(row >> 4) * (uint32_t)(p.w_row_bytes * 16) + (chunk16 >> 2) * 1024 + (chunk16 & 3) * 256 + (row & 15) * 16;
 }
