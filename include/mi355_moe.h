@@ -30,10 +30,10 @@
 extern "C" {
 #endif
 
-/* 230: mi355_fused_moe_k_slices and mi355_moe_flatmm_k_slices added; 220: entry points added;
+/* 240: mi355_fused_moe_down_tile_cols added; 230: mi355_fused_moe_k_slices and mi355_moe_flatmm_k_slices added; 220: entry points added;
  * 210: mi355_fused_moe_traits gained weight_permute and mi355_moe_flatmm_args gained b_shuffle (both appended; a
  * caller built against 200 must be rebuilt), mi355_fused_moe_chosen_tile_rows added */
-#define MI355_MOE_VERSION 230
+#define MI355_MOE_VERSION 240
 
 enum mi355_moe_status
 {
@@ -276,6 +276,12 @@ int32_t mi355_fused_moe_k_slices(const mi355_fused_moe_traits* traits, int32_t t
  * ck_tile's dispatcher selects (fused_moegemm_shape.hpp:43-64); here it is chosen per problem size. */
 int32_t mi355_fused_moe_tile_rows(const mi355_fused_moe_traits* traits, int32_t tokens, int32_t num_experts,
                                   int32_t topk, int32_t hidden_size, int32_t intermediate_size);
+
+/* For harnesses and tests: weight rows (output columns) one workgroup of the down GEMM owns at this problem size (token rows
+ * packed, and on tiles of mi355_fused_moe_tile_rows() rows): 64 (moe_gemm_decode_kernel) or 256; 0 for unsupported traits.  No
+ * counterpart in ck_tile. */
+int32_t mi355_fused_moe_down_tile_cols(const mi355_fused_moe_traits* traits, int32_t tokens, int32_t num_experts, int32_t topk,
+                                       int32_t hidden, int32_t inter);
 
 /* For harnesses and tests: the tile height the last mi355_fused_moe or mi355_fused_moegemm call on `ws` ran with.  Where
  * the routing decides (fp8 operands below about 28 rows per expert on average: a skewed batch whose active experts' rows,

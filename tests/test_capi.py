@@ -156,6 +156,7 @@ for prec, fq, go in ((0, 0, 0), (1, 0, 0), (1, 2, 1), (2, 1, 0), (2, 0, 1)):
         for T, E, K in ((7, 64, 9), (1, 1, 1), (4096, 4, 2)):
             assert lib.mi355_fused_moe_workspace_size(C.byref(t), T, E, K, H, I) == 0, (T, E, K, H, I)
             assert lib.mi355_fused_moe_tile_rows(C.byref(t), T, E, K, H, I) == 0
+            assert lib.mi355_fused_moe_down_tile_cols(C.byref(t), T, E, K, H, I) == 0
             assert lib.mi355_fused_moe_k_slices(C.byref(t), T, E, K, H, I, 1 << 60) == 0
             f = _lib.FusedMoeArgs(block_m=32, hidden_size=H, intermediate_size=I, num_tokens=T, num_experts=E, topk=K, stride_token=H)
             assert lib.mi355_fused_moe(C.byref(t), C.byref(f), None, None) == _lib.E_INVALID

@@ -41,3 +41,22 @@ def test_down_gemms_that_are_cut():
                                     ((1210, 4, 84, 896, 11776), 3)):
         assert ta.fused_moe_tile_rows(fp8(), T, E, K, H, I) == 320
         assert ta.fused_moe_k_slices(fp8(), T, E, K, H, I, 1 << 40) == slices
+
+
+def test_down_gemms_on_the_decode_kernel():
+    """Below 1.6 tiles of 256 columns a compute unit, counted over the experts that can have a row; 8-bit rows of less than 1536
+    bytes below one; 16-bit weights below 8; never on the large tiles."""
+    def cols(dtype, T, K, E, H, I, **kw):
+        traits = ta.fused_moe_traits(prec_i=dtype, prec_w=dtype, prec_o="fp16" if dtype == "fp16" else "bf16", block_m=32, **kw)
+        return ta.fused_moe_down_tile_cols(traits, T, E, K, H, I)
+    # short rows, 1.0 to 1.6 tiles a compute unit: 8 to 14 % slower on the narrow tiles
+    for case in (("int8", 65, 2, 17, 5120, 512), ("fp8", 32, 3, 17, 5184, 512), ("int8", 13, 4, 111, 1664, 576), ("fp8", 142, 6, 128, 640, 1408)):
+        assert cols(*case) == 256, case
+    assert cols("fp8", 97, 8, 25, 3904, 512, fused_quant=1) == 256
+    # rows from 1536 bytes on; short ones below one tile; 16-bit rows
+    for case in (("int8", 98, 5, 53, 1152, 1536), ("int8", 4, 5, 30, 3136, 8896), ("int8", 65, 2, 17, 2560, 512), ("bf16", 65, 2, 17, 5120, 512),
+                 ("fp16", 135, 1, 203, 2304, 1216)):
+        assert cols(*case) == 64, case
+    # past the lines, and large tiles
+    for case in (("fp8", 652, 1, 150, 704, 2048), ("int8", 64, 8, 128, 4096, 1536), ("bf16", 64, 8, 128, 4096, 1536), ("bf16", 4096, 2, 8, 4096, 14336)):
+        assert cols(*case) == 256, case

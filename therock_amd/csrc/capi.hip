@@ -290,6 +290,16 @@ mi355_fused_moe_tile_rows(const mi355_fused_moe_traits* traits, int32_t tokens, 
 }
 
 __attribute__((visibility("default"))) int32_t
+mi355_fused_moe_down_tile_cols(const mi355_fused_moe_traits* traits, int32_t tokens, int32_t num_experts, int32_t topk,
+                               int32_t hidden_size, int32_t intermediate_size)
+{
+    if(traits == nullptr || check_traits(*traits) != MI355_MOE_OK ||
+       !sizes_in_range(tokens, num_experts, topk, hidden_size, intermediate_size))
+        return 0;
+    return down_gemm_tile_cols(*traits, tokens, num_experts, topk, hidden_size, intermediate_size);
+}
+
+__attribute__((visibility("default"))) int32_t
 mi355_fused_moe_chosen_tile_rows(const mi355_fused_moe_traits* traits, int32_t tokens, int32_t num_experts, int32_t topk,
                                  int32_t hidden_size, int32_t intermediate_size, const mi355_moe_workspace* ws, void* stream)
 {

@@ -370,6 +370,12 @@ def fused_moe_tile_rows(traits: fused_moe_traits, tokens, num_experts, topk, hid
                                                      intermediate_size))
 
 
+def fused_moe_down_tile_cols(traits: fused_moe_traits, tokens, num_experts, topk, hidden_size, intermediate_size) -> int:
+    """Output columns one workgroup of the down GEMM owns at this problem size (64 selects the decode kernel, else 256)."""
+    t = traits.pod()
+    return int(_lib.load().mi355_fused_moe_down_tile_cols(C.byref(t), tokens, num_experts, topk, hidden_size, intermediate_size))
+
+
 def fused_moe_k_slices(traits: fused_moe_traits, tokens, num_experts, topk, hidden_size, intermediate_size, ws_bytes) -> int:
     """Slices of K the down GEMM is cut into with a workspace of ws_bytes (1: not cut, 0: too small for the call)."""
     t = traits.pod()
