@@ -60,3 +60,20 @@ def test_down_gemms_on_the_decode_kernel():
     # past the lines, and large tiles
     for case in (("fp8", 652, 1, 150, 704, 2048), ("int8", 64, 8, 128, 4096, 1536), ("bf16", 64, 8, 128, 4096, 1536), ("bf16", 4096, 2, 8, 4096, 14336)):
         assert cols(*case) == 256, case
+
+
+def test_heights_where_the_down_gemm_runs_the_decode_kernel_past_one_tile():
+    """Tiles of 128 and 320 rows stay: at 32 rows popular experts would stream their weights many times.  Of 64 rows and 32 the
+    faster ones, and 32 stays where the rows are short."""
+    def rows(dtype, T, K, E, H, I, **kw):
+        traits = ta.fused_moe_traits(prec_i=dtype, prec_w=dtype, prec_o="fp16" if dtype == "fp16" else "bf16", block_m=32, **kw)
+        return ta.fused_moe_tile_rows(traits, T, E, K, H, I)
+    assert rows("bf16", 698, 8, 203, 576, 6848) == 128
+    assert rows("bf16", 1640, 4, 243, 832, 5312, gate_only=1) == 128
+    assert rows("int8", 426, 8, 124, 640, 4160, fused_quant=1) == 128
+    assert rows("bf16", 1309, 1, 72, 832, 12800, weight_permute=1) == 320
+    assert rows("fp16", 896, 2, 63, 1088, 10496) == 320
+    assert rows("bf16", 98, 8, 35, 1856, 6912) == 32
+    assert rows("fp8", 64, 5, 11, 6848, 3712) == 32
+    assert rows("fp8", 132, 4, 12, 7040, 896) == 32
+    assert rows("int8", 73, 5, 11, 6400, 576, gate_only=1) == 32
