@@ -89,7 +89,7 @@ __device__ inline uint2 exact_codes_8(const float (&o)[8], double s_rcp)
         int c[8];
 #pragma unroll
         for(int i = 0; i < 8; i++)
-            c[i] = NEAREST ? static_cast<int>(__builtin_rintf(q[i])) : static_cast<int>(static_cast<signed char>(quantise_one<false>(q[i])));
+            c[i] = NEAREST ? float_to_int(__builtin_rintf(q[i])) : static_cast<int>(static_cast<signed char>(quantise_one<false>(q[i])));
         return make_uint2(pack_low_bytes(c[0], c[1], c[2], c[3]), pack_low_bytes(c[4], c[5], c[6], c[7]));
     }
 }
