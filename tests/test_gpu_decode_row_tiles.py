@@ -6,9 +6,13 @@ import pytest
 
 from therock_amd import inputs as mi
 
-# (tokens, experts, topk, hidden, inter): rows of the popular expert are about half of tokens * topk
-SHAPES = [(70, 8, 1, 320, 384), (90, 16, 2, 832, 256), (130, 64, 2, 1088, 128), (130, 64, 2, 1088, 192), (1100, 64, 2, 1088, 256),
-          (130, 64, 2, 1856, 128), (130, 64, 2, 1856, 192), (300, 256, 2, 2048, 128)]
+# (tokens, experts, topk, hidden, inter): rows of the popular expert are about half of tokens * topk; and the columns of the
+# down GEMM's tiles with 16-bit and with 8-bit weights (64: the decode kernel)
+DOWN = {(70, 8, 1, 320, 384): (64, 64), (90, 16, 2, 832, 256): (64, 64), (130, 64, 2, 1088, 128): (64, 256), (130, 64, 2, 1088, 192): (64, 256),
+        (130, 64, 2, 1088, 1536): (64, 64), (1100, 64, 2, 1088, 256): (256, 256), (1100, 64, 2, 1088, 160): (256, 256),
+        (1100, 64, 2, 1088, 192): (256, 256), (130, 64, 2, 1856, 128): (64, 256), (130, 64, 2, 1856, 192): (64, 256),
+        (300, 256, 2, 2048, 128): (256, 256), (300, 256, 2, 2304, 160): (256, 256)}
+SHAPES = list(DOWN)
 
 
 def batch(T, E, K, H, I, dtype):
@@ -31,6 +35,15 @@ def test_the_batches_have_both_kinds_of_experts(shape):
     _, rows = batch(*shape, "bf16")
     height = 64 if T > 1000 else 32
     assert rows[1] > height and ((rows > 0) & (rows <= height)).sum() > 3
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16", "fp8", "int8"])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_the_down_gemm_runs_the_kernel_it_is_here_for(shape, dtype):
+    import therock_amd as ta
+    T, E, K, H, I = shape
+    traits = ta.fused_moe_traits(prec_i=dtype, prec_w=dtype, prec_o="fp16" if dtype == "fp16" else "bf16")
+    assert ta.fused_moe_down_tile_cols(traits, T, E, K, H, I) == DOWN[shape][dtype in ("fp8", "int8")]
 
 
 @pytest.mark.gpu
@@ -61,6 +74,6 @@ def test_experts_of_one_and_of_several_row_tiles(shape, dtype):
     assert err <= (3e-2 if dtype == "fp8" else 1e-2)
     per_row = (got - ref).norm(dim=1) / ref.norm(dim=1).clamp_min(1e-30)
     assert float(per_row.max()) <= 6e-2  # a wrong tile or step would show in whole rows
-    if (H * (2 if dtype in ("bf16", "fp16") else 1)) % 64 == 0:
+    if all(n * (2 if dtype in ("bf16", "fp16") else 1) % 64 == 0 for n in (H, I)):  # (the pre-shuffled layout's blocks)
         shuffled, _ = run_fused_moe(cfg, inp, weight_permute=1)
         assert np.array_equal(plain, shuffled)

@@ -120,9 +120,9 @@ def bf16_rows(kind, exponents, cols, seed):
 @pytest.mark.gpu
 @pytest.mark.parametrize("fq", [1, 2])
 @pytest.mark.parametrize("dtype", ["int8", "fp8"])
-# (with a sort unit of 256 there may be more than 2048 rows, which a wave each takes up to 6144 columns of)
-@pytest.mark.parametrize("inter,unit", [(512, 32), (2048, 32), (2176, 32), (4224, 32), (8320, 32), (2176, 256), (4224, 256)])
-def test_requantised_codes_at_boundaries(inter, unit, dtype, fq):
+# (a row to a wave up to 2048 columns, to 256 threads up to 8192, to 512 beyond, which hold 16384 columns of it)
+@pytest.mark.parametrize("inter", [512, 2048, 2176, 4224, 8192, 8320, 16384, 16512])
+def test_requantised_codes_at_boundaries(inter, dtype, fq):
     import torch
     import therock_amd as ta
     exponents = [0, 0, -30, 40, -99, 98, -101, 101, 112, 112]  # (the least value, 2^-19 of the maximum / 64, stays normal)
@@ -145,7 +145,7 @@ def test_requantised_codes_at_boundaries(inter, unit, dtype, fq):
         smooth = (values / 64).contiguous()
     else:
         g_scale[:, inter:] = values / 4096  # 64 of the gate half, 64 of the tokens' scale
-    traits = ta.fused_moe_traits(prec_i=dtype, prec_w=dtype, block_m=unit, gate_only=int(fq == 1), fused_quant=fq)
+    traits = ta.fused_moe_traits(prec_i=dtype, prec_w=dtype, block_m=32, gate_only=int(fq == 1), fused_quant=fq)
     buf = ta.MoeBuffers(traits, T, E, 1, H, inter, "cuda")
     args = ta.make_args(traits, buf, a.view(view), g.view(view), d.view(view), torch.arange(T, dtype=torch.int32, device="cuda").reshape(T, 1),
                         torch.ones((T, 1), device="cuda"), a_scale=torch.full((T,), 64.0, device="cuda"), g_scale=g_scale,

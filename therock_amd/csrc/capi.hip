@@ -400,8 +400,9 @@ int run_fused_moe(const mi355_fused_moe_traits* traits, const mi355_fused_moe_ar
     s.num_experts             = a->num_experts;
     s.topk                    = a->topk;
     // More than 10240 entries: the three launches, though one workgroup takes up to 16384.  It stores the scattered ids and
-    // weights from one compute unit, 3 ns an entry: 12288 entries of 8 / 256 experts 14.5 / 23.5 us, in three launches 13.4 / 21.1,
-    // 16384 entries 22.2 / 30.1 and 14.0 / 20.1; 8192 entries 12.5 / 17.2 and 13.3 / 20.1 (passes: 2000 tokens x 8 of 256 fp8 experts
+    // weights from one compute unit, 1.6 to 1.9 ns an entry past 12288, where the three launches hardly grow: 12288 entries of 8 / 256
+    // experts 14.5 / 23.5 us, in three launches 13.4 / 21.1, 16384 entries 22.2 / 30.1 and 14.0 / 20.1; 8192 entries 12.5 / 17.2 and
+    // 13.3 / 20.1 (passes: 2000 tokens x 8 of 256 fp8 experts
     // 1024 x 1024 247 -> 236 us; 1025 x 8 of 64 bf16 ones, on this side of the line, would take 130 instead of 128).  The counters
     // (32 KB at most) lie where the down GEMM's rows come later, so that no call needs a larger workspace.
     constexpr int64_t kOneWorkgroupMost = 10240;
