@@ -10,7 +10,7 @@ from therock_amd import inputs as mi
 # down GEMM's tiles with 16-bit and with 8-bit weights (64: the decode kernel)
 DOWN = {(70, 8, 1, 320, 384): (64, 64), (90, 16, 2, 832, 256): (64, 64), (130, 64, 2, 1088, 128): (64, 256), (130, 64, 2, 1088, 192): (64, 256),
         (130, 64, 2, 1088, 1536): (64, 64), (1100, 64, 2, 1088, 256): (256, 256), (1100, 64, 2, 1088, 160): (256, 256),
-        (1100, 64, 2, 1088, 192): (256, 256), (130, 64, 2, 1856, 128): (64, 256), (130, 64, 2, 1856, 192): (64, 256),
+        (1100, 64, 2, 1088, 192): (256, 256), (1100, 64, 2, 1856, 256): (256, 256), (130, 64, 2, 1856, 128): (64, 256), (130, 64, 2, 1856, 192): (64, 256),
         (300, 256, 2, 2048, 128): (256, 256), (300, 256, 2, 2304, 160): (256, 256)}
 SHAPES = list(DOWN)
 
