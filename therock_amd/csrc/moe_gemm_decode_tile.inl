@@ -262,8 +262,9 @@
     };
     // Weights that only this workgroup reads are fetched non-temporal: 64 evenly routed tokens of 128 int8 experts 4096 x 1536
     // 371 us, with plain loads 420.  Those of an expert with several row tiles are read by as many workgroups at about the same
-    // time, and with the hint each goes past L2 again: plain loads there take Zipf-routed batches from 250 to 221 us (256 tokens
-    // of that layer), 470 to 403 (the same in bf16), 352 to 324 (393 x 3 of 53 fp8 experts 6464 x 2560).  The walk stands here
+    // time, and with the hint some of it goes past L2 again (a Zipf-routed batch of 256 tokens fetched 574 and 272 MB in its two
+    // GEMMs, with plain loads there 437 and 229).  Passes: 256 Zipf-routed tokens of that layer 249 -> 218 us (other routing 238 ->
+    // 226), in bf16 454 -> 397, 393 x 3 of 53 fp8 experts 6464 x 2560 356 -> 324.  The walk stands here
     // twice because a choice at each load makes the compiler wait for more loads than it has to (decode 1 to 3 % slower); the
     // asm statements differ so that it does not fold the two walks' first loads into one and drop the hint.
     if(WEIGHTS == kOnce || (WEIGHTS == kByTile && tile.expert_tiles == 1))
