@@ -53,3 +53,39 @@ def test_codes_of_rows_of_every_length(inter, dtype):
     codes = np.rint(q) if dtype == "int8" else oracle.e4m3_to_f32(e4m3_codes(q))
     want = torch.from_numpy(codes.astype(np.float32) * scale).to(torch.bfloat16).float().numpy()
     assert np.array_equal(got, want), int((got != want).sum())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["int8", "fp8"])
+@pytest.mark.parametrize("inter", [256, 2176, 8320])  # a wave, 256 and 512 threads to a row
+def test_rows_past_the_padded_list_are_left_alone(inter, dtype):
+    """A row count larger than the padded list: the launch covers whole rounds of rows, and none past the list is touched, whatever
+    the sorted ids after it say.  Output and workspace are those of a count that ends with the list's last unit."""
+    import torch
+    import therock_amd as ta
+    T, E, H, unit, past = 5, 2, 128, 32, 4096
+    view = torch.int8 if dtype == "int8" else torch.float8_e4m3fn
+    traits = ta.fused_moe_traits(prec_i=dtype, prec_w=dtype, block_m=unit, gate_only=1, fused_quant=2)
+    buf = ta.MoeBuffers(traits, T, E, 1, H, inter, "cuda")
+    rows = -(-buf.max_pad // unit) * unit
+    ids = np.full(256, (1 << 24) | T, np.int32)  # padding: slot topk of token `tokens`
+    ids[:3], ids[unit:unit + 2], ids[rows:] = (0, 1, 2), (3, 4), 0
+    assert buf.max_pad < rows < 128 <= len(ids)
+    buf.sorted_ids = torch.from_numpy(ids).cuda()
+    buf.sorted_w = torch.ones(len(ids), device="cuda")
+    buf.sorted_eid = torch.tensor([0] + [1] * 7, dtype=torch.int32, device="cuda")
+    gen = torch.Generator().manual_seed(inter)
+    code = lambda *n: torch.randint(-60, 60, n, generator=gen).float().to(view).cuda()
+    args = ta.make_args(traits, buf, code(T, H), code(E, inter, H), code(E, H, inter), torch.zeros((T, 1), dtype=torch.int32, device="cuda"),
+                        torch.ones((T, 1), device="cuda"), a_scale=torch.full((T,), 0.01, device="cuda"),
+                        g_scale=torch.full((E, inter), 0.01, device="cuda"), d_scale=torch.full((E, H), 0.01, device="cuda"))
+    seen = []
+    for total in (rows, past):
+        print(f"rows past the list: {dtype} {inter}, count {total}", flush=True)
+        buf.ws.fill_(0xA5)
+        buf.total[0] = total
+        assert ta.fused_moegemm(traits, args) == 0.0
+        torch.cuda.synchronize()
+        seen.append((buf.out.clone(), buf.ws.clone()))
+    assert float(seen[0][0].float().abs().max()) > 0 and bool(torch.isfinite(seen[0][0].float()).all())
+    assert torch.equal(seen[0][0], seen[1][0]) and torch.equal(seen[0][1], seen[1][1])

@@ -620,7 +620,7 @@ __global__ __launch_bounds__(LANES < 256 ? 256 : LANES) void moe_requant_y_kerne
                                                              const int* __restrict__ total, int unit, int tokens, int topk,
                                                              int segs,
                                                              unsigned char* __restrict__ yq, float* __restrict__ yscale,
-                                                             int row_blocks, uint4* __restrict__ ones, int64_t n_ones)
+                                                             int max_rows, int row_blocks, uint4* __restrict__ ones, int64_t n_ones)
 {
     constexpr int kThreads = LANES < 256 ? 256 : LANES;
     constexpr bool kMore   = LANES == 512; // a row may have more columns than its threads hold
@@ -641,7 +641,7 @@ __global__ __launch_bounds__(LANES < 256 ? 256 : LANES) void moe_requant_y_kerne
     const int round        = slot / kPerSlab;
     const int64_t group    = (int64_t)(round * 8 + ((blockIdx.x + round) & 7)) * kPerSlab + slot % kPerSlab;
     const int64_t row      = LANES > 64 ? group : group * 4 + (threadIdx.x >> 6);
-    if(row >= total[0])
+    if(row >= min(total[0], max_rows)) // (the grid covers whole rounds, up to 127 rows past the buffers)
         return;
     const int chunks = inter >> 3;
     auto dst = [&](int c) {
@@ -870,8 +870,8 @@ int launch_requant_y(const void* y, int32_t inter, const float* smooth, const in
     const dim3 grid((unsigned)(row_blocks + std::min<int64_t>(ceil_div<int64_t>(n_ones, threads), 4096)));
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, stream, static_cast<const uint16_t*>(y), inter, smooth, sorted_ids,
-                           sorted_expert_ids, total, unit, tokens, topk, segs, static_cast<unsigned char*>(yq), yscale, row_blocks,
-                           static_cast<uint4*>(ones), n_ones);
+                           sorted_expert_ids, total, unit, tokens, topk, segs, static_cast<unsigned char*>(yq), yscale, (int)max_rows,
+                           row_blocks, static_cast<uint4*>(ones), n_ones);
     };
     auto of_type       = [&](auto smooth_tag, auto fp8_tag) {
         constexpr bool S = decltype(smooth_tag)::value, F = decltype(fp8_tag)::value;
