@@ -49,4 +49,3 @@ def kernels():
             name = said.pop("symbol").removesuffix(".kd")
             got[name] = {k: int(v) for k, v in said.items()}
     return got
-

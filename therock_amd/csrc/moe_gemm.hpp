@@ -40,10 +40,10 @@ int gemm_alt_tile_rows(const mi355_fused_moe_traits& t, int32_t tokens, int32_t 
 int gemm_tile_rows(const mi355_fused_moe_traits& t, int32_t tokens, int32_t experts, int32_t topk, int32_t hidden,
                    int32_t inter);
 
-// slices of K the down GEMM of this problem runs with (1: not cut) in a workspace of ws_bytes; 0: too small
 // weight rows (output columns) a workgroup of the down GEMM owns: 64 in the decode kernel, 256 in the others
 int down_gemm_tile_cols(const mi355_fused_moe_traits& t, int32_t tokens, int32_t experts, int32_t topk, int32_t hidden, int32_t inter);
 
+// slices of K the down GEMM of this problem runs with (1: not cut) in a workspace of ws_bytes; 0: too small
 int down_gemm_slices(const mi355_fused_moe_traits& t, int32_t tokens, int32_t experts, int32_t topk, int32_t hidden,
                      int32_t inter, size_t ws_bytes);
 int moe_flatmm_slices(int kind, const mi355_moe_flatmm_args& a, size_t ws_bytes);
